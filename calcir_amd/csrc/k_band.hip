@@ -908,6 +908,14 @@ __device__ __forceinline__ void q2_block_gk(int n, int64_t q, int* g, int* k) {
     *k = int(q - o);
 }
 
+// Four values as the 16 bytes of their BF16 parts: hi (8 bytes), then lo.
+__device__ __forceinline__ float4 q2_split4(const float (&v)[4]) {
+    unsigned h0, l0, h1, l1;
+    split_bf16x2(v[0], v[1], h0, l0);
+    split_bf16x2(v[2], v[3], h1, l1);
+    return float4{__uint_as_float(h0), __uint_as_float(h1), __uint_as_float(l0), __uint_as_float(l1)};
+}
+
 // Per block (one wave): reflectors that do not exist (sweeps past n - 3, or
 // past their last task) are zeroed; T is formed (forward, columnwise), and V
 // and -V T are stored in the operand order of the 16x16x4 MFMA products that
@@ -964,17 +972,29 @@ __global__ void __launch_bounds__(64) q2_prep_kernel(int n, int64_t nblk, float*
     __syncthreads();
     const int l16 = lane & 15, lq = lane >> 4;
     // V^T as the A operand of the W product: register 4 q + e of lane (lq,
-    // l16) holds V(16 q + 4 lq + e, l16)
+    // l16) holds V(16 q + 4 lq + e, l16); -V T as the A operand of the update,
+    // register 4 rt + s of lane (lq, l16): FP32 16x16x4 steps take NV(16 rt +
+    // l16, 4 s + lq), split-BF16 products NV(16 rt + l16, 4 lq + s).  The
+    // split-BF16 operands are split here, once per block instead of once per
+    // block and slab: each 16 bytes hold the hi and lo parts of 4 values.
 #pragma unroll
-    for (int s = 0; s < kQ2R / 4; ++s) V[lane * (kQ2R / 4) + s] = sv[16 * (s >> 2) + 4 * lq + (s & 3)][l16];
-    // -V T as the A operand of the update, register 4 rt + s of lane (lq,
-    // l16): FP32 16x16x4 steps take NV(16 rt + l16, 4 s + lq), split-BF16
-    // 16x16x16 products NV(16 rt + l16, 4 lq + s)
+    for (int q = 0; q < 3; ++q) {
+        float v[4], w[4];
 #pragma unroll
-    for (int rt = 0; rt < 3; ++rt)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            NVT[lane * 12 + 4 * rt + s] = bf16 ? snv[16 * rt + l16][4 * lq + s] : snv[16 * rt + l16][4 * s + lq];
+        for (int e = 0; e < 4; ++e) {
+            v[e] = sv[16 * q + 4 * lq + e][l16];
+            w[e] = bf16 ? snv[16 * q + l16][4 * lq + e] : snv[16 * q + l16][4 * e + lq];
+        }
+        float4* vo = reinterpret_cast<float4*>(V + lane * 12) + q;
+        float4* wo = reinterpret_cast<float4*>(NVT + lane * 12) + q;
+        if (bf16) {
+            *vo = q2_split4(v);
+            *wo = q2_split4(w);
+        } else {
+            *vo = float4{v[0], v[1], v[2], v[3]};
+            *wo = float4{w[0], w[1], w[2], w[3]};
+        }
+    }
     if (lane < kQ2G) tau[lane] = stau[lane];
 }
 
@@ -999,6 +1019,16 @@ __host__ __device__ inline int q2_pitch(int n) {
     const int p = n + kQ2R + 3;
     return p + ((4 - p) & 63);
 }
+typedef short short8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ shortx4 q2_half(float a, float b) {
+    return __builtin_bit_cast(shortx4, (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32));
+}
+__device__ __forceinline__ short8 q2_cat(shortx4 a, shortx4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ floatx4 q2_mfma32(short8 a, short8 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 template <int kQ2NT, bool BF>
 __global__ void __launch_bounds__(kQ2NT) q2_apply_kernel(int n, int ld, const float* __restrict__ Q2all,
                                                           float* __restrict__ Zall, int64_t nblk, int nmat) {
@@ -1112,10 +1142,6 @@ __global__ void __launch_bounds__(kQ2NT) q2_apply_kernel(int n, int ld, const fl
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
             const int g = NG - 1 - gi;
             const int rb = g * kQ2G + 1 + k * kBandNB;
-            const float vs[12] = {va[0].x, va[0].y, va[0].z, va[0].w, va[1].x, va[1].y,
-                                  va[1].z, va[1].w, va[2].x, va[2].y, va[2].z, va[2].w};
-            const float ns[12] = {na[0].x, na[0].y, na[0].z, na[0].w, na[1].x, na[1].y,
-                                  na[1].z, na[1].w, na[2].x, na[2].y, na[2].z, na[2].w};
             // this lane's column, from the block's first row
             float* zc = Zs + l16 * P + rb + 3;
             floatx4 zq[3];
@@ -1124,32 +1150,46 @@ __global__ void __launch_bounds__(kQ2NT) q2_apply_kernel(int n, int ld, const fl
             floatx4 acc[3];
             if constexpr (BF) {
                 // split-BF16x3 (x = hi + lo, products lo*hi + hi*lo + hi*hi
-                // accumulated in FP32) on 16x16x16 BF16 MFMA: lane (lq, l16)
-                // holds k = 4 lq .. 4 lq + 3 of its row (A) or column (B), so
-                // W = V^T Zb comes out as the update's B operand, W(4 lq + r,
-                // l16) in register r, with no transpose
-                floatx4 w = {0.f, 0.f, 0.f, 0.f};
+                // accumulated in FP32), the operands' parts stored by
+                // q2_prep_kernel.  Lane (lq, l16) holds k = 4 lq .. 4 lq + 3
+                // of its row (A) or column (B), so W = V^T Zb comes out as the
+                // update's B operand, W(4 lq + r, l16) in register r, with no
+                // transpose.  Two 16-deep products share one 16x16x32 MFMA
+                // (the same 16 cycles as a 16x16x16): lo*hi beside hi*lo, and
+                // two row tiles' hi*hi.  An odd product has a zero half: a
+                // 16x16x16 and a 16x16x32 one after the other on the same
+                // accumulator gave wrong sums on this device.
+                constexpr shortx4 zero4 = {0, 0, 0, 0};
+                short8 vhl[3], zlh[3];
+                shortx4 vh[3], zh[3];
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
-                    shortx4 vh, vl, zh, zl;
-                    split_bf16(vs[4 * q], vs[4 * q + 1], vs[4 * q + 2], vs[4 * q + 3], vh, vl);
-                    split_bf16(zq[q][0], zq[q][1], zq[q][2], zq[q][3], zh, zl);
-                    w = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vl, zh, w, 0, 0, 0);
-                    w = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vh, zl, w, 0, 0, 0);
-                    w = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vh, zh, w, 0, 0, 0);
+                    const shortx4 vl = q2_half(va[q].z, va[q].w);
+                    shortx4 zl;
+                    vh[q] = q2_half(va[q].x, va[q].y);
+                    split_bf16(zq[q][0], zq[q][1], zq[q][2], zq[q][3], zh[q], zl);
+                    vhl[q] = q2_cat(vl, vh[q]);
+                    zlh[q] = q2_cat(zh[q], zl);
                 }
+                floatx4 w = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 3; ++q) w = q2_mfma32(vhl[q], zlh[q], w);
+                w = q2_mfma32(q2_cat(vh[0], vh[1]), q2_cat(zh[0], zh[1]), w);
+                w = q2_mfma32(q2_cat(vh[2], zero4), q2_cat(zh[2], zero4), w);
                 shortx4 wh, wl;
                 split_bf16(w[0], w[1], w[2], w[3], wh, wl);
+                const short8 whl = q2_cat(wh, wl), wh0 = q2_cat(wh, zero4);
 #pragma unroll
                 for (int rt = 0; rt < 3; ++rt) {
-                    acc[rt] = *reinterpret_cast<const floatx4*>(zc + 16 * rt + 4 * lq);
-                    shortx4 nh, nl;
-                    split_bf16(ns[4 * rt], ns[4 * rt + 1], ns[4 * rt + 2], ns[4 * rt + 3], nh, nl);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(nl, wh, acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(nh, wl, acc[rt], 0, 0, 0);
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(nh, wh, acc[rt], 0, 0, 0);
+                    const shortx4 nh = q2_half(na[rt].x, na[rt].y), nl = q2_half(na[rt].z, na[rt].w);
+                    acc[rt] = q2_mfma32(q2_cat(nl, nh), whl, zq[rt]);
+                    acc[rt] = q2_mfma32(q2_cat(nh, zero4), wh0, acc[rt]);
                 }
             } else {
+            const float vs[12] = {va[0].x, va[0].y, va[0].z, va[0].w, va[1].x, va[1].y,
+                                  va[1].z, va[1].w, va[2].x, va[2].y, va[2].z, va[2].w};
+            const float ns[12] = {na[0].x, na[0].y, na[0].z, na[0].w, na[1].x, na[1].y,
+                                  na[1].z, na[1].w, na[2].x, na[2].y, na[2].z, na[2].w};
             floatx4 w0 = {0.f, 0.f, 0.f, 0.f}, w1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
