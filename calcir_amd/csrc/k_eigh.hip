@@ -1172,11 +1172,7 @@ int tridiag_single(int n, int ld, T* A, T* d, T* e, T* tau, T* P, T* buf, hipStr
 
 // 1/q from the hardware reciprocal (about 24 bits) refined by Newton-Raphson
 // steps r <- r + r (1 - q r): one step gives about 48 bits (measured max
-// relative error 2.2e-15), two give full double precision.  The Sturm count
-// below needs only the signs of its recurrence: a relative error of a few
-// ulps in e^2/q is a perturbation of the off-diagonal of that size, far below
-// the bisection tolerance of an FP32-derived T (1024 eps ||T||); an FP64 T
-// (tolerance 4 eps ||T||) takes the second step.
+// relative error 2.2e-15), two give full double precision.
 template <bool FULL>
 __device__ __forceinline__ double nr_rcp(double q) {
     double r = __builtin_amdgcn_rcp(q);
@@ -1185,72 +1181,116 @@ __device__ __forceinline__ double nr_rcp(double q) {
     return r;
 }
 
-// Number of eigenvalues of T below x (Sturm sequence count).  |q| >= pivmin
-// keeps every reciprocal finite.
-template <bool FULL>
-__device__ __forceinline__ int sturm_count(int n, const double* sd, const double* se2, double x,
-                                           double pivmin) {
-    double q = sd[0] - x;
-    if (fabs(q) < pivmin) q = -pivmin;
-    int c = q < 0.0;
-    for (int k = 1; k < n; ++k) {
-        q = (sd[k] - x) - se2[k - 1] * nr_rcp<FULL>(q);
-        if (fabs(q) < pivmin) q = -pivmin;
-        c += q < 0.0;
+// Number of eigenvalues of T below x: the sign changes of the leading
+// principal minors p_k of T - x I,
+//     p_{k+1} = (d_k - x) p_k - e_{k-1}^2 p_{k-1}.
+// The quotient form q_k = p_k / p_{k-1} needs a reciprocal per row (16 cycles
+// on its own, and a chain of about 60 cycles from row to row); the minors need
+// none: a subtraction, a product and one FMA on the chain.  Each row's error
+// is a relative error of a few eps in its d_k - x and e_{k-1}^2, as in the
+// quotient form.  sde[k] = (d_k, e_{k-1}^2) of T scaled to norm at most 1, the
+// squares at least kSturmFloor, so a row grows the pair (p_k, p_{k-1}) by less
+// than 4 and two rows shrink it by no more than that floor: rescaling the pair
+// to 1 every kSturmRows rows keeps both within FP64's range.  A minor that is
+// exactly zero has its neighbours of opposite sign and counts once whatever
+// its own sign.  The signs are shifted into a register and their changes
+// counted once per kSturmRows rows.  Bound by FP64 issue: 256 matrices of n = 2048
+// (FP32-derived T, 36 counts per eigenvalue) take 6.0 ms, 14.4 ms in the
+// quotient form; one matrix, bound by the chain, 0.99 and 2.7 ms.
+constexpr int kSturmRows = 16;
+constexpr double kSturmFloor = 0x1p-110;
+__device__ __forceinline__ int sturm_count(int n, const double2* __restrict__ sde, double x) {
+    double p0 = 0.0, p1 = 1.0;  // p_{k-1}, p_k
+    unsigned bits = 0;          // signs of the minors so far, the last in bit 0
+    int c = 0;
+    auto row = [&](const double2& t) {
+        const double p2 = fma(t.x - x, p1, -(t.y * p0));
+        bits = __builtin_amdgcn_alignbit(bits, unsigned(__double2hiint(p2)), 31);
+        p0 = p1;
+        p1 = p2;
+    };
+    // kSturmRows / 2 rows of T are read ahead of the ones in use, so a row's
+    // LDS read is off the chain (past the last row: the reductions and counts
+    // that follow T in LDS, more than kSturmRows rows of them, never used)
+    constexpr int H = kSturmRows / 2;
+    double2 ta[H], tb[H];
+    auto read = [&](double2(&t)[H], int k) {
+#pragma unroll
+        for (int j = 0; j < H; ++j) t[j] = sde[k + j];
+    };
+    read(ta, 0);
+    int k = 0;
+    for (; k + kSturmRows <= n; k += kSturmRows) {
+        read(tb, k + H);
+#pragma unroll
+        for (int j = 0; j < H; ++j) row(ta[j]);
+        read(ta, k + kSturmRows);
+#pragma unroll
+        for (int j = 0; j < H; ++j) row(tb[j]);
+        c += __popc((bits ^ (bits >> 1)) & ((1u << kSturmRows) - 1));
+        const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+        p0 = ldexp(p0, -ex);
+        p1 = ldexp(p1, -ex);
     }
-    return c;
+    const int rest = n - k;
+    for (; k < n; ++k) row(sde[k]);
+    return c + __popc((bits ^ (bits >> 1)) & ((1u << rest) - 1));
 }
 
 template <typename T>
 __global__ void __launch_bounds__(kEigNT)
 bisect_kernel(int n, const T* __restrict__ dall, const T* __restrict__ eall, double* __restrict__ wall) {
-    extern __shared__ double shd[];
-    double* sd = shd;
-    double* se2 = shd + n;
-    double* sr = shd + 2 * n;  // 3 * (kEigNT/64) reductions, then kEigNT multisection counts
+    extern __shared__ __align__(16) double shd[];
+    double2* const sde = reinterpret_cast<double2*>(shd);
+    double* const sr = shd + 2 * n;  // 2 * (kEigNT/64) reductions, then kEigNT multisection counts
     const int b = blockIdx.y, tid = threadIdx.x;
     const T* d = dall + size_t(b) * n;
     const T* e = eall + size_t(b) * n;
-    double lo = DBL_MAX, hi = -DBL_MAX, emax = 0.0;
+    double lo = DBL_MAX, hi = -DBL_MAX;
     for (int k = tid; k < n; k += kEigNT) {
         const double dk = double(d[k]);
         const double ek = (k < n - 1) ? double(e[k]) : 0.0;
         const double ekm = (k > 0) ? double(e[k - 1]) : 0.0;
-        sd[k] = dk;
-        se2[k] = ek * ek;
+        sde[k] = double2{dk, ekm};
         const double rad = fabs(ek) + fabs(ekm);
         lo = fmin(lo, dk - rad);
         hi = fmax(hi, dk + rad);
-        emax = fmax(emax, ek * ek);
     }
     for (int off = 32; off > 0; off >>= 1) {
         lo = fmin(lo, __shfl_xor(lo, off, 64));
         hi = fmax(hi, __shfl_xor(hi, off, 64));
-        emax = fmax(emax, __shfl_xor(emax, off, 64));
     }
     const int lane = tid & 63, wave = tid >> 6;
     if (lane == 0) {
         sr[wave] = lo;
         sr[4 + wave] = hi;
-        sr[8 + wave] = emax;
     }
     __syncthreads();
-    double gl = sr[0], gu = sr[4], e2 = sr[8];
+    double gl = sr[0], gu = sr[4];
     for (int w = 1; w < kEigNT / 64; ++w) {
         gl = fmin(gl, sr[w]);
         gu = fmax(gu, sr[4 + w]);
-        e2 = fmax(e2, sr[8 + w]);
     }
-    const double tnorm = fmax(fabs(gl), fabs(gu));
-    const double pivmin = DBL_MIN * fmax(1.0, e2);
-    const double widen = 4.0 * DBL_EPSILON * tnorm + 4.0 * pivmin;
+    // T scaled by a power of two (exact) to norm at most 1
+    double tnorm = fmax(fabs(gl), fabs(gu));
+    const int ex = (tnorm > 0.0) ? __builtin_amdgcn_frexp_exp(tnorm) : 0;
+    for (int k = tid; k < n; k += kEigNT) {
+        const double2 t = sde[k];
+        const double es = ldexp(t.y, -ex);
+        sde[k] = double2{ldexp(t.x, -ex), fmax(es * es, kSturmFloor)};
+    }
+    gl = ldexp(gl, -ex);
+    gu = ldexp(gu, -ex);
+    tnorm = ldexp(tnorm, -ex);
+    const double widen = 4.0 * DBL_EPSILON * tnorm + 4.0 * DBL_MIN;
     gl -= widen;
     gu += widen;
+    __syncthreads();
     // multisection: Sturm counts at kEigNT interior points of [gl, gu] give
     // every eigenvalue a starting bracket kEigNT + 1 times narrower
-    int* scnt = reinterpret_cast<int*>(sr + 12);
+    int* scnt = reinterpret_cast<int*>(sr + 8);
     const double step = (gu - gl) / double(kEigNT + 1);
-    scnt[tid] = sturm_count<sizeof(T) == 8>(n, sd, se2, gl + step * double(tid + 1), pivmin);
+    scnt[tid] = sturm_count(n, sde, gl + step * double(tid + 1));
     __syncthreads();
     const int j = blockIdx.x * kEigNT + tid;
     if (j >= n) return;
@@ -1266,12 +1306,12 @@ bisect_kernel(int n, const T* __restrict__ dall, const T* __restrict__ eall, dou
     const double abstol = (sizeof(T) == 4 ? 1024.0 : 4.0) * DBL_EPSILON * tnorm;
     for (int it = 0; it < 128 && (c - a) > fmax(2.0 * DBL_EPSILON * (fabs(a) + fabs(c)), abstol); ++it) {
         const double mid = 0.5 * (a + c);
-        if (sturm_count<sizeof(T) == 8>(n, sd, se2, mid, pivmin) > j)
+        if (sturm_count(n, sde, mid) > j)
             c = mid;
         else
             a = mid;
     }
-    wall[size_t(b) * n + j] = 0.5 * (a + c);
+    wall[size_t(b) * n + j] = ldexp(0.5 * (a + c), ex);
 }
 
 __device__ __forceinline__ double hash_uniform(uint32_t a, uint32_t b) {
