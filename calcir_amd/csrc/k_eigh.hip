@@ -1322,25 +1322,69 @@ __device__ __forceinline__ double hash_uniform(uint32_t a, uint32_t b) {
     return double(z >> 11) * (2.0 / 9007199254740992.0) - 1.0;
 }
 
-// 3 FP64 arrays and a byte array of n x n, rounded up to 256 bytes so that
-// the next matrix's arrays stay aligned
+// FP64 array of n x n (the vectors) and the factorisation's carried pair every
+// kInvSeg rows, rounded up to 256 bytes so that the next matrix's arrays stay
+// aligned
+constexpr int kInvSeg = 8;
+__host__ __device__ inline size_t invit_segs(int n) { return (size_t(n) + kInvSeg - 1) / kInvSeg; }
 __host__ __device__ inline size_t invit_scratch_bytes(int n) {
-    return (25 * ((size_t(n) + 63) & ~size_t(63)) * n + 255) & ~size_t(255);
+    return (8 * ((size_t(n) + 63) & ~size_t(63)) * (size_t(n) + 2 * invit_segs(n)) + 255) & ~size_t(255);
 }
 
-// Scratch of one matrix (invit_scratch_bytes): FP64 arrays X (the vectors),
-// R (reciprocal pivots) and L (multipliers), then the pivot flags F (bytes),
-// each of n rows by n eigenvalues padded to a multiple of 64: element (k, c),
-// c the eigenvalue index, at [(c / 64) 64 n + 64 k + c % 64].  Lanes run along
+// Row i of the LU factorisation of T - lambda I with partial pivoting, from
+// the carried pair (a, bs) = the working row's entries in columns i, i + 1;
+// sub = e(i), dn = d(i + 1) - lambda, en = e(i + 1) (0 past the end).  Gives
+// the reciprocal pivot r, U's entries (u1, u2) right of it, the multiplier l
+// and whether the rows were exchanged, and carries the pair to row i + 1.  A
+// pivot below pivmin (0 included) is taken as +-pivmin, so reciprocals stay
+// finite and |l| <= 1.  An FP32-derived T takes the refined hardware
+// reciprocal for both r and l, an FP64 T IEEE quotients.
+struct LuRow {
+    double r, u1, u2, l;
+    bool piv;
+};
+template <typename T>
+__device__ __forceinline__ LuRow invit_lu_row(double sub, double dn, double en, double pivmin, double& a, double& bs) {
+    LuRow o;
+    o.piv = !(fabs(a) >= fabs(sub));
+    if (!o.piv && fabs(a) < pivmin) a = (a < 0.0) ? -pivmin : pivmin;
+    const double den = o.piv ? sub : a, num = o.piv ? a : sub;
+    if constexpr (sizeof(T) == 8) {
+        o.r = 1.0 / den;
+        o.l = num / den;
+    } else {
+        o.r = nr_rcp<false>(den);
+        o.l = num * o.r;
+    }
+    if (fabs(den) < pivmin) {
+        const double u0 = (den < 0.0) ? -pivmin : pivmin;
+        o.r = (sizeof(T) == 8) ? 1.0 / u0 : nr_rcp<false>(u0);
+    }
+    o.u1 = o.piv ? dn : bs;
+    o.u2 = o.piv ? en : 0.0;
+    const double an = o.piv ? bs - o.l * dn : dn - o.l * bs;
+    bs = o.piv ? -o.l * en : en;
+    a = an;
+    return o;
+}
+
+// Scratch of one matrix (invit_scratch_bytes): the FP64 vectors X, n rows by n
+// eigenvalues padded to a multiple of 64, element (k, c), c the eigenvalue
+// index, at [(c / 64) 64 n + 64 k + c % 64], then the carried pairs of the
+// factorisation in the same form with ceil(n / kInvSeg) rows.  Lanes run along
 // c, so every access is coalesced, and a wave's successive rows are adjacent
-// 512-byte blocks (a row-major n x n layout put them n elements apart).  The LU of T - lambda_c I with partial pivoting
-// has U = (u0, u1, u2) per row; only 1/u0 is kept: u1 and u2 are rebuilt from
-// T, the flag and the previous row's multiplier (a pivoted row has u1 =
-// d(i+1) - lambda, u2 = e(i+1); an unpivoted row u2 = 0 and u1 the carried
-// e(i), times -l(i-1) after a pivoted row), which cuts the scratch traffic by
-// a third.  The first iteration's right-hand side is regenerated from its
-// seed, so X is first written by the back substitution.  The second iteration
-// reuses the factorisation.  Factors and
+// 512-byte blocks.  The LU factors are not kept: they would be 17 bytes per
+// (row, eigenvalue), written once and read three times, which with the
+// vectors bound the kernel by its scratch traffic (112 bytes; 27.9 ms for 256
+// matrices of n = 2048).  The first forward pass keeps the carried pair every
+// kInvSeg rows; a back substitution refactors a segment of that many rows into
+// registers from its pair, and the second iteration's forward pass refactors
+// as it goes.  That is four factorisations instead of one against 48 bytes of
+// traffic: 12.9 ms (one matrix: 2.3 -> 1.35 ms; FP64, n = 256, 64 matrices: 0.34
+// -> 0.20 ms).  Segments of 4 rows, or registers for 3 or 4 waves per SIMD,
+// took 14.0 to 27 ms.  The same operations in the same order give the same
+// factors every time.  The first iteration's right-hand side is regenerated
+// from its seed, so X is first written by the back substitution.  Factors and
 // vectors are FP64 even for an FP32-derived T: eigenvectors of eigenvalues
 // closer than ~1e-7 ||T|| (but not clustered) are only told apart by factors
 // accurate beyond FP32, and near-degenerate pivots grow the vector past the
@@ -1349,27 +1393,23 @@ template <typename T>
 __global__ void __launch_bounds__(kEigNT)
 invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ eall,
              const double* __restrict__ wall, T* __restrict__ Zall, unsigned char* __restrict__ scr, int b0) {
-    extern __shared__ double shd[];
-    double* sd = shd;
-    double* se = shd + n;
+    extern __shared__ __align__(16) double shd[];
+    double2* const sde = reinterpret_cast<double2*>(shd);  // (d(k), e(k)), e(n - 1) = 0
     const int bl = blockIdx.y, b = b0 + bl, tid = threadIdx.x;
     const T* d = dall + size_t(b) * n;
     const T* e = eall + size_t(b) * n;
     const double* w = wall + size_t(b) * n;
     T* Z = Zall + size_t(b) * n * ld;
-    // element (k, c) at col(c) + 64 k: tiles of 64 eigenvalues (one wave),
+    // element (k, c) of X at col(c) + 64 k: tiles of 64 eigenvalues (one wave),
     // rows contiguous within a tile, so a lane's walk down the rows streams
     // 512-byte blocks per wave
-    const size_t nn = ((size_t(n) + 63) & ~size_t(63)) * n;
+    const size_t n64 = (size_t(n) + 63) & ~size_t(63);
+    const int nseg = int(invit_segs(n));
     auto col = [n](int c) { return size_t(c >> 6) * 64 * n + (c & 63); };
     double* const SX = reinterpret_cast<double*>(scr + size_t(bl) * invit_scratch_bytes(n));
-    double* const SR = SX + nn;
-    double* const SL = SR + nn;
-    unsigned char* const SF = reinterpret_cast<unsigned char*>(SL + nn);
-    for (int k = tid; k < n; k += kEigNT) {
-        sd[k] = double(d[k]);
-        se[k] = (k < n - 1) ? double(e[k]) : 0.0;
-    }
+    double* const SA = SX + n64 * n;
+    double* const SB = SA + n64 * nseg;
+    for (int k = tid; k < n; k += kEigNT) sde[k] = double2{double(d[k]), (k < n - 1) ? double(e[k]) : 0.0};
     __syncthreads();
     const int c = blockIdx.x * kEigNT + tid;
     if (c >= n) return;
@@ -1384,128 +1424,84 @@ invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ ea
     while (cend + 1 < n && cend + 1 - c < kMaxCluster && joins_cluster(w, cend + 1)) ++cend;
     const bool single = cend == c;
 
+    constexpr int S = kInvSeg;
     double lam_prev = 0.0;
     for (int mb = c; mb <= cend; ++mb) {
         double lam = w[mb];
         if (mb > c) lam = fmax(lam, lam_prev + 10.0 * DBL_EPSILON * fmax(fabs(lam_prev), 1.0));
         lam_prev = lam;
         double* X = SX + col(mb);
-        double* R = SR + col(mb);
-        double* Lm = SL + col(mb);
-        unsigned char* F = SF + col(mb);
+        const size_t scol = size_t(mb >> 6) * 64 * nseg + (mb & 63);
+        double* CA = SA + scol;
+        double* CB = SB + scol;
+        // row i: e(i) is carried from the row before, (d, e)(i + 1) read
+        double sub;
+        auto lu = [&](int i, double& a, double& bs) {
+            const double2 t = sde[i + 1];
+            const LuRow o = invit_lu_row<T>(sub, t.x - lam, t.y, pivmin, a, bs);
+            sub = t.y;
+            return o;
+        };
         // iteration 1, forward: factor T - lam I = P L U.  Its right-hand
         // side is a seeded vector b taken as already transformed by P L^{-1}
         // (the start vector is P L b, as in EISPACK's tinvit), so the first
         // back substitution regenerates b and no vector is stored here.
-        double a = sd[0] - lam;
-        double bs = (n > 1) ? se[0] : 0.0;
-        for (int i = 0; i < n - 1; ++i) {
-            const double sub = se[i];
-            const double dn = sd[i + 1] - lam;
-            const double en = (i + 1 < n - 1) ? se[i + 1] : 0.0;
-            double u0, l;
-            unsigned char fl;
-            if (fabs(a) >= fabs(sub)) {
-                // a pivot below pivmin (0 included) is taken as +-pivmin, as
-                // the back substitution's reciprocal takes it; the reciprocal
-                // then stays finite and |l| <= 1
-                if (fabs(a) < pivmin) a = (a < 0.0) ? -pivmin : pivmin;
-                l = (sizeof(T) == 8) ? sub / a : sub * nr_rcp<false>(a);
-                u0 = a;
-                a = dn - l * bs;
-                bs = en;
-                fl = 0;
-            } else {
-                l = (sizeof(T) == 8) ? a / sub : a * nr_rcp<false>(sub);
-                u0 = sub;
-                a = bs - l * dn;
-                bs = -l * en;
-                fl = 1;
-            }
-            if (fabs(u0) < pivmin) u0 = (u0 < 0.0) ? -pivmin : pivmin;
-            // reciprocal pivot: the back substitution multiplies; an FP32-derived
-            // T takes the refined hardware reciprocal, an FP64 T the IEEE one
-            R[size_t(i) * 64] = (sizeof(T) == 8) ? 1.0 / u0 : nr_rcp<false>(u0);
-            Lm[size_t(i) * 64] = l;
-            F[size_t(i) * 64] = fl;
+        double a = sde[0].x - lam;
+        double bs = sde[0].y;
+        sub = bs;
+        const int nfull = (n - 1) / S;  // full segments of the n - 1 factored rows
+        for (int sg = 0; sg < nfull; ++sg) {
+            CA[size_t(sg) * 64] = a;
+            CB[size_t(sg) * 64] = bs;
+#pragma unroll
+            for (int j = 0; j < S; ++j) lu(sg * S + j, a, bs);
+        }
+        if (nfull * S < n - 1) {
+            CA[size_t(nfull) * 64] = a;
+            CB[size_t(nfull) * 64] = bs;
+            for (int i = nfull * S; i < n - 1; ++i) lu(i, a, bs);
         }
         if (fabs(a) < pivmin) a = (a < 0.0) ? -pivmin : pivmin;
         const double alast = a;
         double scale = 1.0, big = 0.0, yi = hash_uniform(uint32_t(mb), uint32_t(n - 1));
-        // The solves' loops read each row's factors (and vector) from the
-        // scratch kPf rows ahead, into a ring of kPf register slots: a slot is
-        // read again for the row kPf further on as soon as its row is solved,
-        // so a row's reads are in flight while the kPf - 1 rows before it are
-        // solved.  Each pass is a chain of dependent rows, and at a few waves
-        // per SIMD the read latency of one row at a time set the kernel's
-        // time.  Rows of the last partial ring are solved one at a time.
-        constexpr int kPf = 4;
-        double rr[kPf], rl[kPf], rx[kPf];
-        int rf[kPf];
         for (int it = 0; it < 2; ++it) {
             if (it == 1) {
-                // forward with the kept factorisation: P L^{-1} (scale x)
+                // forward, factoring again: P L^{-1} (scale x)
                 yi = X[0] * scale;
-                // row i: X(i + 1), L(i), F(i)
-                auto ld = [&](int j, int i) {
-                    i = min(i, n - 2);
-                    rx[j] = X[size_t(i + 1) * 64];
-                    rl[j] = Lm[size_t(i) * 64];
-                    rf[j] = F[size_t(i) * 64];
-                };
-                auto row = [&](int i, double xn, double l, int f) {
+                a = sde[0].x - lam;
+                bs = sde[0].y;
+                sub = bs;
+                auto row = [&](int i, double xn) {
+                    const LuRow o = lu(i, a, bs);
                     const double yn = xn * scale;
-                    double yo;
-                    if (f == 0) {
-                        yo = yi;
-                        yi = yn - l * yi;
-                    } else {
-                        yo = yn;
-                        yi = yi - l * yn;
-                    }
+                    const double yo = o.piv ? yn : yi;
+                    yi = o.piv ? yi - o.l * yn : yn - o.l * yi;
                     X[size_t(i) * 64] = yo;
                 };
-                const int nfull = ((n - 1) / kPf) * kPf;  // rows 0 .. nfull-1 through the ring
+                // X(i + 1) of a segment's rows is read a segment ahead
+                double xa[S];
                 if (nfull > 0) {
 #pragma unroll
-                    for (int j = 0; j < kPf; ++j) ld(j, j);
+                    for (int j = 0; j < S; ++j) xa[j] = X[size_t(j + 1) * 64];
                 }
-                for (int i0 = 0; i0 < nfull; i0 += kPf) {
+                for (int sg = 0; sg < nfull; ++sg) {
+                    double xc[S];
 #pragma unroll
-                    for (int j = 0; j < kPf; ++j) {
-                        row(i0 + j, rx[j], rl[j], rf[j]);
-                        ld(j, i0 + j + kPf);
+                    for (int j = 0; j < S; ++j) {
+                        xc[j] = xa[j];
+                        xa[j] = X[size_t(min((sg + 1) * S + j + 1, n - 1)) * 64];
                     }
+#pragma unroll
+                    for (int j = 0; j < S; ++j) row(sg * S + j, xc[j]);
                 }
-                for (int i = nfull; i < n - 1; ++i)
-                    row(i, X[size_t(i + 1) * 64], Lm[size_t(i) * 64], F[size_t(i) * 64]);
+                for (int i = nfull * S; i < n - 1; ++i) row(i, X[size_t(i + 1) * 64]);
             }
-            // backward: U x = y, u1/u2 rebuilt from T and the flags
+            // backward: U x = y
             double x1 = yi / alast, x2 = 0.0;
             X[size_t(n - 1) * 64] = x1;
             double nrm2 = x1 * x1;
             big = x1;
-            int fi = (n > 1) ? F[size_t(n - 2) * 64] : 0;
-            // row i: R(i), L(i - 1), F(i - 1) (rows i > 0), X(i) (second iteration)
-            auto ld = [&](int j, int i) {
-                i = max(i, 0);
-                const int ip = max(i - 1, 0);
-                rr[j] = R[size_t(i) * 64];
-                rl[j] = Lm[size_t(ip) * 64];
-                rf[j] = F[size_t(ip) * 64];
-                rx[j] = (it == 1) ? X[size_t(i) * 64] : 0.0;
-            };
-            auto row = [&](int i, double r, double lpv, int fpv, double xr) {
-                const int fp = (i > 0) ? fpv : 0;
-                const double lp = (i > 0) ? lpv : 0.0;
-                double u1, u2;
-                if (fi) {
-                    u1 = sd[i + 1] - lam;
-                    u2 = (i + 1 < n - 1) ? se[i + 1] : 0.0;
-                } else {
-                    u1 = (i > 0 && fp) ? -lp * se[i] : se[i];
-                    u2 = 0.0;
-                }
+            auto row = [&](int i, double r, double u1, double u2, double xr) {
                 const double rhs = (it == 0) ? hash_uniform(uint32_t(mb), uint32_t(i)) : xr;
                 const double xi = (rhs - u1 * x1 - u2 * x2) * r;
                 X[size_t(i) * 64] = xi;
@@ -1513,25 +1509,48 @@ invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ ea
                 if (fabs(xi) >= fabs(big)) big = xi;  // first largest component in ascending order
                 x2 = x1;
                 x1 = xi;
-                fi = fp;
             };
-            // rows n-2 .. n-1-nfull through the ring, then the rest one at a time
-            const int nfull = ((n - 1) / kPf) * kPf;
-            if (nfull > 0) {
+            // a segment's rows factored again from its carried pair, then
+            // solved; the next segment's pair and right-hand sides are read
+            // while this one is worked on
+            double pa, pb, px[S];
+            auto fetch = [&](int sg) {
+                const int q = max(sg, 0);
+                pa = CA[size_t(q) * 64];
+                pb = CB[size_t(q) * 64];
 #pragma unroll
-                for (int j = 0; j < kPf; ++j) ld(j, n - 2 - j);
-            }
-            for (int i0 = n - 2; i0 > n - 2 - nfull; i0 -= kPf) {
-#pragma unroll
-                for (int j = 0; j < kPf; ++j) {
-                    row(i0 - j, rr[j], rl[j], rf[j], rx[j]);
-                    ld(j, i0 - j - kPf);
+                for (int j = 0; j < S; ++j) px[j] = (it == 1) ? X[size_t(q * S + j) * 64] : 0.0;
+            };
+            if (nfull * S < n - 1) {
+                const int i0 = nfull * S, m = n - 1 - i0;
+                for (int q = m - 1; q >= 0; --q) {  // fewer than S rows: factored up to each
+                    a = CA[size_t(nfull) * 64];
+                    bs = CB[size_t(nfull) * 64];
+                    sub = sde[i0].y;
+                    LuRow o{};
+                    for (int i = 0; i <= q; ++i) o = lu(i0 + i, a, bs);
+                    row(i0 + q, o.r, o.u1, o.u2, (it == 1) ? X[size_t(i0 + q) * 64] : 0.0);
                 }
             }
-            for (int i = n - 2 - nfull; i >= 0; --i) {
-                const int ip = max(i - 1, 0);
-                row(i, R[size_t(i) * 64], Lm[size_t(ip) * 64], F[size_t(ip) * 64],
-                    (it == 1) ? X[size_t(i) * 64] : 0.0);
+            if (nfull > 0) fetch(nfull - 1);
+            for (int sg = nfull - 1; sg >= 0; --sg) {
+                const int i0 = sg * S;
+                double r[S], u1[S], u2[S], xs[S];
+                a = pa;
+                bs = pb;
+                sub = sde[i0].y;
+#pragma unroll
+                for (int j = 0; j < S; ++j) xs[j] = px[j];
+                fetch(sg - 1);
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    const LuRow o = lu(i0 + j, a, bs);
+                    r[j] = o.r;
+                    u1[j] = o.u1;
+                    u2[j] = o.u2;
+                }
+#pragma unroll
+                for (int j = S - 1; j >= 0; --j) row(i0 + j, r[j], u1[j], u2[j], xs[j]);
             }
             // orthogonalise against the cluster's earlier vectors
             if (mb > c) {
@@ -1550,9 +1569,18 @@ invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ ea
             scale = 1.0 / sqrt(nrm2);
         }
         if (single) {
-            // normalise, largest component positive, straight into Z
+            // normalise, largest component positive, straight into Z (eight
+            // rows' reads in flight together)
             const double f = (big < 0.0) ? -scale : scale;
-            for (int k = 0; k < n; ++k) Z[size_t(k) * ld + mb] = T(X[size_t(k) * 64] * f);
+            int k = 0;
+            for (; k + 8 <= n; k += 8) {
+                double v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = X[size_t(k + j) * 64];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) Z[size_t(k + j) * ld + mb] = T(v[j] * f);
+            }
+            for (; k < n; ++k) Z[size_t(k) * ld + mb] = T(X[size_t(k) * 64] * f);
             continue;
         }
         // cluster members stay in scratch, normalised, for the later members
