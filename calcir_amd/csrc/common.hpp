@@ -147,14 +147,6 @@ constexpr int kXcds = 8;
 #if defined(__HIPCC__)
 namespace cir {
 
-// calcIR.cu:1457-1460.  Contraction is disabled so that dx - L*round(dx/L)
-// is rounded exactly as written (the FP32 cutoff decision depends on it).
-template <typename T>
-__device__ __forceinline__ T minimage(T dx, T boxl) {
-#pragma clang fp contract(off)
-    return dx - boxl * round(dx / boxl);
-}
-
 // Periodic box of one frame.  Rectangular boxes (the reference's case,
 // calcIR.cu:404-405) hold the diagonal; triclinic boxes follow the GROMACS
 // convention a = (a0,0,0), b = (b0,b1,0), c = (c0,c1,c2), stored per frame as
@@ -162,7 +154,8 @@ __device__ __forceinline__ T minimage(T dx, T boxl) {
 template <typename T>
 struct PBox {
     T a0, b0, b1, c0, c1, c2;
-    bool tri;  // some off-diagonal element is nonzero
+    T ia0, ib1, ic2;  // 1 / a0, 1 / b1, 1 / c2
+    bool tri;         // some off-diagonal element is nonzero
 };
 
 // boxk 0: 3 floats (diagonal) per frame; 1: 9 floats (a, b, c rows).
@@ -186,20 +179,48 @@ __device__ __forceinline__ PBox<T> load_box(const float* box, int boxk, int f) {
         B.c2 = T(q[8]);
         B.tri = q[3] != 0.0f || q[6] != 0.0f || q[7] != 0.0f;
     }
+    B.ia0 = T(1) / B.a0;
+    B.ib1 = T(1) / B.b1;
+    B.ic2 = T(1) / B.c2;
     return B;
 }
 
+// dx / boxl to the nearest integer by the reciprocal of boxl.  `near` is set
+// where that integer might not be round(dx / boxl): the product q is within a
+// few eps |q| of the quotient, so the two round alike unless q lies that close
+// to a half-integer (where an IEEE quotient and rounding half away from zero
+// are needed; also every q too large to have a fraction).
+template <typename T>
+__device__ __forceinline__ T image_round(T dx, T inv, bool& near) {
+    constexpr T eps = sizeof(T) == 4 ? T(1.2e-7) : T(2.3e-16);
+    const T q = dx * inv, r = rint(q);
+    near |= fabs(fabs(q - r) - T(0.5)) <= T(4) * eps * (fabs(q) + T(1));
+    return r;
+}
+
 // Minimum image of a separation.  Rectangular: calcIR.cu:1457-1460 per axis
-// (bit for bit the reference form).  Triclinic: the lattice vectors are
+// (bit for bit the reference form; three IEEE quotients and roundings cost
+// more than the rest of a pair's arithmetic, so the integers come from the
+// box's reciprocals unless one is near a tie).  Triclinic: the lattice vectors are
 // removed in the order c, b, a, each by the rounded fractional coordinate
 // along its own axis (the GROMACS form for reduced boxes).
 template <typename T>
 __device__ __forceinline__ void minimage3(T& dx, T& dy, T& dz, const PBox<T>& B) {
+    // dx - L round(dx / L) rounded exactly as written: the FP32 cutoff
+    // decision depends on it
 #pragma clang fp contract(off)
     if (!B.tri) {
-        dx = minimage<T>(dx, B.a0);
-        dy = minimage<T>(dy, B.b1);
-        dz = minimage<T>(dz, B.c2);
+        bool near = false;
+        T rx = image_round<T>(dx, B.ia0, near), ry = image_round<T>(dy, B.ib1, near),
+          rz = image_round<T>(dz, B.ic2, near);
+        if (near) {
+            rx = round(dx / B.a0);
+            ry = round(dy / B.b1);
+            rz = round(dz / B.c2);
+        }
+        dx = dx - B.a0 * rx;
+        dy = dy - B.b1 * ry;
+        dz = dz - B.c2 * rz;
         return;
     }
     T s = round(dz / B.c2);
@@ -232,6 +253,14 @@ template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
+}
+
+// Make this wave's LDS stores visible to its own later LDS loads (a wave's LDS
+// operations complete in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 }  // namespace cir

@@ -61,14 +61,6 @@ __device__ __forceinline__ float bwave_sum(float x) {
     return __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
 }
 
-// Make this wave's LDS stores visible to its own later LDS loads (a wave's LDS
-// operations complete in order; this keeps the compiler from moving them).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Wave sums of 32 per-lane values x[k], written to out[k] (LDS).  Two lane
 // swaps halve the values per lane (after them lane l holds the partials of
 // columns k + 8 (l >> 4), k < 8), 16-lane row sums finish them, and lane

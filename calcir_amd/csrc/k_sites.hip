@@ -2,17 +2,26 @@
 // the exciton Hamiltonian build (gfx950).
 //
 // Field + sites (calcIR.cu:1020-1168 and the per-row part of get_kappa_GPU,
-// calcIR.cu:1245-1304): one lane per chromophore; the molecules of a frame
-// are staged in LDS tiles as SoA (FP32 oxygen for the cutoff decision,
-// real_t H1/H2/M' with the M site already relocated), so every lane reads
-// the tile from LDS instead of the strided AoS global array.  Field sums are
-// Neumaier-compensated.
+// calcIR.cu:1245-1304): one wave per chromophore.  Its lanes test 64 molecules
+// at a time against the cutoff (oxygens in LDS) and collect the ones inside in
+// a list; the field of the listed molecules is then summed 64 at a time.  With
+// a lane per chromophore and the field evaluated where a molecule lies inside,
+// nearly every molecule lies inside some lane's sphere, so each wave evaluated
+// the field of all of them with 7% of its lanes (32 frames of 2048 OH: 1.72
+// ms, against 0.15 ms here).  Field sums are FP64 for FP32 sites and
+// Neumaier-compensated for FP64 ones.
 //
-// Hamiltonian (calcIR.cu:1306-1404): a 64x64 tile per workgroup over the
-// site records; every element is computed once, the tile is written
-// column-major with lanes along the row index (coalesced), and the
-// transition-dipole formula is evaluated in a symmetric operation order so
-// that H(i,j) == H(j,i) bit for bit.
+// Hamiltonian (calcIR.cu:1306-1404): a 64x64 tile on or below the diagonal per
+// workgroup over the site records; every element is computed once and written
+// to both triangles, lanes along the rows of each (the mirrored tile through
+// LDS), so H(i,j) == H(j,i) bit for bit.  Bound by its arithmetic (about 60
+// instructions an element).  32 frames of 2048 OH in FP32: 0.44
+// ms with every element of both triangles computed, 0.26 ms here, against 0.105
+// ms for writing H at the rate of a large copy.
+
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
 
 #include "common.hpp"
 #include "sites.hpp"
@@ -21,26 +30,69 @@
 namespace cir {
 
 constexpr int kFieldBlock = 256;
-constexpr int kFieldTile = 256;  // molecules staged per LDS tile
+constexpr int kFieldWaves = kFieldBlock / 64;
+constexpr int kFieldChrom = 16;    // chromophores per workgroup
+constexpr int kFieldTile = 4096;   // molecules whose oxygens are staged in LDS at a time (48 KB)
 
 // The discrete cutoff decision (calcIR.cu:1106-1113), always in FP32 with
-// the reference's operation order, identical in every precision form.
+// the reference's operation order, identical in every precision form:
+// !(sqrt(r2) > cutoff) with the correctly rounded root, as a comparison of r2
+// with the largest value whose root does not exceed the cutoff
+// (cutoff_square, on the host: the rounded root is monotonic).
 __device__ __forceinline__ bool within_cutoff(float ox, float oy, float oz, float hx, float hy,
-                                              float hz, const PBox<float>& B, float cutoff) {
+                                              float hz, const PBox<float>& B, float cut2) {
 #pragma clang fp contract(off)
     float d0 = ox - hx, d1 = oy - hy, d2 = oz - hz;
     minimage3<float>(d0, d1, d2, B);
-    const float r = __fsqrt_rn(d0 * d0 + d1 * d1 + d2 * d2);
-    return !(r > cutoff);
+    return !(d0 * d0 + d1 * d1 + d2 * d2 > cut2);
 }
+
+float cutoff_square(float cutoff) {
+    if (std::isnan(cutoff) || std::isinf(cutoff)) return cutoff;
+    if (cutoff < 0.f) return -1.f;  // no separation is below a negative cutoff
+    float t = cutoff * cutoff;
+    if (std::isinf(t)) t = FLT_MAX;
+    while (t > 0.f && std::sqrt(t) > cutoff) t = std::nextafter(t, 0.f);
+    for (;;) {
+        const float u = std::nextafter(t, INFINITY);
+        if (std::isinf(u) || std::sqrt(u) > cutoff) return t;
+        t = u;
+    }
+}
+
+// Sum over a wave's lanes of a field component: FP64 for FP32 sites, whose
+// terms carry FP32 rounding; compensated pairs for FP64 sites.
+template <typename T>
+struct FieldSum;
+template <>
+struct FieldSum<float> {
+    double s = 0.0;
+    __device__ __forceinline__ void add(float v) { s += double(v); }
+    __device__ __forceinline__ float total() const { return float(wave_sum(s)); }
+};
+template <>
+struct FieldSum<double> {
+    Compensated<double> s;
+    __device__ __forceinline__ void add(double v) { s.add(v); }
+    __device__ __forceinline__ double total() const {
+        Compensated<double> t = s;
+        for (int off = 32; off > 0; off >>= 1) {
+            const double os = __shfl_xor(t.sum, off, 64), oc = __shfl_xor(t.c, off, 64);
+            t.add(os);
+            t.c += oc;
+        }
+        return t.value();
+    }
+};
 
 template <typename T>
 __global__ void __launch_bounds__(kFieldBlock)
-eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int rules, float cutoff,
+eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int rules, float cut2,
                    const float* __restrict__ xyz, const float* __restrict__ box, int boxk, MapT<T> mc,
                    T* __restrict__ sites) {
-    __shared__ float sO[3][kFieldTile];
-    __shared__ T sA[9][kFieldTile];  // H1, H2, negative site (x,y,z each)
+    extern __shared__ float sO[];  // x, y, z of min(nmol, kFieldTile) oxygens
+    __shared__ int list[kFieldWaves][128];
+    __shared__ T sE[kFieldChrom][3];
 
     const int f = blockIdx.y;
     const int nmol = natoms / natom_mol;
@@ -54,43 +106,53 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
     // msite_bisector rule builds one for it instead.
     const bool built_m = (rules & kRuleMsiteBisector) && natom_mol == 3;
     const bool have_m = natom_mol >= 4 || built_m;
-
-    const int chrom = blockIdx.x * kFieldBlock + threadIdx.x;
-    const bool active = chrom < N;
-    const int n = active ? chrom / nchrom_mol : 0;
     // calcIR.cu:1061-1070 picks H1 or H2 by chrom % 2 whatever nchrom_mol is
     // (with nchrom_mol 1, even molecules use H1 and odd ones H2); the
     // oh_per_molecule rule takes H(1 + chrom % nchrom_mol).
-    const int hatom = 1 + ((rules & kRuleOhPerMolecule) ? chrom % nchrom_mol : chrom % 2);
-    float hxf = 0, hyf = 0, hzf = 0;
-    if (active) {
-        hxf = x[3 * (n * natom_mol + hatom) + 0];
-        hyf = x[3 * (n * natom_mol + hatom) + 1];
-        hzf = x[3 * (n * natom_mol + hatom) + 2];
-    }
-    const T hx = T(hxf), hy = T(hyf), hz = T(hzf);
+    auto hatom_of = [&](int chrom) {
+        return 1 + ((rules & kRuleOhPerMolecule) ? chrom % nchrom_mol : chrom % 2);
+    };
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c0 = blockIdx.x * kFieldChrom;
+    const int ts = min(nmol, kFieldTile);  // pitch of the staged coordinates
     const T bohr = T(kBohrPerNm);
-    Compensated<T> ex, ey, ez;
-
-    for (int m0 = 0; m0 < nmol; m0 += kFieldTile) {
-        const int cnt = min(kFieldTile, nmol - m0);
+    auto stage = [&](int m0) {
+        const int cnt = min(ts, nmol - m0);
+        for (int t = tid; t < cnt; t += kFieldBlock) {
+            const float* mx = x + 3 * size_t(m0 + t) * natom_mol;
+            sO[t] = mx[0];
+            sO[ts + t] = mx[1];
+            sO[2 * ts + t] = mx[2];
+        }
+    };
+    if (nmol <= kFieldTile) {
+        stage(0);
         __syncthreads();
-        for (int t = threadIdx.x; t < cnt; t += kFieldBlock) {
-            const float* mx = x + 3 * size_t((m0 + t) * natom_mol);
-            const float ox = mx[0], oy = mx[1], oz = mx[2];
-            sO[0][t] = ox;
-            sO[1][t] = oy;
-            sO[2][t] = oz;
-            for (int c = 0; c < 3; ++c) {
-                sA[0 + c][t] = T(mx[3 + c]);
-                sA[3 + c][t] = T(mx[6 + c]);
-            }
-            const T o[3] = {T(ox), T(oy), T(oz)};
-            T m[3] = {T(0), T(0), T(0)};
+    }
+    // every wave of a workgroup runs the same number of chromophores, so the
+    // barriers of the staged tiles are reached by all of them
+#pragma unroll 1
+    for (int q = wave; q < kFieldChrom; q += kFieldWaves) {
+        const int chrom = c0 + q;
+        const bool active = chrom < N;
+        const int n = active ? chrom / nchrom_mol : 0;
+        const float* xh = x + 3 * (size_t(n) * natom_mol + hatom_of(active ? chrom : 0));
+        const float hxf = xh[0], hyf = xh[1], hzf = xh[2];
+        const T hx = T(hxf), hy = T(hyf), hz = T(hzf);
+        FieldSum<T> ex, ey, ez;
+        // the field of molecule m's charged sites at this chromophore's H
+        auto field = [&](int m) {
+            const float* mx = x + 3 * size_t(m) * natom_mol;
+            T a[9];
+#pragma unroll
+            for (int c = 0; c < 6; ++c) a[c] = T(mx[3 + c]);
+            const T o[3] = {T(mx[0]), T(mx[1]), T(mx[2])};
+            T ms[3] = {T(0), T(0), T(0)};
             if (built_m) {
                 // the TIP4P negative site on the HOH bisector, 0.015 nm from O
-                T h1[3] = {T(mx[3]) - o[0], T(mx[4]) - o[1], T(mx[5]) - o[2]};
-                T h2[3] = {T(mx[6]) - o[0], T(mx[7]) - o[1], T(mx[8]) - o[2]};
+                T h1[3] = {a[0] - o[0], a[1] - o[1], a[2] - o[2]};
+                T h2[3] = {a[3] - o[0], a[4] - o[1], a[5] - o[2]};
                 minimage3<T>(h1[0], h1[1], h1[2], Bt);
                 minimage3<T>(h2[0], h2[1], h2[2], Bt);
                 const T r1 = sqrt(h1[0] * h1[0] + h1[1] * h1[1] + h1[2] * h1[2]);
@@ -98,54 +160,86 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
                 T bi[3];
                 for (int c = 0; c < 3; ++c) bi[c] = h1[c] / r1 + h2[c] / r2;
                 const T rb = sqrt(bi[0] * bi[0] + bi[1] * bi[1] + bi[2] * bi[2]);
-                for (int c = 0; c < 3; ++c) m[c] = o[c] + T(kOMTip4p) * bi[c] / rb;
+                for (int c = 0; c < 3; ++c) ms[c] = o[c] + T(kOMTip4p) * bi[c] / rb;
             } else if (have_m) {
-                m[0] = T(mx[9]);
-                m[1] = T(mx[10]);
-                m[2] = T(mx[11]);
+                for (int c = 0; c < 3; ++c) ms[c] = T(mx[9 + c]);
                 if (imodel != 0) {
                     // calcIR.cu:1124-1140: M moved to 0.015 nm along O->M
-                    T om[3] = {m[0] - o[0], m[1] - o[1], m[2] - o[2]};
+                    T om[3] = {ms[0] - o[0], ms[1] - o[1], ms[2] - o[2]};
                     minimage3<T>(om[0], om[1], om[2], Bt);
                     const T rom = sqrt(om[0] * om[0] + om[1] * om[1] + om[2] * om[2]);
-                    for (int c = 0; c < 3; ++c) m[c] = o[c] + T(kOMTip4p) * om[c] / rom;
+                    for (int c = 0; c < 3; ++c) ms[c] = o[c] + T(kOMTip4p) * om[c] / rom;
                 }
             }
-            for (int c = 0; c < 3; ++c) sA[6 + c][t] = m[c];
-        }
-        __syncthreads();
-        if (!active) continue;
-        for (int t = 0; t < cnt; ++t) {
-            const int m = m0 + t;
-            if (m == n) continue;  // calcIR.cu:1099
-            if (!within_cutoff(sO[0][t], sO[1][t], sO[2][t], hxf, hyf, hzf, Bf, cutoff)) continue;
-            for (int s = 0; s < (have_m ? 3 : 2); ++s) {
-                T dx = hx - sA[3 * s + 0][t], dy = hy - sA[3 * s + 1][t], dz = hz - sA[3 * s + 2][t];
+            for (int c = 0; c < 3; ++c) a[6 + c] = ms[c];
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+                if (s == 2 && !have_m) break;
+                T dx = hx - a[3 * s + 0], dy = hy - a[3 * s + 1], dz = hz - a[3 * s + 2];
                 minimage3<T>(dx, dy, dz, Bt);
                 dx = dx * bohr;
                 dy = dy * bohr;
                 dz = dz * bohr;
                 const T r = sqrt(dx * dx + dy * dy + dz * dz);
-                const T q = (s < 2) ? T(kQH) : T(-kQM);
-                const T qr3 = q / (r * r * r);
+                const T qc = (s < 2) ? T(kQH) : T(-kQM);
+                const T qr3 = qc / (r * r * r);
                 ex.add(qr3 * dx);
                 ey.add(qr3 * dy);
                 ez.add(qr3 * dz);
             }
+        };
+        int cnt = 0;  // molecules in the wave's list
+        int* const lw = list[wave];
+        for (int m0 = 0; m0 < nmol; m0 += kFieldTile) {
+            if (nmol > kFieldTile) {
+                __syncthreads();
+                stage(m0);
+                __syncthreads();
+            }
+            const int tc = min(ts, nmol - m0);
+            for (int t0 = 0; t0 < tc; t0 += 64) {
+                const int t = t0 + lane, ti = min(t, tc - 1);
+                const bool in = within_cutoff(sO[ti], sO[ts + ti], sO[2 * ts + ti], hxf, hyf, hzf, Bf, cut2) &&
+                                t < tc && active && m0 + t != n;  // calcIR.cu:1099
+                const unsigned long long mask = __ballot(in);
+                if (mask == 0) continue;
+                if (in) lw[cnt + __popcll(mask & ((1ull << lane) - 1))] = m0 + t;
+                cnt += __popcll(mask);
+                if (cnt >= 64) {
+                    wave_lds_sync();
+                    field(lw[lane]);
+                    cnt -= 64;
+                    const int left = lw[64 + lane];
+                    wave_lds_sync();
+                    if (lane < cnt) lw[lane] = left;
+                    wave_lds_sync();
+                }
+            }
+        }
+        wave_lds_sync();
+        if (lane < cnt) field(lw[lane]);
+        const T tx = ex.total(), ty = ey.total(), tz = ez.total();
+        if (lane == 0) {
+            sE[q][0] = tx;
+            sE[q][1] = ty;
+            sE[q][2] = tz;
         }
     }
-    if (!active) return;
+    __syncthreads();
+    const int chrom = c0 + tid;
+    if (tid >= kFieldChrom || chrom >= N) return;
 
     // own OH unit vector, TDM position and maps (calcIR.cu:1047-1080, 1253-1304)
-    const float* no = x + 3 * size_t(n * natom_mol);
+    const float* no = x + 3 * size_t(chrom / nchrom_mol) * natom_mol;
+    const float* nh = no + 3 * hatom_of(chrom);
     const T ox = T(no[0]), oy = T(no[1]), oz = T(no[2]);
-    T ux = hx - ox, uy = hy - oy, uz = hz - oz;
+    T ux = T(nh[0]) - ox, uy = T(nh[1]) - oy, uz = T(nh[2]) - oz;
     minimage3<T>(ux, uy, uz, Bt);
     const T r = sqrt(ux * ux + uy * uy + uz * uz);
     ux /= r;
     uy /= r;
     uz /= r;
-    const T E = ex.value() * ux + ey.value() * uy + ez.value() * uz;
+    const T E = sE[tid][0] * ux + sE[tid][1] * uy + sE[tid][2] * uz;
     const T w = mc.w0 + mc.w1 * E + mc.w2 * E * E;
     const T xx = mc.x0 + mc.x1 * w;
     const T p = mc.p0 + mc.p1 * w;
@@ -185,6 +279,9 @@ hamiltonian_kernel(int N, int ld, int nchrom_mol, int hod, T avef, T wi0, T wi1,
     // per-tile site data: E, w, x, p, s = x*mup, u(3), r(3)
     __shared__ T rs[11][kHTile];
     __shared__ T cs[11][kHTile];
+    __shared__ T mir[kHTile][kHTile + 1];
+    // tiles on or below the diagonal (with the padding rows below N)
+    if (blockIdx.x < blockIdx.y) return;
     const int f = blockIdx.z;
     const int i0 = blockIdx.x * kHTile, j0 = blockIdx.y * kHTile;
     const T* S = sites + size_t(f) * CIR_NSITE * N;
@@ -212,8 +309,8 @@ hamiltonian_kernel(int N, int ld, int nchrom_mol, int hod, T avef, T wi0, T wi1,
     const PBox<T> bb = load_box<T>(box, boxk, f);
     const int tx = tid % kHTile, ty = tid / kHTile;
     const int i = i0 + tx;
-    if (i >= ld) return;
     T* Hf = H + size_t(f) * N * ld;
+    const bool mirror = i0 != j0;
     for (int q = 0; q < kHTile / 4; ++q) {
         const int jl = ty + 4 * q;
         const int j = j0 + jl;
@@ -235,7 +332,16 @@ hamiltonian_kernel(int N, int ld, int nchrom_mol, int hod, T avef, T wi0, T wi1,
                                         cs[5][jl], cs[6][jl], cs[7][jl], cs[8][jl], cs[9][jl], cs[10][jl], bb);
             h = g * (rs[4][tx] * cs[4][jl]) * T(kCmPerHartree);
         }
-        Hf[size_t(j) * ld + i] = h;
+        if (i < ld) Hf[size_t(j) * ld + i] = h;
+        if (mirror) mir[jl][tx] = h;
+    }
+    if (!mirror) return;
+    // the same elements above the diagonal: column i0 + c, rows j0 + lane
+    __syncthreads();
+    const int j = j0 + tx;
+    for (int q = 0; q < kHTile / 4; ++q) {
+        const int c = ty + 4 * q;
+        if (i0 + c < N && j < N) Hf[size_t(i0 + c) * ld + j] = mir[tx][c];
     }
 }
 
@@ -244,9 +350,11 @@ int launch_eproj_sites(int nframes, int natoms, int natom_mol, int nchrom_mol, i
                        float cutoff, const float* xyz, const float* box, int boxk, const MapCoef& mc,
                        void* sites, hipStream_t s) {
     const int N = (natoms / natom_mol) * nchrom_mol;
-    dim3 grid(unsigned(ceil_div(N, kFieldBlock)), unsigned(nframes));
-    hipLaunchKernelGGL(eproj_sites_kernel<T>, grid, dim3(kFieldBlock), 0, s, natoms, natom_mol,
-                       nchrom_mol, imodel, rules, cutoff, xyz, box, boxk, map_t<T>(mc), static_cast<T*>(sites));
+    dim3 grid(unsigned(ceil_div(N, kFieldChrom)), unsigned(nframes));
+    const size_t sm = size_t(std::min(natoms / natom_mol, kFieldTile)) * 3 * sizeof(float);
+    hipLaunchKernelGGL(eproj_sites_kernel<T>, grid, dim3(kFieldBlock), sm, s, natoms, natom_mol,
+                       nchrom_mol, imodel, rules, cutoff_square(cutoff), xyz, box, boxk, map_t<T>(mc),
+                       static_cast<T*>(sites));
     CIR_CHECK_LAUNCH();
     return CIR_OK;
 }

@@ -27,15 +27,20 @@ __device__ __forceinline__ T tdc_geometry(T uix, T uiy, T uiz, T rix, T riy, T r
                                           T rjy, T rjz, const PBox<T>& bb) {
     T dr[3] = {rix - rjx, riy - rjy, riz - rjz};
     minimage3<T>(dr[0], dr[1], dr[2], bb);
-    const T r = sqrt(dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2]);
-    const T inv = T(1) / r;
+    const T r2 = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+    // 1 / r: the hardware's reciprocal root is within one ulp in FP32
+    T inv;
+    if constexpr (sizeof(T) == 4)
+        inv = __builtin_amdgcn_rsqf(r2);
+    else
+        inv = T(1) / sqrt(r2);
     const T d0 = dr[0] * inv, d1 = dr[1] * inv, d2 = dr[2] * inv;
     const T uu = uix * ujx + uiy * ujy + uiz * ujz;
     const T ur = uix * d0 + uiy * d1 + uiz * d2;
     const T vr = ujx * d0 + ujy * d1 + ujz * d2;
-    const T rb = r * T(kBohrPerNm);
+    const T ib = inv * T(1.0 / kBohrPerNm);
     const T t = ur * vr;
-    return (uu - T(3) * t) / (rb * rb * rb);
+    return (uu - T(3) * t) * (ib * ib * ib);
 }
 
 }  // namespace cir
