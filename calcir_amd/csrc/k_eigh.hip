@@ -51,9 +51,9 @@ constexpr int kBtPass = 2 * kBtNB;  // reflectors per back-transform pass over Z
 constexpr int kEigNT = 256;  // threads per block of bisection / inverse iteration
 constexpr double kClusterRel = 1e-7;
 constexpr int kMaxCluster = 128;
-constexpr int kSingleMinN = 512;     // matrices at least this large run the whole-GPU tridiagonalisation
-constexpr int kSingleMaxBatch = 16;  //   in batches of at most this many (one workgroup per
-                                     //   matrix needs more matrices to fill the GPU)
+constexpr int kSingleMinN = 512;     // matrices at least this large may run the whole-GPU tridiagonalisation
+constexpr int kSingleMaxBatch = 16;  //   in batches of at most this many
+constexpr int kSinglePer = 512;      //   and at most n / kSinglePer (use_whole_gpu)
 
 // Eigenvalue k joins the cluster of k-1 (ascending w).
 __device__ __forceinline__ bool joins_cluster(const double* w, int k) {
@@ -1669,28 +1669,190 @@ yt_kernel(int n, int ld, int j0, int off, int kb, int mrows, const T* __restrict
 
 inline size_t larft_smem_bytes(size_t esz) { return (size_t(kBtNB) * (kBtNB + 1) + kBtNB) * esz; }
 
-// The FP32 batched path can reduce to tridiagonal form in two stages
-// (k_band.hip); the few-matrix whole-GPU path and FP64 reduce in one stage.
-// CIR_EIGH_STAGES=1 or 2 in the environment forces one form where both apply
-// (tests compare them); otherwise the two-stage form is taken from
-// kTwoStageMinN on (at 256 matrices per batch the two forms take the same
-// time near n = 1024; at n = 2048 the two-stage form takes 12% less).
-constexpr int kTwoStageMinN = 1024;
-inline bool use_two_stage(size_t esz, int batch, int n) {
+// How a batch is reduced to tridiagonal form:
+//   two stages (k_band.hip)   FP32 up to sb_max_n(), from kTwoStageMinN on
+//   one stage, whole GPU      a few matrices, one at a time, a grid per step
+//   one stage, batched        one workgroup per matrix
+// The lines, from both sides measured (ms per batch): two stages against one
+// workgroup per matrix, 64 matrices, n = 320 5.1 / 4.6, n = 400 7.0 / 6.8, n =
+// 512 9.5 / 10.7, n = 640 13.4 / 17.1, 24 of n = 1000 23.8 / 43; against the
+// whole-GPU form, one matrix of n = 512 8.8 / 13.8, n = 1024 22.6 / 30.7, n =
+// 2048 66.5 / 73.5, 8 of n = 512 8.9 / 104.  The whole-GPU form takes a time
+// that grows with the batch (n = 1024 in FP64: 27 per matrix), the batched form
+// one that does not up to a matrix per CU (76), and the ratio of the two grows
+// with n: the whole-GPU form runs batches of up to n / kSinglePer matrices.
+// CIR_EIGH_STAGES=1 or 2 in the environment forces one or two stages where
+// both apply (tests compare them).
+constexpr int kTwoStageMinN = 448;
+inline bool use_two_stage(size_t esz, int n) {
     if (esz != sizeof(float) || n > sb_max_n() || n < 2 * kBandNB + 2) return false;
     if (deterministic_mode()) return true;  // the form without float atomics
-    if (n >= kSingleMinN && batch <= kSingleMaxBatch) return false;
     const char* fv = std::getenv("CIR_EIGH_STAGES");
     const int forced = fv ? std::atoi(fv) : 0;
     if (forced == 1) return false;
     if (forced == 2) return true;
     return n >= kTwoStageMinN;
 }
+inline bool use_whole_gpu(int batch, int n) {
+    return n >= kSingleMinN && batch <= kSingleMaxBatch && int64_t(batch) * kSinglePer <= n;
+}
+
+// The two-stage form's T carries the rounding of N bulge-chasing sweeps over
+// every element of the band: in FP32 about three times the one-stage form's
+// backward error (2048-OH Hamiltonians: eigenvalues 6.5e-7 against 2.1e-7 of
+// the spectrum, spectral density 1.7e-6 against 4e-7).  Where the reduction is
+// bound by its chains rather than by its arithmetic (small matrices, small
+// batches) three N^3 products cost little, and the eigenpairs get one step of
+// first-order correction from a copy of H: with the residuals C = H V - V L
+// and D = V^T C, lambda_j += D_jj and V += V E, E_ij = D_ij / (lambda_j -
+// lambda_i).  E is antisymmetric, so V stays orthogonal to second order.
+// Only C needs FP32's full accuracy (H's diagonal, its largest entries, is
+// taken out of the product and applied in FP64 with the eigenvalue); D and E
+// are corrections, formed in split-BF16x3.  After it: eigenvalues 1.6e-7, the
+// density 4e-7.  One matrix of n = 2048: 0.8 of 66 ms; 48 of n = 766: 1.7 of 18.
+constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16;
+inline bool use_refine(int batch, int n) { return n < kRefineMaxN || batch <= kRefineMaxBatch; }
+
+constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
+// C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major:
+// 64 x 64 tiles, four waves of one 32x32 fragment on the FP32 MFMA.
+__global__ void __launch_bounds__(256)
+residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __restrict__ Vall,
+                const double* __restrict__ wall, float* __restrict__ Call) {
+    __shared__ float As[kRqK][kRqT + 4], Bs[kRqK][kRqT + 4];
+    const int b = blockIdx.z, m0 = blockIdx.y * kRqT, n0 = blockIdx.x * kRqT;
+    const float* H = Hall + size_t(b) * n * ld;
+    const float* V = Vall + size_t(b) * n * ld;
+    float* C = Call + size_t(b) * n * ld;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
+    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    // each thread stages 4 values of either operand, 64 consecutive ones per wave
+    const int c = tid & 63, k0 = tid >> 6;
+    const int cm = min(m0 + c, n - 1), cn = min(n0 + c, n - 1);
+    float ra[4], rb[4];
+    auto load = [&](int kb) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = kb + k0 + 4 * q, kc = min(k, n - 1);
+            ra[q] = (kc == cm) ? 0.f : H[size_t(kc) * ld + cm];
+            rb[q] = (k < n) ? V[size_t(kc) * ld + cn] : 0.f;
+        }
+    };
+    floatx16 acc;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
+    load(0);
+    for (int kb = 0; kb < n; kb += kRqK) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            As[k0 + 4 * q][c] = ra[q];
+            Bs[k0 + 4 * q][c] = rb[q];
+        }
+        __syncthreads();
+        load(kb + kRqK);
+#pragma unroll
+        for (int k = 0; k < kRqK; k += 2)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[k + h][wm + l32], Bs[k + h][wn + l32], acc, 0, 0, 0);
+    }
+    const int k = n0 + wn + l32;
+    const double lam = wall[size_t(b) * n + min(k, n - 1)];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int i = m0 + wm + 8 * (q >> 2) + 4 * h + (q & 3);
+        if (i < n && k < n) {
+            const double v = double(V[size_t(i) * ld + k]);
+            C[size_t(i) * ld + k] = float(double(acc[q]) + (double(H[size_t(i) * ld + i]) - lam) * v);
+        }
+    }
+}
+
+// D -> E in place, the diagonal of D into dl.  E takes the symmetric part of
+// D: its antisymmetric part is V's own loss of orthogonality and the product's
+// rounding, which divided by small gaps would make it worse.  Pairs whose gap
+// is not large against D_ij are left as they are: a rotation by E_ij taken to
+// first order lengthens its vectors by E_ij^2, which the bound keeps below
+// FP32's rounding, and what a pair's mixing does to the results is D_ij against
+// the frequencies that they resolve, whatever the gap.  One workgroup per tile
+// on or above the diagonal and its mirror image.
+constexpr double kRotationGap = 2048.0;
+constexpr int kRotT = 32;
+__global__ void __launch_bounds__(256)
+rotation_kernel(int n, int ld, const double* __restrict__ wall, float* __restrict__ Dall, float* __restrict__ dlall) {
+    __shared__ float lo[kRotT][kRotT + 1];  // the mirror tile, then its new values
+    const int I = blockIdx.y * kRotT, J = blockIdx.x * kRotT, b = blockIdx.z;
+    if (I > J) return;
+    const double* w = wall + size_t(b) * n;
+    float* D = Dall + size_t(b) * n * ld;
+    const int c = threadIdx.x % kRotT, r0 = threadIdx.x / kRotT;
+    for (int r = r0; r < kRotT; r += 256 / kRotT)
+        if (J + r < n && I + c < n) lo[r][c] = D[size_t(J + r) * ld + I + c];
+    __syncthreads();
+    float up[kRotT * kRotT / 256];
+#pragma unroll
+    for (int q = 0; q < kRotT * kRotT / 256; ++q) {
+        const int r = r0 + q * (256 / kRotT), i = I + r, j = J + c;
+        up[q] = 0.f;
+        if (i < n && j < n) {
+            const double d = 0.5 * (double(D[size_t(i) * ld + j]) + double(lo[c][r]));
+            const double gap = w[j] - w[i];
+            if (i == j) dlall[size_t(b) * n + j] = float(d);
+            if (i != j && fabs(gap) > kRotationGap * fabs(d)) up[q] = float(d / gap);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kRotT * kRotT / 256; ++q) {
+        const int r = r0 + q * (256 / kRotT), i = I + r, j = J + c;
+        if (i < n && j < n) D[size_t(i) * ld + j] = up[q];
+        lo[c][r] = -up[q];
+    }
+    __syncthreads();
+    if (I != J)
+        for (int r = r0; r < kRotT; r += 256 / kRotT)
+            if (J + r < n && I + c < n) D[size_t(J + r) * ld + I + c] = lo[r][c];
+}
+
+// w_k += dl_k, then kept ascending (a running maximum: neighbours closer than
+// the corrections' own error may come out exchanged).  One workgroup per matrix.
+__global__ void __launch_bounds__(1024)
+correct_w_kernel(int n, const float* __restrict__ dlall, double* __restrict__ wall) {
+    extern __shared__ __align__(16) double sw_[];  // 2 n
+    const int b = blockIdx.x;
+    double* w = wall + size_t(b) * n;
+    for (int k = threadIdx.x; k < n; k += 1024) sw_[k] = w[k] + double(dlall[size_t(b) * n + k]);
+    double* a = sw_;
+    double* c = sw_ + n;
+    for (int off = 1; off < n; off <<= 1) {
+        __syncthreads();
+        for (int k = threadIdx.x; k < n; k += 1024) c[k] = (k >= off) ? fmax(a[k], a[k - off]) : a[k];
+        double* t = a;
+        a = c;
+        c = t;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < n; k += 1024) w[k] = a[k];
+}
+
+// V += P over n rows of pitch ld (columns past n: P's are not defined)
+__global__ void __launch_bounds__(256)
+add_rows_kernel(int n, int ld, const float* __restrict__ Pall, float* __restrict__ Vall) {
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j >= n) return;
+    const size_t o = (size_t(blockIdx.z) * n + blockIdx.y) * ld + j;
+    Vall[o] += Pall[o];
+}
+
+// The matrices' copy for the refinement
+__global__ void __launch_bounds__(256)
+copy4_kernel(int64_t cnt, const float4* __restrict__ src, float4* __restrict__ dst) {
+    for (int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x; q < cnt; q += int64_t(gridDim.x) * 256) dst[q] = src[q];
+}
 
 struct EighWork {
     size_t off_d, off_e, off_tau, off_vw, off_g, off_t, off_w1, off_w2, off_s1, off_scr, total;
-    size_t off_bnd, off_p1, off_p2, off_yh, off_mm, off_q2;  // two-stage buffers
-    bool two;
+    size_t off_bnd, off_p1, off_p2, off_yh, off_mm, off_q2, off_h, off_r;  // two-stage buffers
+    bool two, refine;
     int sub;  // matrices per inverse-iteration pass
 };
 
@@ -1698,7 +1860,7 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
     EighWork L{};
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t o = 0;
-    L.two = use_two_stage(esz, batch, n);
+    L.two = use_two_stage(esz, n);
     if (L.two) {
         L.off_bnd = o;
         o = al(o + esz * batch * size_t(n) * kBandW);
@@ -1712,6 +1874,11 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
         o = al(o + esz * batch * size_t(kBandNB) * kBandNB);
         L.off_q2 = o;
         o = al(o + esz * batch * size_t(q2_blocks(n)) * kQ2BlockFloats);
+        L.refine = use_refine(batch, n);
+        L.off_h = o;
+        if (L.refine) o = al(o + esz * batch * size_t(n) * ld);
+        L.off_r = o;
+        if (L.refine) o = al(o + esz * batch * size_t(n) * ld);
     }
     L.off_d = o;
     o = al(o + esz * batch * n);
@@ -1765,6 +1932,13 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
             float* q2 = reinterpret_cast<float*>(work + L.off_q2);
             {
                 ProfScope ps(prof, CIR_PH_TRIDIAG, s);
+                if (L.refine) {
+                    const int64_t cnt = int64_t(batch) * n * ld / 4;
+                    hipLaunchKernelGGL(copy4_kernel, dim3(unsigned(std::min<int64_t>(ceil_div(cnt, 256), 8192))), dim3(256),
+                                       0, s, cnt, reinterpret_cast<const float4*>(A),
+                                       reinterpret_cast<float4*>(work + L.off_h));
+                    CIR_CHECK_LAUNCH();
+                }
                 CIR_TRY(sy2sb(batch, n, ld, A, bnd, tau, reinterpret_cast<float*>(work + L.off_p1),
                               reinterpret_cast<float*>(work + L.off_yh), reinterpret_cast<float*>(work + L.off_mm),
                               s));
@@ -1775,7 +1949,7 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
         }
     }
     if (L.two) {
-    } else if (n >= kSingleMinN && batch <= kSingleMaxBatch) {
+    } else if (use_whole_gpu(batch, n)) {
         ProfScope ps(prof, CIR_PH_TRIDIAG, s);
         T* s1 = reinterpret_cast<T*>(work + L.off_s1);
         for (int b = 0; b < batch; ++b)
@@ -1905,6 +2079,43 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
             CIR_CHECK_LAUNCH();
         }
         CIR_TRY(mm(mrows, n, kb, W1, P, 1, pn, W2, 1, P, pn, Zs, ld, 1, mat, -1.0, 1.0));
+    }
+    if constexpr (sizeof(T) == sizeof(float)) {
+        if (L.refine) {
+            float* H = reinterpret_cast<float*>(work + L.off_h);  // then D, E
+            float* C = reinterpret_cast<float*>(work + L.off_r);  // then V E
+            float* dl = reinterpret_cast<float*>(W1);             // free now: batch x n
+            const int64_t mat = int64_t(n) * ld;
+            const unsigned nt = unsigned(ceil_div(n, kRqT)), nc = unsigned(ceil_div(n, 256)),
+                           nr = unsigned(ceil_div(n, kRotT));
+            hipLaunchKernelGGL(residual_kernel, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, H, V, w, C);
+            CIR_CHECK_LAUNCH();
+            auto product = [&](const float* a, int64_t a_m, int64_t a_k, const float* bb, float* c) {
+                GemmArgs g;
+                g.M = g.N = g.K = n;
+                g.batch = batch;
+                g.A = a;
+                g.a_m = a_m;
+                g.a_k = a_k;
+                g.B = bb;
+                g.b_k = ld;
+                g.b_n = 1;
+                g.C = c;
+                g.c_m = ld;
+                g.c_n = 1;
+                g.a_b = g.b_b = g.c_b = mat;
+                return gemm(CIR_PREC_BF16X3, g, s);
+            };
+            CIR_TRY(product(V, 1, ld, C, H));
+            hipLaunchKernelGGL(rotation_kernel, dim3(nr, nr, unsigned(batch)), dim3(256), 0, s, n, ld, w, H, dl);
+            CIR_CHECK_LAUNCH();
+            CIR_TRY(product(V, ld, 1, H, C));
+            hipLaunchKernelGGL(add_rows_kernel, dim3(nc, unsigned(n), unsigned(batch)), dim3(256), 0, s, n, ld, C, V);
+            CIR_CHECK_LAUNCH();
+            hipLaunchKernelGGL(correct_w_kernel, dim3(unsigned(batch)), dim3(1024), 2 * size_t(n) * sizeof(double), s, n, dl,
+                               w);
+            CIR_CHECK_LAUNCH();
+        }
     }
     return CIR_OK;
 }
