@@ -566,11 +566,9 @@ static_assert(kBandNB * (kBandW / 4) <= kSbNT, "one step's new band rows must fi
 static_assert((2 * kSbG - 1) * kBandNB + kBandNB <= kSbWR, "window must hold a step's rows plus the read-ahead");
 
 
-// Row r of a group's band is stream row v = r + off (sb_stream), which sits in
-// window row v mod kSbWR; its element (r, c), r - c < kBandW, is at
-// sb_rowbase(r, off) - c.
-__device__ __forceinline__ int sb_rowbase(int r, int off) { return ((r + off) & (kSbWR - 1)) * kSbWP + r; }
-
+// Row r of a group's band is stream row v = r + off (SbStream), which sits in
+// window row v mod kSbWR; its element (r, c), r - c < kBandW, is r - c floats
+// into that row.
 // The groups' band rows as one stream.  Group g (sweeps kSbG g ..) starts at
 // step st(g) and its row r is stream row r - kSbG g + 32 st(g), so that task k
 // of the group's wave j, at step t = st(g) + k + 2 j, works on the 32 stream
@@ -609,53 +607,108 @@ __device__ __forceinline__ float from_low_half(float x) {
     return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[0]);
 }
 
+// Householder scalars for a vector with first element alpha and tail square sum
+// sigma > 0: beta = -sign(alpha) |x|, tau = (beta - alpha) / beta, scale = 1 /
+// (alpha - beta).  |x| from the hardware's reciprocal root y with one
+// Newton step each way (the residual of |x|^2, of tau beta and of scale
+// (alpha - beta), each by one FMA, so each result is within an ulp); the IEEE
+// root and quotients are three chains of a dozen dependent instructions on a
+// task's critical path.  Squares too small for the hardware root take those.
+__device__ __forceinline__ void sb_householder(float alpha, float sigma, float& beta, float& tau, float& scale) {
+    const float a2 = alpha * alpha + sigma;
+    if (!(a2 >= 1e-30f && a2 <= 1e30f)) {
+        const float nrm = sqrtf(a2);
+        beta = alpha >= 0.f ? -nrm : nrm;
+        tau = (beta - alpha) / beta;
+        scale = 1.f / (alpha - beta);
+        return;
+    }
+    const float y = __builtin_amdgcn_rsqf(a2);
+    float nrm = a2 * y;
+    nrm = fmaf(fmaf(-nrm, nrm, a2), 0.5f * y, nrm);
+    beta = alpha >= 0.f ? -nrm : nrm;
+    const float yb = alpha >= 0.f ? -y : y;  // about 1 / beta
+    const float den = alpha - beta;
+    tau = -den * yb;
+    tau = fmaf(fmaf(-tau, beta, -den), yb, tau);
+    const float r = __builtin_amdgcn_rcpf(den);
+    scale = fmaf(fmaf(-den, r, 1.f), r, r);
+}
+
+// Sum over the 32 lanes of each half wave, in every lane of the half.
+__device__ __forceinline__ float half_sum(float x) {
+    x = brow_sum16(x);
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+
 // One wave's share of a bulge-chasing step: task (s, k) of its sweep.
 // Lane l: row i = l & 31 of the task's block, column half h = l >> 5
 // (columns 16 h .. 16 h + 15).  pv / ptau: the sweep's previous reflector
 // (columns of the previous block, this lane's half), replaced by this task's;
 // q2val: this task's reflector as a Q2 block column.  The wave's scratch sc
 // holds v, the two reduced vectors and a per-lane sink for masked-off stores.
-// Every window access is unconditional (lanes outside the block read a row
-// inside it and discard the value, or store to the sink), so the accesses of
-// a task issue back to back.  The diagonal block is read at the start (no
-// earlier part of the task writes it), and the left application to the block
-// below and the two-sided update of the diagonal block share one pass of
-// reductions.
-__device__ void sb_task(int n, int s, int k, int off, float* w, float* sc, float (&pv)[16], float& ptau, float& q2val,
-                        int lane) {
+// FULL: a block of 32 rows, every task but a sweep's last.  The last one's
+// lanes outside the block read a row inside it and discard the value.  All the
+// window's reads are issued together, the diagonal block's at the start (no
+// earlier part of the task writes it); read where they are used, the compiler
+// put each of the masked ones into a branch of its own with a wait behind it
+// (16 LDS latencies per task).  dofs: window offset of D(max(i, j), min(i, j))
+// for column j = 16 h + c, against the block's first row; rows are 64 floats,
+// so an offset past the window's end wraps with a mask.  The left application
+// to the block below and the two-sided update of the diagonal block share one
+// pass of reductions.
+template <bool FULL>
+__device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, float* sc, const int (&dofs)[16],
+                                        float (&pv)[16], float& ptau, float& q2val, int lane) {
     constexpr int NB = kBandNB;
+    constexpr int WMASK = kSbWR * kSbWP - 1;
     float* vs = sc;
     float* wsB = sc + NB;
     float* wsD = sc + 2 * NB;
     float* sink = sc + 3 * NB + lane;
     const int i = lane & 31, h = lane >> 5;
     const int r0 = s + 1 + k * NB;
-    const int len = min(NB, n - r0);
-    const int p0 = r0 - NB;
-    const bool rowok = i < len;
-    const int rb = sb_rowbase(r0 + min(i, len - 1), off);  // this lane's row (clamped into the block)
+    const int len = FULL ? NB : min(NB, n - r0);
+    const bool rowok = FULL || i < len;
+    const int R = ((r0 + off) & (kSbWR - 1)) * kSbWP;  // window offset of the block's first row
+    // this lane's row (clamped into the block): element (row, c) at wr[row - c]
+    const int ic = FULL ? i : min(i, len - 1);
+    float* const wr = w + ((R + ic * kSbWP) & WMASK);
     float bk[16], dd[16];
     float x = 0.f;
     if (k == 0) {
-        const float v = w[rb - s];
-        x = rowok ? v : 0.f;
+        x = wr[ic + 1];  // column s
     } else {
-        // the block below the previous one, columns p0 .. p0 + NB - 1
-        const float* bp = w + (rb - p0 - 16 * h - 15);
+        // the block below the previous one, columns r0 - NB + 16 h ..
+        const float* bp = wr + (NB + ic - 16 * h - 15);
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const float v = bp[15 - c];
-            bk[c] = rowok ? v : 0.f;
-        }
+        for (int c = 0; c < 16; ++c) bk[c] = bp[15 - c];
     }
     // the diagonal block D (rows/cols r0 .. r0+len-1), both triangles, from
     // its lower triangle
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
-        const int j = 16 * h + c;
-        const int ra = min(max(i, j), len - 1), cb = min(min(i, j), ra);
-        const float v = w[sb_rowbase(r0 + ra, off) - (r0 + cb)];
-        dd[c] = (rowok && j < len) ? v : 0.f;
+        if constexpr (FULL) {
+            dd[c] = w[(R + dofs[c]) & WMASK];
+        } else {
+            const int j = 16 * h + c, ra = min(max(i, j), len - 1), cb = min(min(i, j), ra);
+            dd[c] = w[(R + ra * kSbWP + ra - cb) & WMASK];
+        }
+    }
+    if constexpr (!FULL) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) asm volatile("" : "+v"(dd[c]));  // read above, masked here
+#pragma unroll
+        for (int c = 0; c < 16; ++c) dd[c] = (rowok && 16 * h + c < len) ? dd[c] : 0.f;
+        if (k == 0) {
+            x = rowok ? x : 0.f;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) asm volatile("" : "+v"(bk[c]));
+#pragma unroll
+            for (int c = 0; c < 16; ++c) bk[c] = rowok ? bk[c] : 0.f;
+        }
     }
     if (k > 0) {
         // the previous reflector from the right (this fills the bulge)
@@ -670,18 +723,12 @@ __device__ void sb_task(int n, int s, int k, int off, float* w, float* sc, float
         for (int c = 0; c < 16; ++c) bk[c] -= f * pv[c];
         x = from_low_half(bk[0]);  // the block's first column, from the h = 0 lanes
     }
-    // reflector annihilating x[1..len)
-    const float sq = (h == 0 && i >= 1 && i < len) ? x * x : 0.f;
-    const float sigma = bwave_sum(sq);
+    // reflector annihilating x[1..len) (x is the same in both halves)
+    const float sigma = half_sum((i >= 1 && rowok) ? x * x : 0.f);
     const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 0));
     float tau = 0.f, beta = alpha, scale = 0.f;
-    if (sigma > 0.f) {
-        const float nrm = sqrtf(alpha * alpha + sigma);
-        beta = alpha >= 0.f ? -nrm : nrm;
-        tau = (beta - alpha) / beta;
-        scale = 1.f / (alpha - beta);
-    }
-    const float vi = (i == 0) ? 1.f : (i < len ? x * scale : 0.f);
+    if (__builtin_amdgcn_readfirstlane(__float_as_int(sigma)) != 0) sb_householder(alpha, sigma, beta, tau, scale);
+    const float vi = (i == 0) ? 1.f : (rowok ? x * scale : 0.f);
     if (h == 0) vs[i] = vi;
     wave_lds_sync();
     float vj[16];
@@ -722,7 +769,7 @@ __device__ void sb_task(int n, int s, int k, int off, float* w, float* sc, float
         for (int c = 1; c < 8; ++c) zz = (ri == c) ? z[c] : zz;
         if (ri < 8) wsB[16 * h + 8 * ((lane >> 4) & 1) + ri] = zz;
     }
-    const float kk = bwave_sum(h == 0 ? pp * vi : 0.f);
+    const float kk = half_sum(pp * vi);  // (pp is the same in both halves)
     const float K = -0.5f * tau * kk;
     const float wi = pp + K * vi;
     if (h == 0) wsD[i] = wi;
@@ -740,12 +787,12 @@ __device__ void sb_task(int n, int s, int k, int off, float* w, float* sc, float
             }
         }
         if (rowok) {
-            float* bq = w + (rb - p0 - 16 * h - 15);
+            float* bq = wr + (NB + ic - 16 * h - 15);
 #pragma unroll
             for (int c = 0; c < 16; ++c) bq[15 - c] = bk[c];
         }
     } else if (h == 0 && rowok) {
-        w[rb - s] = (i == 0) ? beta : 0.f;
+        wr[ic + 1] = (i == 0) ? beta : 0.f;
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -755,7 +802,7 @@ __device__ void sb_task(int n, int s, int k, int off, float* w, float* sc, float
         for (int e = 0; e < 4; ++e) {
             const int c = 4 * q + e, j = 16 * h + c;
             dd[c] -= vi * tw[e] + wi * vj[c];
-            float* dst = (rowok && j < len && j <= i) ? w + (rb - r0 - j) : sink;
+            float* dst = (rowok && j <= i) ? wr + (i - j) : sink;
             *dst = dd[c];
         }
     }
@@ -844,6 +891,12 @@ __global__ void __launch_bounds__(kSbNT) sb2st_kernel(int n, float* __restrict__
         float pv[16], ptau = 0.f;
 #pragma unroll
         for (int c = 0; c < 16; ++c) pv[c] = 0.f;
+        int dofs[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int i = lane & 31, j = 16 * (lane >> 5) + c;
+            dofs[c] = max(i, j) * kSbWP + abs(i - j);
+        }
         SbStream my(n);
         int64_t q2o = 0;  // first Q2 block of this wave's sweep
         for (int t = 0; t < nstep; ++t) {
@@ -858,7 +911,13 @@ __global__ void __launch_bounds__(kSbNT) sb2st_kernel(int n, float* __restrict__
             }
             const bool act = s < nsweep && k >= 0 && k < sb_tasks(n, s);
             float q2val = 0.f;
-            if (act) sb_task(n, s, k, 32 * my.st - kSbG * my.g, win, sc, pv, ptau, q2val, lane);
+            if (act) {
+                const int off = 32 * my.st - kSbG * my.g;
+                if (s + 1 + (k + 1) * NB <= n)
+                    sb_task<true>(n, s, k, off, win, sc, dofs, pv, ptau, q2val, lane);
+                else
+                    sb_task<false>(n, s, k, off, win, sc, dofs, pv, ptau, q2val, lane);
+            }
             __syncthreads();
             // the rows read ahead are written before this step's stores are
             // issued, so waiting for the read waits only for memory operations
