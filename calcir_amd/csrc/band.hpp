@@ -33,8 +33,8 @@ constexpr int kQ2BlockFloats = 2 * kQ2R * kQ2G + kQ2G;
 
 // Stage 1 for a batch: A (n x n, ld, lower triangle used) -> band rows BND
 // (n x kBandW each), reflectors in A and tau (n each).  Work arrays per
-// matrix: P n x 2NB, Yh n x NB, Mm NB x NB.
-int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, float* Yh, float* Mm, hipStream_t s);
+// matrix: P n x 2NB, Yh n x NB.
+int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, float* Yh, hipStream_t s);
 // Stage 2: band rows -> d, e (n each; e[n-1] = 0) and the bulge-chasing
 // reflectors by blocks Q2 (q2_blocks(n) * kQ2BlockFloats).
 int sb2st(int batch, int n, float* BND, float* d, float* e, float* Q2, hipStream_t s);

@@ -8,7 +8,7 @@
 //     registers (one workgroup per matrix); the trailing matrix then gets the
 //     two-sided update A22 <- Q^T A22 Q on its lower triangle, batched over
 //     every matrix: X = A22 Yh with Yh = Y T (sb_symm_kernel), W = X -
-//     Y (Yh^T X)/2 (two small products), A22 -= W Y^T + Y W^T
+//     Y (Yh^T X)/2 (sb_w_kernel), A22 -= W Y^T + Y W^T
 //     (sb_syr2k_kernel), on 32x32x2 FP32 MFMA.
 //   Stage 2, band -> tridiagonal (sb2st_kernel): bulge chasing, one workgroup
 //     per matrix, sweeps in groups of kSbG run by the group's waves in
@@ -31,7 +31,6 @@
 #include <cfloat>
 
 #include "band.hpp"
-#include "gemm.hpp"
 #include "split_bf16.hpp"
 #include "tuner.hpp"
 
@@ -86,23 +85,63 @@ __device__ __forceinline__ void wave_colsums32(const float (&x)[32], int lane, f
     if (i < 8) out[8 * (lane >> 4) + i] = v;
 }
 
+// Householder scalars for a vector with first element alpha and tail square sum
+// sigma > 0: beta = -sign(alpha) |x|, tau = (beta - alpha) / beta, scale = 1 /
+// (alpha - beta).  |x| from the hardware's reciprocal root y with one
+// Newton step each way (the residual of |x|^2, of tau beta and of scale
+// (alpha - beta), each by one FMA, so each result is within an ulp); the IEEE
+// root and quotients are three chains of a dozen dependent instructions on a
+// task's critical path.  Squares too small for the hardware root take those.
+__device__ __forceinline__ void sb_householder(float alpha, float sigma, float& beta, float& tau, float& scale) {
+    const float a2 = alpha * alpha + sigma;
+    if (!(a2 >= 1e-30f && a2 <= 1e30f)) {
+        const float nrm = sqrtf(a2);
+        beta = alpha >= 0.f ? -nrm : nrm;
+        tau = (beta - alpha) / beta;
+        scale = 1.f / (alpha - beta);
+        return;
+    }
+    const float y = __builtin_amdgcn_rsqf(a2);
+    float nrm = a2 * y;
+    nrm = fmaf(fmaf(-nrm, nrm, a2), 0.5f * y, nrm);
+    beta = alpha >= 0.f ? -nrm : nrm;
+    const float yb = alpha >= 0.f ? -y : y;  // about 1 / beta
+    const float den = alpha - beta;
+    tau = -den * yb;
+    tau = fmaf(fmaf(-tau, beta, -den), yb, tau);
+    const float r = __builtin_amdgcn_rcpf(den);
+    scale = fmaf(fmaf(-den, r, 1.f), r, r);
+}
+
 // Householder QR of one panel below the band and everything the trailing
 // update needs.  Panel rows r0..n-1 (m = n - r0 of them) are spread over the
 // threads, rows tid + 512 i (i < RPT) per thread, all NB columns in
-// registers.  Per column c: one block sum for the norm, one for the 32
-// products v^T P(:, c') (the trailing columns' w and, for c' < c, the Gram
-// column Y^T v of the T factor).  Outputs: the diagonal block and R into BND,
-// tau, Y into A (back-transform layout) and into the Y half of the row-major
-// panel P (absolute rows, pitch 2 NB), Yh = Y T row-major (panel rows,
-// pitch NB).
+// registers.  One block sum per column c: the 32 products of its part below
+// row c, x, with every column (x itself among them, so the norm); with row c,
+// which its thread publishes, v^T P(:, c') = scale x^T P(:, c') + P(c, c') for
+// v = (1, scale x): the trailing columns' w and, for c' < c, the Gram column
+// Y^T v of the T factor.  One barrier per column: every wave adds up the
+// waves' partial sums itself, lane q the total of column q, and takes the
+// updates' factors from its lanes.  Columns are worked on in blocks of 8,
+// rotated to the front of the registers, so that register indices are
+// constants in a loop body of 8 columns.  Bound by the chain of a column
+// (sums, scalars, update); a norm sum, the products and the totals as three
+// sums with three barriers, and selects over all 32 columns, took 145 .. 190
+// us per panel for up to a matrix per CU; this takes 47 .. 71 us (RPT 1 .. 4,
+// one matrix; 256 matrices of RPT = 4 move 270 MB and take 155 us).  Outputs: the diagonal block and R
+// into BND, tau, Y into A (back-transform layout) and into the Y half of the
+// row-major panel P (absolute rows, pitch 2 NB), Yh = Y T row-major (panel
+// rows, pitch NB).
 template <int RPT>
 __global__ void __launch_bounds__(kPanNT) sb_panel_kernel(int n, int ld, int j0, float* __restrict__ Aall,
                                                           float* __restrict__ BNDall, float* __restrict__ tauall,
                                                           float* __restrict__ Pall, float* __restrict__ Yhall) {
-    constexpr int NB = kBandNB;
-    __shared__ float redA[kPanNW], redC[kPanNW][NB], dotv[NB], taus[NB], salpha;
-    __shared__ float gram[NB][NB + 1], Tm[NB][NB + 1];
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NB = kBandNB, CB = 8;
+    static_assert(NB == 32, "the column sums and the rotation are written for 32 columns");
+    __shared__ float redC[2][kPanNW][NB], taus[NB];
+    __shared__ __align__(16) float rowc[2][NB], gram[NB][NB + 4], Tc[NB][NB + 4];
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float* A = Aall + size_t(b) * n * ld;
     float* BND = BNDall + size_t(b) * n * kBandW;
     float* P = Pall + size_t(b) * n * 2 * NB;
@@ -122,94 +161,95 @@ __global__ void __launch_bounds__(kPanNT) sb_panel_kernel(int n, int ld, int j0,
         for (int c = 0; c < NB; ++c) p[i][c] = (row < m) ? A[size_t(j0 + c) * ld + r0 + row] : 0.f;
     }
 
+    // register column q holds column (q + CB blk) mod NB
 #pragma unroll 1
-    for (int c = 0; c < NB; ++c) {
-        // norm of the column below row c, and its head
-        float s = 0.f;
+    for (int blk = 0; blk < NB / CB; ++blk) {
 #pragma unroll
-        for (int i = 0; i < RPT; ++i) {
-            const int row = tid + kPanNT * i;
-            float x = 0.f;
+        for (int cc = 0; cc < CB; ++cc) {
+            const int c = CB * blk + cc, buf = cc & 1;
+            float dots[NB];
 #pragma unroll
-            for (int q = 0; q < NB; ++q) x = (q == c) ? p[i][q] : x;
-            if (row > c) s += x * x;
-        }
-        s = bwave_sum(s);
-        if (lane == 0) redA[wave] = s;
-        if (tid == c) {
-            float x = 0.f;
+            for (int q = 0; q < NB; ++q) dots[q] = 0.f;
 #pragma unroll
-            for (int q = 0; q < NB; ++q) x = (q == c) ? p[0][q] : x;
-            salpha = x;
-        }
-        __syncthreads();
-        float sigma = 0.f;
+            for (int i = 0; i < RPT; ++i) {
+                const float x = (tid + kPanNT * i > c) ? p[i][cc] : 0.f;
 #pragma unroll
-        for (int w = 0; w < kPanNW; ++w) sigma += redA[w];
-        const float alpha = salpha;
-        float tau = 0.f, beta = alpha, scale = 0.f;
-        if (sigma > 0.f) {
-            const float nrm = sqrtf(alpha * alpha + sigma);
-            beta = alpha >= 0.f ? -nrm : nrm;
-            tau = (beta - alpha) / beta;
-            scale = 1.f / (alpha - beta);
-        }
-        // v below the unit; row c keeps beta (the R diagonal) and counts as 1
-        float v[RPT];
+                for (int q = 0; q < NB; ++q) dots[q] += x * p[i][q];
+            }
+            wave_colsums32(dots, lane, redC[buf][wave]);
+            if (tid == c) {
 #pragma unroll
-        for (int i = 0; i < RPT; ++i) {
-            const int row = tid + kPanNT * i;
+                for (int q = 0; q < NB; q += 4)
+                    *reinterpret_cast<float4*>(&rowc[buf][q]) = float4{p[0][q], p[0][q + 1], p[0][q + 2], p[0][q + 3]};
+            }
+            __syncthreads();
+            const int q = lane & 31;
+            float tot = 0.f;
 #pragma unroll
-            for (int q = 0; q < NB; ++q)
-                if (q == c) {
-                    if (row > c) p[i][q] *= scale;
-                    if (row == c) p[i][q] = beta;
-                    v[i] = (row > c) ? p[i][q] : (row == c ? 1.f : 0.f);
+            for (int w = 0; w < kPanNW; ++w) tot += redC[buf][w][q];
+            const float pcq = rowc[buf][q];
+            const float sigma = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tot), cc));
+            const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pcq), cc));
+            float tau = 0.f, beta = alpha, scale = 0.f;
+            if (sigma > 0.f) sb_householder(alpha, sigma, beta, tau, scale);
+            tot = scale * tot + pcq;  // v^T P(:, column of register q)
+            if (wave == 0) {
+                const int qc = (q + CB * blk) & (NB - 1);
+                if (lane < NB && qc < c) gram[c][qc] = tot;
+                if (lane == 0) taus[c] = tau;
+            }
+            const float f = tau * tot;
+            float v[RPT];
+#pragma unroll
+            for (int i = 0; i < RPT; ++i) {
+                const int row = tid + kPanNT * i;
+                const float y = p[i][cc] * scale;
+                v[i] = (row > c) ? y : (row == c ? 1.f : 0.f);
+                p[i][cc] = (row > c) ? y : (row == c ? beta : p[i][cc]);
+            }
+            // trailing panel columns: P(:, c') -= tau v (v^T P(:, c'))
+            auto update = [&](int q0, int q1) {
+#pragma unroll
+                for (int u = q0; u < q1; ++u) {
+                    const float fu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), u));
+#pragma unroll
+                    for (int i = 0; i < RPT; ++i) p[i][u] -= fu * v[i];
                 }
+            };
+            update(cc + 1, CB);
+            if (blk < 3) update(CB, 2 * CB);
+            if (blk < 2) update(2 * CB, 3 * CB);
+            if (blk < 1) update(3 * CB, 4 * CB);
         }
-        // v^T P(:, c') over rows >= c, every c'
-        float dots[NB];
 #pragma unroll
-        for (int q = 0; q < NB; ++q) dots[q] = 0.f;
+        for (int i = 0; i < RPT; ++i) {
+            float t[CB];
 #pragma unroll
-        for (int i = 0; i < RPT; ++i)
+            for (int q = 0; q < CB; ++q) t[q] = p[i][q];
 #pragma unroll
-            for (int q = 0; q < NB; ++q) dots[q] += v[i] * p[i][q];
-        wave_colsums32(dots, lane, redC[wave]);
-        __syncthreads();
-        if (tid < NB) {
-            float t = 0.f;
+            for (int q = 0; q < NB - CB; ++q) p[i][q] = p[i][q + CB];
 #pragma unroll
-            for (int w = 0; w < kPanNW; ++w) t += redC[w][tid];
-            dotv[tid] = t;
-            if (tid < c) gram[tid][c] = t;  // (Y^T v_c) of the earlier reflectors
-            if (tid == c) taus[c] = tau;
-        }
-        __syncthreads();
-        // trailing panel columns: P(:, c') -= tau v (v^T P(:, c'))
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            if (q <= c) continue;
-            const float f = tau * dotv[q];
-#pragma unroll
-            for (int i = 0; i < RPT; ++i) p[i][q] -= f * v[i];
+            for (int q = 0; q < CB; ++q) p[i][NB - CB + q] = t[q];
         }
     }
 
-    // T factor (forward, columnwise): T(c, c) = tau_c, T(0:c, c) = -tau_c T(0:c, 0:c) Y^T v_c
-    for (int c = 0; c < NB; ++c) {
-        if (tid < NB) {
-            const int t = tid;
+    // T factor (forward, columnwise): T(c, c) = tau_c, T(0:c, c) = -tau_c
+    // T(0:c, 0:c) Y^T v_c; wave 0, lane t the row t of T in registers
+    if (wave == 0) {
+        wave_lds_sync();
+        const int t = lane;
+        float Tr[NB];
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
             float acc = 0.f;
-            if (t < c)
-                for (int q = t; q < c; ++q) acc += Tm[t][q] * gram[q][c];
-            if (t < c) Tm[t][c] = -taus[c] * acc;
-            if (t == c) Tm[c][c] = taus[c];
-            if (t > c) Tm[t][c] = 0.f;
+#pragma unroll
+            for (int q = 0; q < c; ++q) acc += Tr[q] * gram[c][q];
+            const float tc = taus[c];
+            Tr[c] = (t == c) ? tc : (t < c ? -tc * acc : 0.f);
+            if (t < NB) Tc[c][t] = Tr[c];
         }
-        __syncthreads();
+        if (t < NB) tauall[size_t(b) * n + j0 + t] = taus[t];
     }
-    if (tid < NB) tauall[size_t(b) * n + j0 + tid] = taus[tid];
     // R (upper triangle of rows r0..r0+NB-1) into the band rows
     if (tid < NB && tid < m) {
 #pragma unroll
@@ -221,30 +261,44 @@ __global__ void __launch_bounds__(kPanNT) sb_panel_kernel(int n, int ld, int j0,
     // the band part of these columns is in BND now)
     for (int c = 0; c < NB; ++c)
         for (int r = tid; r < r0 + c && r < n; r += kPanNT) A[size_t(j0 + c) * ld + r] = 0.f;
-    // Y into A, P1, P2 and Yh = Y T
+    // Y into A and P
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
         const int row = tid + kPanNT * i;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) p[i][c] = (row < c) ? 0.f : (row == c ? 1.f : p[i][c]);
         if (row >= m) continue;
-        float y[NB];
 #pragma unroll
-        for (int c = 0; c < NB; ++c) y[c] = (row < c) ? 0.f : (row == c ? 1.f : p[i][c]);
-#pragma unroll
-        for (int c = 0; c < NB; ++c) A[size_t(j0 + c) * ld + r0 + row] = y[c];
+        for (int c = 0; c < NB; ++c) A[size_t(j0 + c) * ld + r0 + row] = p[i][c];
         float4* pr = reinterpret_cast<float4*>(P + size_t(r0 + row) * 2 * NB);
-        float4* yr = reinterpret_cast<float4*>(Yh + size_t(row) * NB);
 #pragma unroll
-        for (int q = 0; q < NB / 4; ++q) pr[q] = float4{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
-        float yh[NB];
+        for (int q = 0; q < NB / 4; ++q)
+            pr[q] = float4{p[i][4 * q], p[i][4 * q + 1], p[i][4 * q + 2], p[i][4 * q + 3]};
+    }
+    __syncthreads();
+    // Yh = Y T, four columns at a time
 #pragma unroll
-        for (int c = 0; c < NB; ++c) {
-            float acc = 0.f;
+    for (int c0 = 0; c0 < NB; c0 += 4) {
+        float acc[RPT][4];
 #pragma unroll
-            for (int q = 0; q <= c; ++q) acc += y[q] * Tm[q][c];
-            yh[c] = acc;
+        for (int i = 0; i < RPT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][e] = 0.f;
+#pragma unroll
+        for (int q = 0; q < c0 + 4; q += 4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float4 t = *reinterpret_cast<const float4*>(&Tc[c0 + e][q]);  // T(q .. q + 3, c0 + e)
+#pragma unroll
+                for (int i = 0; i < RPT; ++i)
+                    acc[i][e] += p[i][q] * t.x + p[i][q + 1] * t.y + p[i][q + 2] * t.z + p[i][q + 3] * t.w;
+            }
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const int row = tid + kPanNT * i;
+            if (row < m)
+                *reinterpret_cast<float4*>(Yh + size_t(row) * NB + c0) = float4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
         }
-#pragma unroll
-        for (int q = 0; q < NB / 4; ++q) yr[q] = float4{yh[4 * q], yh[4 * q + 1], yh[4 * q + 2], yh[4 * q + 3]};
     }
 }
 
@@ -358,6 +412,89 @@ __global__ void __launch_bounds__(256) sb_symm_kernel(int n, int ld, int r0, con
     }
 }
 
+// W = X - Y (Yh^T X) / 2 in place of X, one workgroup per matrix: the 32 x 32
+// product M = Yh^T X with the rows split over the waves in blocks of 32 (its
+// partial sums added in wave order), then each wave's blocks of W, formed
+// transposed (MFMA row = column of W) so that a lane holds 4 consecutive
+// columns of its row.  32x32x2 FP32 MFMA; lane half h takes positions 16 h + q
+// of a K = 32 sum.  As two launches of the general product, one workgroup of
+// 64 x 64 tiles each for the first: 54 us for one matrix of N = 2048; this
+// takes 22 us.
+__global__ void __launch_bounds__(kPanNT) sb_w_kernel(int n, int r0, const float* __restrict__ Yhall,
+                                                      float* __restrict__ Pall) {
+    constexpr int NB = kBandNB;
+    __shared__ float red[kPanNW][NB][NB + 1];
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = n - r0, nblk = (m + 31) / 32;
+    const float* Yh = Yhall + size_t(b) * n * NB;
+    float* P = Pall + size_t(b) * n * 2 * NB + size_t(r0) * 2 * NB;
+    floatx16 acc;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
+    float a0[16], x0[16];
+    auto load = [&](int blk) {  // rows past m: clamped, Yh zeroed below
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int r = min(blk * 32 + 2 * q + h, m - 1);
+            a0[q] = Yh[size_t(r) * NB + l32];
+            x0[q] = P[size_t(r) * 2 * NB + NB + l32];
+        }
+    };
+    if (wave < nblk) load(wave);
+    for (int blk = wave; blk < nblk; blk += kPanNW) {
+        float a[16], x[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            a[q] = (blk * 32 + 2 * q + h < m) ? a0[q] : 0.f;
+            x[q] = x0[q];
+        }
+        if (blk + kPanNW < nblk) load(blk + kPanNW);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], x[q], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) red[wave][8 * (q >> 2) + 4 * h + (q & 3)][l32] = acc[q];
+    __syncthreads();
+    for (int e = tid; e < NB * NB; e += kPanNT) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < kPanNW; ++w) t += red[w][e / NB][e % NB];
+        red[0][e / NB][e % NB] = -0.5f * t;  // (an element is read and written by one thread)
+    }
+    __syncthreads();
+    float mk[16];  // -M(16 h + q, l32) / 2
+#pragma unroll
+    for (int q = 0; q < 16; ++q) mk[q] = red[0][16 * h + q][l32];
+    for (int blk = wave; blk < nblk; blk += kPanNW) {
+        const int r = blk * 32 + l32;
+        float* row = P + size_t(min(r, m - 1)) * 2 * NB;
+        float y[16];
+        floatx16 d;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 t = *reinterpret_cast<const float4*>(row + 16 * h + 4 * q);
+            y[4 * q] = t.x;
+            y[4 * q + 1] = t.y;
+            y[4 * q + 2] = t.z;
+            y[4 * q + 3] = t.w;
+            const float4 u = *reinterpret_cast<const float4*>(row + NB + 8 * q + 4 * h);
+            d[4 * q] = u.x;
+            d[4 * q + 1] = u.y;
+            d[4 * q + 2] = u.z;
+            d[4 * q + 3] = u.w;
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) d = __builtin_amdgcn_mfma_f32_32x32x2f32(mk[q], y[q], d, 0, 0, 0);
+        if (r < m) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<float4*>(row + NB + 8 * q + 4 * h) =
+                    float4{d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]};
+        }
+    }
+}
+
 // Word 3 of a raw buffer resource on gfx9-family GPUs (32-bit data format,
 // no swizzle, range checking on offsets).
 constexpr int kBufferWord3 = 0x00020000;
@@ -466,7 +603,7 @@ __global__ void __launch_bounds__(256) sb_band_tail_kernel(int n, int ld, int jl
     }
 }
 
-int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, float* Yh, float* Mm, hipStream_t s) {
+int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, float* Yh, hipStream_t s) {
     constexpr int NB = kBandNB;
     if (n > sb_max_n()) return fail(CIR_ERR_ARG, "sy2sb: n too large for the register panel");
     {
@@ -496,47 +633,9 @@ int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, 
         // X = A22 Yh into the W half of P
         hipLaunchKernelGGL(sb_symm_kernel, grid, dim3(256), 0, s, n, ld, r0, A, Yh, P, batch);
         CIR_CHECK_LAUNCH();
-        const int64_t ps = int64_t(n) * 2 * NB;
-        GemmArgs g;
-        // Mm = Yh^T X (NB x NB)
-        g.batch = batch;
-        g.M = NB;
-        g.N = NB;
-        g.K = m;
-        g.A = Yh;
-        g.a_m = 1;
-        g.a_k = NB;
-        g.a_b = int64_t(n) * NB;
-        g.B = P + size_t(r0) * 2 * NB + NB;
-        g.b_k = 2 * NB;
-        g.b_n = 1;
-        g.b_b = ps;
-        g.C = Mm;
-        g.c_m = NB;
-        g.c_n = 1;
-        g.c_b = int64_t(NB) * NB;
-        CIR_TRY(gemm(CIR_PREC_FP32, g, s));
-        // W = X - Y Mm / 2 in place of X
-        g = GemmArgs{};
-        g.batch = batch;
-        g.M = m;
-        g.N = NB;
-        g.K = NB;
-        g.A = P + size_t(r0) * 2 * NB;
-        g.a_m = 2 * NB;
-        g.a_k = 1;
-        g.a_b = ps;
-        g.B = Mm;
-        g.b_k = NB;
-        g.b_n = 1;
-        g.b_b = int64_t(NB) * NB;
-        g.C = P + size_t(r0) * 2 * NB + NB;
-        g.c_m = 2 * NB;
-        g.c_n = 1;
-        g.c_b = ps;
-        g.alpha = -0.5;
-        g.beta = 1.0;
-        CIR_TRY(gemm(CIR_PREC_FP32, g, s));
+        // W = X - Y (Yh^T X) / 2 in place of X
+        hipLaunchKernelGGL(sb_w_kernel, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, r0, Yh, P);
+        CIR_CHECK_LAUNCH();
         // A22 -= W Y^T + Y W^T (lower triangle)
         hipLaunchKernelGGL(sb_syr2k_kernel, grid, dim3(256), 0, s, n, ld, r0, A, P, batch);
         CIR_CHECK_LAUNCH();
@@ -605,34 +704,6 @@ __device__ __forceinline__ float half_pair_sum(float x) {
 // The value of lane i (i < 32) in lanes i and i + 32.
 __device__ __forceinline__ float from_low_half(float x) {
     return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false)[0]);
-}
-
-// Householder scalars for a vector with first element alpha and tail square sum
-// sigma > 0: beta = -sign(alpha) |x|, tau = (beta - alpha) / beta, scale = 1 /
-// (alpha - beta).  |x| from the hardware's reciprocal root y with one
-// Newton step each way (the residual of |x|^2, of tau beta and of scale
-// (alpha - beta), each by one FMA, so each result is within an ulp); the IEEE
-// root and quotients are three chains of a dozen dependent instructions on a
-// task's critical path.  Squares too small for the hardware root take those.
-__device__ __forceinline__ void sb_householder(float alpha, float sigma, float& beta, float& tau, float& scale) {
-    const float a2 = alpha * alpha + sigma;
-    if (!(a2 >= 1e-30f && a2 <= 1e30f)) {
-        const float nrm = sqrtf(a2);
-        beta = alpha >= 0.f ? -nrm : nrm;
-        tau = (beta - alpha) / beta;
-        scale = 1.f / (alpha - beta);
-        return;
-    }
-    const float y = __builtin_amdgcn_rsqf(a2);
-    float nrm = a2 * y;
-    nrm = fmaf(fmaf(-nrm, nrm, a2), 0.5f * y, nrm);
-    beta = alpha >= 0.f ? -nrm : nrm;
-    const float yb = alpha >= 0.f ? -y : y;  // about 1 / beta
-    const float den = alpha - beta;
-    tau = -den * yb;
-    tau = fmaf(fmaf(-tau, beta, -den), yb, tau);
-    const float r = __builtin_amdgcn_rcpf(den);
-    scale = fmaf(fmaf(-den, r, 1.f), r, r);
 }
 
 // Sum over the 32 lanes of each half wave, in every lane of the half.

@@ -1851,7 +1851,7 @@ copy4_kernel(int64_t cnt, const float4* __restrict__ src, float4* __restrict__ d
 
 struct EighWork {
     size_t off_d, off_e, off_tau, off_vw, off_g, off_t, off_w1, off_w2, off_s1, off_scr, total;
-    size_t off_bnd, off_p1, off_p2, off_yh, off_mm, off_q2, off_h, off_r;  // two-stage buffers
+    size_t off_bnd, off_p1, off_yh, off_q2, off_h, off_r;  // two-stage buffers
     bool two, refine;
     int sub;  // matrices per inverse-iteration pass
 };
@@ -1866,12 +1866,8 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
         o = al(o + esz * batch * size_t(n) * kBandW);
         L.off_p1 = o;
         o = al(o + esz * batch * size_t(n) * 2 * kBandNB);
-        L.off_p2 = o;
-        o = al(o + esz * batch * size_t(n) * 2 * kBandNB);
         L.off_yh = o;
         o = al(o + esz * batch * size_t(n) * kBandNB);
-        L.off_mm = o;
-        o = al(o + esz * batch * size_t(kBandNB) * kBandNB);
         L.off_q2 = o;
         o = al(o + esz * batch * size_t(q2_blocks(n)) * kQ2BlockFloats);
         L.refine = use_refine(batch, n);
@@ -1940,8 +1936,7 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
                     CIR_CHECK_LAUNCH();
                 }
                 CIR_TRY(sy2sb(batch, n, ld, A, bnd, tau, reinterpret_cast<float*>(work + L.off_p1),
-                              reinterpret_cast<float*>(work + L.off_yh), reinterpret_cast<float*>(work + L.off_mm),
-                              s));
+                              reinterpret_cast<float*>(work + L.off_yh), s));
             }
             ProfScope ps(prof, CIR_PH_BULGE, s);
             CIR_TRY(sb2st(batch, n, bnd, dd, ee, q2, s));
