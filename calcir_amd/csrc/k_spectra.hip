@@ -310,7 +310,7 @@ slot_fixup_kernel(int n, int nslot, int ldy, const int* __restrict__ action, con
 //   p = 9..14 iiFjj: (4,3) (5,3) (3,4) (5,4) (3,5) (4,5).
 // One row's terms of the 15 forms (Re, Im) into acc.
 template <typename T>
-__device__ __forceinline__ void corr_row(const T (&m)[9], const T (&yr)[9], const T (&yi)[9], double (&acc)[30]) {
+__device__ __forceinline__ void corr_row(const T (&m)[9], const T (&yr)[9], const T (&yi)[9], double (&acc)[32]) {
 #pragma unroll
     for (int p = 0; p < 15; ++p) {
         const int pb = (p < 9) ? p : ((p == 9 || p == 14) ? 4 : (p == 10 || p == 12) ? 5 : 3);
@@ -320,117 +320,148 @@ __device__ __forceinline__ void corr_row(const T (&m)[9], const T (&yr)[9], cons
     }
 }
 
-// The block's sums of acc, combined into IR, VV and VH (calcIR.cu:646-648,
-// 736-745) and stored at o[0..5].
-template <int NT>
-__device__ __forceinline__ void corr_finish(double (&acc)[30], double (*red)[30], double* o) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// Sums over the 64 lanes of 32 values x[k], stored at out[k] (LDS).  Two lane
+// swaps halve the values per lane (after them lane l holds the partials of
+// values k + 8 (l >> 4), k < 8), rotations in rows of 16 lanes finish them,
+// and lane 16 R + i (i < 8) stores value 8 R + i.
+__device__ __forceinline__ double lane_swap32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double lane_swap16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+template <int ROR>
+__device__ __forceinline__ double add_row_ror(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x120 + ROR, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x120 + ROR, 0xf, 0xf, false);
+    return x + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ void wave_sums32(const double (&x)[32], int lane, double* out) {
+    double y[16], z[8];
 #pragma unroll
-    for (int p = 0; p < 30; ++p) {
-        const double v = wave_sum(acc[p]);
-        if (lane == 0) red[wave][p] = v;
+    for (int k = 0; k < 16; ++k) y[k] = lane_swap32(x[k], x[k + 16]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        z[k] = lane_swap16(y[k], y[k + 8]);
+        z[k] = add_row_ror<8>(z[k]);
+        z[k] = add_row_ror<4>(z[k]);
+        z[k] = add_row_ror<2>(z[k]);
+        z[k] = add_row_ror<1>(z[k]);
     }
-    __syncthreads();
-    if (tid == 0) {
-        double t[30];
-        for (int p = 0; p < 30; ++p) {
-            t[p] = 0.0;
-            for (int w = 0; w < NT / 64; ++w) t[p] += red[w][p];
-        }
-        double ir[2] = {0, 0}, iiii[2] = {0, 0}, ijij[2] = {0, 0}, iijj[2] = {0, 0};
-        for (int c = 0; c < 2; ++c) {
-            for (int p = 0; p < 3; ++p) ir[c] += t[2 * p + c];
-            for (int p = 3; p < 6; ++p) iiii[c] += t[2 * p + c];
-            for (int p = 6; p < 9; ++p) ijij[c] += t[2 * p + c];
-            for (int p = 9; p < 15; ++p) iijj[c] += t[2 * p + c];
-        }
-        for (int c = 0; c < 2; ++c) {
-            o[c] = ir[c];
-            o[2 + c] = (3.0 * iiii[c] + iijj[c] + 4.0 * ijij[c]) / 15.0;
-            o[4 + c] = (2.0 * iiii[c] - iijj[c] + 6.0 * ijij[c]) / 30.0;
-        }
-    }
+    const int i = lane & 15;
+    double v = z[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) v = (i == k) ? z[k] : v;
+    if (i < 8) out[8 * (lane >> 4) + i] = v;
 }
 
-// One block per slot: the 15 bilinear forms, stored at out[6*target[s] ...].
-template <typename T>
-__global__ void __launch_bounds__(kSpNT)
+// The 15 bilinear forms of one slot per block, combined into IR, VV and VH
+// (calcIR.cu:646-648, 736-745) at out[6 target ..].  FIX: each of the slot's
+// columns is first set as its action says (idle: zero, origin: M(t), hold: the
+// old state; propagated: left as the propagation wrote them).
+//
+// Bound by the loads of the slot's 9 + 9 columns out of rows of ldy: a wave
+// takes 64 rows at a time and reads them with consecutive lanes on consecutive
+// columns (7 rows' lines per load; a lane per row touched 64 lines per load,
+// 15 us of line lookups on the slot's one CU at N = 2048), then turns them
+// through LDS, 9 words a row (odd, so without bank conflicts).  The 30 sums
+// are folded by lane swaps, 56 additions a wave instead of 30 x 6 shuffles.
+// With one lane adding up the waves: 21 us at N = 2048 and 8 slots, 12 us at
+// N = 256.
+template <typename T, int NT, bool FIX>
+__global__ void __launch_bounds__(NT)
 correlate_kernel(int n, int nslot, int ldy, const int* __restrict__ action, const int* __restrict__ target,
-                 const T* __restrict__ sites, const T* __restrict__ Y, double* __restrict__ out) {
-    __shared__ double red[kSpNT / 64][30];
-    const int s = blockIdx.x, tid = threadIdx.x;
+                 const T* __restrict__ sites, const T* __restrict__ Yold, T* __restrict__ Y, double* __restrict__ out) {
+    constexpr int NW = NT / 64;
+    __shared__ T turn[NW][64 * 9];
+    __shared__ double red[NW][32], tot[32];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int act = action ? action[s] : 2;
-    if (act != 1 && act != 2) return;
+    if (!FIX && act != 1 && act != 2) return;
     const int ncols = 9 * nslot;
-    double acc[30];
+    T* Ys = Y + 9 * s;
+    const T* mu = sites + size_t(CIR_SITE_MU) * n;
+    double acc[32];
 #pragma unroll
-    for (int p = 0; p < 30; ++p) acc[p] = 0.0;
-    for (int i = tid; i < n; i += kSpNT) {
-        const T* yr = Y + size_t(i) * ldy + 9 * s;
-        const T* yi = yr + ncols;
-        T m[9], vr[9], vi[9];
-#pragma unroll
-        for (int b = 0; b < 9; ++b) {
-            m[b] = sites[size_t(CIR_SITE_MU + b) * n + i];
-            vr[b] = yr[b];
-            vi[b] = yi[b];
-        }
-        corr_row(m, vr, vi, acc);
-    }
-    corr_finish<kSpNT>(acc, red, out + 6 * size_t(target ? target[s] : 0));
-}
-
-// slot_fixup_kernel and correlate_kernel in one launch, one block per slot:
-// each row's nine columns of the slot are set as the action says (idle: zero,
-// origin: M(t), hold: the old state; propagated: left as the propagation wrote
-// them) and, for an origin or a propagated slot, the forms summed from the
-// same values in the same order as correlate_kernel sums them.
-template <typename T>
-__global__ void __launch_bounds__(kSpNT)
-slot_correlate_kernel(int n, int nslot, int ldy, const int* __restrict__ action, const int* __restrict__ target,
-                      const T* __restrict__ sites, const T* __restrict__ Yold, T* __restrict__ Ynew,
-                      double* __restrict__ out) {
-    __shared__ double red[kSpNT / 64][30];
-    const int s = blockIdx.x, tid = threadIdx.x;
-    const int act = action[s];
-    const int ncols = 9 * nslot;
-    double acc[30];
-#pragma unroll
-    for (int p = 0; p < 30; ++p) acc[p] = 0.0;
-    for (int i = tid; i < n; i += kSpNT) {
-        T* yr = Ynew + size_t(i) * ldy + 9 * s;
-        T* yi = yr + ncols;
-        if (act == 0 || act == 3) {
-            const T* orr = Yold + size_t(i) * ldy + 9 * s;
-#pragma unroll
-            for (int b = 0; b < 9; ++b) {
-                yr[b] = (act == 3) ? orr[b] : T(0);
-                yi[b] = (act == 3) ? orr[ncols + b] : T(0);
+    for (int p = 0; p < 32; ++p) acc[p] = 0.0;
+    for (int r0 = 64 * wave; r0 < n; r0 += 64 * NW) {
+        const int nr = min(64, n - r0);
+        if (FIX && act != 2) {
+            // the columns' new values, with consecutive lanes on consecutive columns
+            const T* Yo = Yold + 9 * s;
+            for (int e = lane; e < 9 * nr; e += 64) {
+                const int i = r0 + e / 9, c = e % 9;
+                const size_t o = size_t(i) * ldy + c;
+                Ys[o] = (act == 1) ? mu[size_t(c) * n + i] : (act == 3) ? Yo[o] : T(0);
+                Ys[o + ncols] = (act == 3) ? Yo[o + ncols] : T(0);
             }
-            continue;
+            if (act != 1) continue;
         }
-        T m[9], vr[9], vi[9];
+        T m[9], yr[9], yi[9];
 #pragma unroll
-        for (int b = 0; b < 9; ++b) m[b] = sites[size_t(CIR_SITE_MU + b) * n + i];
-        if (act == 1) {
+        for (int b = 0; b < 9; ++b) m[b] = (lane < nr) ? mu[size_t(b) * n + r0 + lane] : T(0);
+        if (FIX && act == 1) {
 #pragma unroll
             for (int b = 0; b < 9; ++b) {
-                vr[b] = m[b];
-                vi[b] = T(0);
-                yr[b] = vr[b];
+                yr[b] = m[b];
                 yi[b] = T(0);
             }
         } else {
+            T fr[9], fi[9];
 #pragma unroll
-            for (int b = 0; b < 9; ++b) {
-                vr[b] = yr[b];
-                vi[b] = yi[b];
+            for (int j = 0; j < 9; ++j) {
+                const int e = lane + 64 * j;
+                const T* y = Ys + size_t(r0 + e / 9) * ldy + e % 9;
+                fr[j] = (e < 9 * nr) ? y[0] : T(0);
+                fi[j] = (e < 9 * nr) ? y[ncols] : T(0);
             }
+#pragma unroll
+            for (int j = 0; j < 9; ++j) turn[wave][lane + 64 * j] = fr[j];
+            wave_lds_sync();
+#pragma unroll
+            for (int b = 0; b < 9; ++b) yr[b] = turn[wave][9 * lane + b];
+            wave_lds_sync();
+#pragma unroll
+            for (int j = 0; j < 9; ++j) turn[wave][lane + 64 * j] = fi[j];
+            wave_lds_sync();
+#pragma unroll
+            for (int b = 0; b < 9; ++b) yi[b] = turn[wave][9 * lane + b];
+            wave_lds_sync();
         }
-        corr_row(m, vr, vi, acc);
+        corr_row(m, yr, yi, acc);
     }
     if (act != 1 && act != 2) return;
-    corr_finish<kSpNT>(acc, red, out + 6 * size_t(target[s]));
+    wave_sums32(acc, lane, red[wave]);
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane < 32) {
+        double t = red[0][lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) t += red[w][lane];
+        tot[lane] = t;
+    }
+    wave_lds_sync();
+    if (lane < 2) {
+        const int c = lane;
+        double ir = 0, iiii = 0, ijij = 0, iijj = 0;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) ir += tot[2 * p + c];
+#pragma unroll
+        for (int p = 3; p < 6; ++p) iiii += tot[2 * p + c];
+#pragma unroll
+        for (int p = 6; p < 9; ++p) ijij += tot[2 * p + c];
+#pragma unroll
+        for (int p = 9; p < 15; ++p) iijj += tot[2 * p + c];
+        double* o = out + 6 * size_t(target ? target[s] : 0);
+        o[c] = ir;
+        o[2 + c] = (3.0 * iiii + iijj + 4.0 * ijij) / 15.0;
+        o[4 + c] = (2.0 * iiii - iijj + 6.0 * ijij) / 30.0;
+    }
 }
 
 // cuFFT C2R contract (calcIR.cu:790-791): y[k] = Re X0 + 2 sum_j Re(X_j
@@ -927,30 +958,35 @@ int slot_fixup(int prec, int n, int nslot, int ldy, const int* action, const voi
     return CIR_OK;
 }
 
-int slot_correlate(int prec, int n, int nslot, int ldy, const int* action, const int* target, const void* sites,
-                   const void* Yold, void* Ynew, double* out, hipStream_t s) {
-    if (prec == CIR_PREC_FP64)
-        hipLaunchKernelGGL(slot_correlate_kernel<double>, dim3(nslot), dim3(kSpNT), 0, s, n, nslot, ldy, action,
-                           target, static_cast<const double*>(sites), static_cast<const double*>(Yold),
-                           static_cast<double*>(Ynew), out);
+// Waves for the rows, 64 a wave: up to 4 for small boxes, where more waves only
+// add to the final sums, else 16 (8 in FP64, twice the registers).
+template <typename T, bool FIX>
+static int correlate_slots(int n, int nslot, int ldy, const int* action, const int* target, const void* sites,
+                           const void* Yold, void* Y, double* out, hipStream_t s) {
+    constexpr int kWide = sizeof(T) == 8 ? 512 : 1024;
+    if (n <= 4 * kSpNT)
+        hipLaunchKernelGGL((correlate_kernel<T, kSpNT, FIX>), dim3(nslot), dim3(kSpNT), 0, s, n, nslot, ldy, action,
+                           target, static_cast<const T*>(sites), static_cast<const T*>(Yold), static_cast<T*>(Y), out);
     else
-        hipLaunchKernelGGL(slot_correlate_kernel<float>, dim3(nslot), dim3(kSpNT), 0, s, n, nslot, ldy, action,
-                           target, static_cast<const float*>(sites), static_cast<const float*>(Yold),
-                           static_cast<float*>(Ynew), out);
+        hipLaunchKernelGGL((correlate_kernel<T, kWide, FIX>), dim3(nslot), dim3(kWide), 0, s, n, nslot, ldy, action,
+                           target, static_cast<const T*>(sites), static_cast<const T*>(Yold), static_cast<T*>(Y), out);
     CIR_CHECK_LAUNCH();
     return CIR_OK;
 }
 
+int slot_correlate(int prec, int n, int nslot, int ldy, const int* action, const int* target, const void* sites,
+                   const void* Yold, void* Ynew, double* out, hipStream_t s) {
+    return prec == CIR_PREC_FP64
+               ? correlate_slots<double, true>(n, nslot, ldy, action, target, sites, Yold, Ynew, out, s)
+               : correlate_slots<float, true>(n, nslot, ldy, action, target, sites, Yold, Ynew, out, s);
+}
+
 int correlate(int prec, int n, int nslot, int ldy, const int* action, const int* target, const void* sites,
               const void* Y, double* out, hipStream_t s) {
-    if (prec == CIR_PREC_FP64)
-        hipLaunchKernelGGL(correlate_kernel<double>, dim3(nslot), dim3(kSpNT), 0, s, n, nslot, ldy, action, target,
-                           static_cast<const double*>(sites), static_cast<const double*>(Y), out);
-    else
-        hipLaunchKernelGGL(correlate_kernel<float>, dim3(nslot), dim3(kSpNT), 0, s, n, nslot, ldy, action, target,
-                           static_cast<const float*>(sites), static_cast<const float*>(Y), out);
-    CIR_CHECK_LAUNCH();
-    return CIR_OK;
+    void* y = const_cast<void*>(Y);  // (only read without FIX)
+    return prec == CIR_PREC_FP64
+               ? correlate_slots<double, false>(n, nslot, ldy, action, target, sites, nullptr, y, out, s)
+               : correlate_slots<float, false>(n, nslot, ldy, action, target, sites, nullptr, y, out, s);
 }
 
 // ---------------------------------------------------------------------------
