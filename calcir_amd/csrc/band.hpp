@@ -11,7 +11,6 @@ constexpr int kBandNB = 32;           // band half-width (panel width of stage 1
 constexpr int kBandW = 2 * kBandNB;   // stored band row: r - c in [0, 2 NB)
 constexpr int kQ2G = 16;              // sweeps per compact-WY block of the bulge-chasing reflectors
 constexpr int kQ2R = 48;              // rows of such a block (NB + kQ2G - 1, padded)
-constexpr int kQ2S = 16;              // eigenvector columns per workgroup in the Q2 back-transform
 
 // Largest n of the stage-1 register panel (4 rows of 512 threads below the band).
 inline int sb_max_n() { return 4 * 512 + kBandNB; }
@@ -22,10 +21,11 @@ __host__ __device__ inline int sb_tasks(int n, int s) { return (s <= n - 3) ? (n
 // reflectors of sweeps g kQ2G .. g kQ2G + kQ2G - 1 at position k; its index is
 // q2_block_offset(n, g) + k, and group g has sb_tasks(n, g kQ2G) blocks.
 __host__ __device__ inline int q2_groups(int n) { return n >= 3 ? (n - 2 + kQ2G - 1) / kQ2G : 0; }
+// (groups alternate between sweeps at multiples of 32 and 16 more, each kind
+// with one task fewer from one to the next)
 __host__ __device__ inline int64_t q2_block_offset(int n, int g) {
-    int64_t o = 0;
-    for (int q = 0; q < g; ++q) o += sb_tasks(n, q * kQ2G);
-    return o;
+    const int64_t ne = (g + 1) / 2, no = g / 2;
+    return g + ne * ((n - 2) / kBandNB) - ne * (ne - 1) / 2 + no * ((n - 2 - kQ2G) / kBandNB) - no * (no - 1) / 2;
 }
 inline int64_t q2_blocks(int n) { return q2_block_offset(n, q2_groups(n)); }
 // floats per block: V (kQ2R x kQ2G, column per reflector), tau (kQ2G), -V T (kQ2R x kQ2G)

@@ -1042,16 +1042,16 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Group and position of block q of a matrix.
 __device__ __forceinline__ void q2_block_gk(int n, int64_t q, int* g, int* k) {
-    int gg = 0;
-    int64_t o = 0;
-    const int ng = q2_groups(n);
-    for (; gg < ng; ++gg) {
-        const int t = sb_tasks(n, gg * kQ2G);
-        if (q < o + t) break;
-        o += t;
+    int lo = 0, hi = q2_groups(n);  // the last group that starts at or before q
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (q2_block_offset(n, mid) <= q)
+            lo = mid;
+        else
+            hi = mid;
     }
-    *g = gg;
-    *k = int(q - o);
+    *g = lo;
+    *k = int(q - q2_block_offset(n, lo));
 }
 
 // Four values as the 16 bytes of their BF16 parts: hi (8 bytes), then lo.
@@ -1123,6 +1123,7 @@ __global__ void __launch_bounds__(64) q2_prep_kernel(int n, int64_t nblk, float*
     // l16, 4 s + lq), split-BF16 products NV(16 rt + l16, 4 lq + s).  The
     // split-BF16 operands are split here, once per block instead of once per
     // block and slab: each 16 bytes hold the hi and lo parts of 4 values.
+    float4 vp[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         float v[4], w[4];
@@ -1131,266 +1132,373 @@ __global__ void __launch_bounds__(64) q2_prep_kernel(int n, int64_t nblk, float*
             v[e] = sv[16 * q + 4 * lq + e][l16];
             w[e] = bf16 ? snv[16 * q + l16][4 * lq + e] : snv[16 * q + l16][4 * e + lq];
         }
-        float4* vo = reinterpret_cast<float4*>(V + lane * 12) + q;
-        float4* wo = reinterpret_cast<float4*>(NVT + lane * 12) + q;
+        float4* vo = reinterpret_cast<float4*>(V) + 64 * q + lane;
+        float4* wo = reinterpret_cast<float4*>(NVT) + 64 * q + lane;
         if (bf16) {
-            *vo = q2_split4(v);
+            vp[q] = q2_split4(v);
             *wo = q2_split4(w);
         } else {
             *vo = float4{v[0], v[1], v[2], v[3]};
             *wo = float4{w[0], w[1], w[2], w[3]};
         }
     }
+    if (bf16) {
+        // V: the hi parts of row tiles 0 and 1, their lo parts, both of tile 2
+        float4* vo = reinterpret_cast<float4*>(V) + lane;
+        vo[0] = float4{vp[0].x, vp[0].y, vp[1].x, vp[1].y};
+        vo[64] = float4{vp[0].z, vp[0].w, vp[1].z, vp[1].w};
+        vo[128] = vp[2];
+    }
     if (lane < kQ2G) tau[lane] = stau[lane];
 }
 
-// Z <- Q2 Z on one 16-column slab of one matrix, the slab in LDS (rows past n
-// zero).  Blocks apply group by group from the last group, positions in
-// ascending order.  Block (g, k) spans rows 16 g + 1 + 32 k .. 16 g + 47 +
-// 32 k, so it must follow (g, k - 1) and, of the group after it, (g + 1, k - 1)
-// and (g + 1, k); group g takes position k at step k + (G - 1 - g), which
-// orders all of these, and the blocks of one step, (g, k), (g + 1, k + 1), ...,
-// start 48 rows apart and touch disjoint rows.  Group g belongs to wave
-// (G - 1 - g) mod (waves per workgroup), which reads its next block's
-// operands while it applies the current one.  A block: W = V^T Zb
-// (16 x 16, K = 48) and Zb += (-V T) W, as 16x16x4 FP32 MFMA, W passed from
-// one product to the next in registers.
-constexpr int kQ2MaxGroups = 160;
-static_assert(kQ2MaxGroups * kQ2G >= 4 * 512 + kBandNB, "group table too small for sb_max_n()");
-// The slab is stored column by column, row r of Z at index r + 3 of its
-// column (block rows then start at multiples of 4, so a lane's 4 rows are one
-// 16-byte access), with a column pitch of 4 mod 64 floats (the 16 columns of
-// one access fall in distinct banks) covering rows n .. n + 47 as zeros.
-__host__ __device__ inline int q2_pitch(int n) {
-    const int p = n + kQ2R + 3;
-    return p + ((4 - p) & 63);
-}
 typedef short short8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ shortx4 q2_half(float a, float b) {
-    return __builtin_bit_cast(shortx4, (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32));
+typedef unsigned long long q2_parts __attribute__((ext_vector_type(2)));
+// Four values split into their BF16 parts: lo's four and hi's four, 8 bytes each.
+__device__ __forceinline__ q2_parts q2_split(floatx4 v) {
+    unsigned h0, l0, h1, l1;
+    split_bf16x2(v[0], v[1], h0, l0);
+    split_bf16x2(v[2], v[3], h1, l1);
+    return q2_parts{l0 | (unsigned long long)(l1) << 32, h0 | (unsigned long long)(h1) << 32};
 }
-__device__ __forceinline__ short8 q2_cat(shortx4 a, shortx4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ short8 q2_lo_hi(q2_parts p) { return __builtin_bit_cast(short8, p); }
+__device__ __forceinline__ short8 q2_hi_lo(q2_parts p) { return __builtin_bit_cast(short8, q2_parts{p[1], p[0]}); }
+__device__ __forceinline__ short8 q2_ops(float4 a) {
+    return __builtin_bit_cast(short8, floatx4{a.x, a.y, a.z, a.w});
+}
 __device__ __forceinline__ floatx4 q2_mfma32(short8 a, short8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-template <int kQ2NT, bool BF>
-__global__ void __launch_bounds__(kQ2NT) q2_apply_kernel(int n, int ld, const float* __restrict__ Q2all,
-                                                          float* __restrict__ Zall, int64_t nblk, int nmat) {
+// Z <- Q2 Z on one slab of 16 CT columns of one matrix.  Blocks apply group by
+// group from the last group g = NG - 1 (gi = NG - 1 - g ascending), positions
+// k in ascending order; block (g, k) covers the row tiles (16 rows each, tile
+// i from row 16 i + 1) g + 2 k .. g + 2 k + 2.
+//
+// The rows stream through the workgroup's waves: wave w takes the groups gi =
+// w, w + NW, ..., holds the three tiles of its block in registers, and after
+// block k passes the first two, which its group does not touch again, on as
+// slot k to the next wave, whose own block k needs just them behind the tile
+// it carries (its group starts one tile earlier; that first tile no earlier
+// group touches, so it comes from Z).  Slots go through short queues in LDS
+// (kQ2Fifo deep); the last wave's go back to Z and the first wave reads them
+// there for the following round of groups.  A group has as many slots as
+// blocks, ceil of its tiles / 2, and its successor at most one more, for which
+// the rows are past the end: zeros.
+//
+// Every wait is for a slot of an earlier group or for the room that a later
+// group's reads leave, the waves take their blocks in the order of (round,
+// k), and a group of the first wave waits for nothing of its own round, so
+// every wait ends (and is bounded all the same: one that ran far past any
+// block's time marks the slab, which is then written as NaN).
+//
+// Bound by the issue of the split's vector instructions (70% of the cycles)
+// beside the MFMAs.  A block's operands, 6 KB, are read per wave straight into
+// registers a block ahead, and serve all of the wave's columns: they pass the
+// CU's vector cache and the L2 once per 16 CT columns.  The whole slab in LDS
+// (16 columns, 128 KB at N = 2048, which also bounded N) moved them for every
+// 16 columns, in three times the lines: 47.7 ms for 256 matrices of N = 2048 in
+// split BF16, 34.7 with CT = 4.
+constexpr int kQ2Fifo = 2;
+constexpr int kQ2Cus = 256;
+
+// One block on CT column tiles of three row tiles each, the column tiles'
+// chains side by side.
+template <int CT, bool BF>
+__device__ __forceinline__ void q2_block(const float4 (&va)[3], const float4 (&na)[3], floatx4 (&z0)[CT],
+                                         floatx4 (&z1)[CT], floatx4 (&z2)[CT]) {
+    if constexpr (BF) {
+        // split BF16 (x = hi + lo), the operands' parts stored by
+        // q2_prep_kernel.  Lane (lq, l16) holds k = 4 lq .. 4 lq + 3 of its
+        // row (A) or column (B), so W = V^T Zb comes out as the update's B
+        // operand, W(4 lq + r, l16) in register r, with no transpose.  Two
+        // 16-deep products share one 16x16x32 MFMA (the same 16 cycles as a
+        // 16x16x16): for W the row tiles 0 and 1 side by side (hi*lo, lo*hi,
+        // hi*hi), elsewhere the operand's (hi, lo) with the columns' (lo, hi)
+        // and then with their (hi, lo), which adds the lo*lo part as well and
+        // needs no zero halves.  (A 16x16x16 and a 16x16x32 one after the
+        // other on the same accumulator gave wrong sums on this device.)
+        const short8 vh = q2_ops(va[0]), vl = q2_ops(va[1]), v2 = q2_ops(va[2]);
+        q2_parts p2[CT], pw[CT];
+        short8 zh[CT], zl[CT];
+        floatx4 w[CT];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            const q2_parts p0 = q2_split(z0[j]), p1 = q2_split(z1[j]);
+            zl[j] = __builtin_bit_cast(short8, q2_parts{p0[0], p1[0]});
+            zh[j] = __builtin_bit_cast(short8, q2_parts{p0[1], p1[1]});
+            w[j] = q2_mfma32(vh, zl[j], floatx4{0.f, 0.f, 0.f, 0.f});
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j) w[j] = q2_mfma32(vl, zh[j], w[j]);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            p2[j] = q2_split(z2[j]);
+            w[j] = q2_mfma32(v2, q2_lo_hi(p2[j]), w[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j) w[j] = q2_mfma32(v2, q2_hi_lo(p2[j]), w[j]);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) w[j] = q2_mfma32(vh, zh[j], w[j]);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) pw[j] = q2_split(w[j]);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            z0[j] = q2_mfma32(q2_ops(na[0]), q2_lo_hi(pw[j]), z0[j]);
+            z1[j] = q2_mfma32(q2_ops(na[1]), q2_lo_hi(pw[j]), z1[j]);
+            z2[j] = q2_mfma32(q2_ops(na[2]), q2_lo_hi(pw[j]), z2[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            z0[j] = q2_mfma32(q2_ops(na[0]), q2_hi_lo(pw[j]), z0[j]);
+            z1[j] = q2_mfma32(q2_ops(na[1]), q2_hi_lo(pw[j]), z1[j]);
+            z2[j] = q2_mfma32(q2_ops(na[2]), q2_hi_lo(pw[j]), z2[j]);
+        }
+    } else {
+        const float vs[12] = {va[0].x, va[0].y, va[0].z, va[0].w, va[1].x, va[1].y,
+                              va[1].z, va[1].w, va[2].x, va[2].y, va[2].z, va[2].w};
+        const float ns[12] = {na[0].x, na[0].y, na[0].z, na[0].w, na[1].x, na[1].y,
+                              na[1].z, na[1].w, na[2].x, na[2].y, na[2].z, na[2].w};
+        floatx4 w0[CT], w1[CT];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) w0[j] = w1[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) {
+                    const floatx4 z = q == 0 ? z0[j] : q == 1 ? z1[j] : z2[j];
+                    w0[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q + e], z[e], w0[j], 0, 0, 0);
+                    w1[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q + e + 1], z[e + 1], w1[j], 0, 0, 0);
+                }
+        // W as the next product's B operand: register s of lane (lq, l16)
+        // must hold W(4 s + lq, l16), the accumulator holds W(4 lq + r, l16)
+        // in register r, so the 4 x 4 (lq, r) blocks of each column are
+        // transposed across lanes: the off-diagonal 2 x 2 blocks by
+        // v_permlane32_swap, then each 2 x 2 block by v_permlane16_swap
+        float wb[CT][4];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wb[j][r] = w0[j][r] + w1[j][r];
+            auto p0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(wb[j][0]), __float_as_uint(wb[j][2]), false, false);
+            auto p1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(wb[j][1]), __float_as_uint(wb[j][3]), false, false);
+            auto q0 = __builtin_amdgcn_permlane16_swap(p0[0], p1[0], false, false);
+            auto q1 = __builtin_amdgcn_permlane16_swap(p0[1], p1[1], false, false);
+            wb[j][0] = __uint_as_float(q0[0]);
+            wb[j][1] = __uint_as_float(q0[1]);
+            wb[j][2] = __uint_as_float(q1[0]);
+            wb[j][3] = __uint_as_float(q1[1]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                z0[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ns[s], wb[j][s], z0[j], 0, 0, 0);
+                z1[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ns[4 + s], wb[j][s], z1[j], 0, 0, 0);
+                z2[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ns[8 + s], wb[j][s], z2[j], 0, 0, 0);
+            }
+    }
+}
+
+template <int NW, int CT, bool BF>
+__global__ void __launch_bounds__(64 * NW) q2_apply_kernel(int n, int ld, const float* __restrict__ Q2all,
+                                                           float* __restrict__ Zall, int64_t nblk, int nmat) {
+    constexpr int S = 16 * CT;  // columns
     extern __shared__ __align__(16) float q2_smem[];
-    __shared__ int goff[kQ2MaxGroups], done[kQ2MaxGroups], snstep, stuck;
+    // slots passed on by each wave (the last wave: stored to Z), slots taken
+    __shared__ int made[NW], taken[NW], stuck;
     // Workgroup i runs on XCD i mod 8 (round-robin dispatch); XCD x takes the
     // x-th eighth of the (matrix, slab) list in order, so the slabs that run
     // together on one XCD belong to one matrix, start together, and read the
     // same block operands through that XCD's L2.
-    const int nslab = (n + kQ2S - 1) / kQ2S;
+    const int nslab = (n + S - 1) / S;
     const int64_t total = int64_t(nslab) * nmat, per = (total + kXcds - 1) / kXcds;
     const int64_t pos = int64_t(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
     if (pos >= total) return;
     const int b = int(pos / nslab), slab = int(pos % nslab);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c0 = slab * kQ2S;
-    const int P = q2_pitch(n);
-    float* Zs = q2_smem;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+    const int c0 = slab * S;
     float* Z = Zall + size_t(b) * n * ld;
     const float* Q2 = Q2all + size_t(b) * nblk * kQ2BlockFloats;
     const int NG = q2_groups(n);
-    if (tid == 0) {
-        int o = 0, ns = 0;
-        for (int g = 0; g < NG; ++g) {
-            const int t = sb_tasks(n, g * kQ2G);
-            goff[g] = o;
-            done[g] = 0;
-            o += t;
-            ns = max(ns, (NG - 1 - g) + t);
-        }
-        snstep = ns;
-        stuck = 0;
-    }
-    for (int e = tid; e < P * kQ2S; e += kQ2NT) {
-        const int r = e / kQ2S - 3, c = e % kQ2S;
-        Zs[c * P + r + 3] = (r >= 0 && r < n && c0 + c < n) ? Z[size_t(r) * ld + c0 + c] : 0.f;
-    }
+    if (tid < NW) made[tid] = taken[tid] = 0;
+    if (tid == 0) stuck = 0;
     __syncthreads();
-    const int nstep = snstep;
-    const int l16 = lane & 15, lq = lane >> 4;
-    constexpr int NW = kQ2NT / 64;
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    // Group index gi = NG - 1 - g is active at step t when gi <= t and
-    // t - gi < its task count; the task count grows with gi, so the active
-    // groups of a step are an interval [lo, hi] whose ends never decrease.
-    auto tasks_of = [&](int gi) { return sb_tasks(n, (NG - 1 - gi) * kQ2G); };
-    int lo = 0;
-    // this wave's first active group at step t (t never decreasing), or -1
-    auto first_of = [&](int t) {
-        const int hi = min(t, NG - 1);
-        while (lo <= hi && t - lo >= tasks_of(lo)) ++lo;
-        const int g = lo + ((wv - lo) & (NW - 1));
-        return g <= hi ? g : -1;
+    // tasks of group gi, none before the first
+    auto tasks_of = [&](int gi) { return gi < 0 ? 0 : sb_tasks(n, (NG - 1 - gi) * kQ2G); };
+    auto wait_for = [&](int* count, int need) {
+        for (int spin = 0; __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < need; ++spin) {
+            if (spin > (1 << 22) || stuck) {
+                stuck = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
     };
-    auto load_ops = [&](int t, int gi, float4 (&va)[3], float4 (&na)[3]) {
-        const int g = NG - 1 - gi;
-        const float* blk = Q2 + size_t(goff[g] + t - gi) * kQ2BlockFloats;
-        const float4* V4 = reinterpret_cast<const float4*>(blk + lane * (kQ2R / 4));
-        const float4* N4 = reinterpret_cast<const float4*>(blk + kQ2R * kQ2G + kQ2G + lane * 12);
+    auto publish = [&](int* count, int v) {
+        if (lane == 0) __hip_atomic_store(count, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    // this matrix as a raw buffer, offsets in bytes: rows past n lie past its
+    // end, where reads give zeros and stores are dropped (as are the stores of
+    // columns past n, given an offset past any buffer's)
+    const __amdgpu_buffer_rsrc_t rsZ = __builtin_amdgcn_make_buffer_rsrc(Z, 0, n * ld * 4, kBufferWord3);
+    // row tile i of Z
+    auto load_tile = [&](int i, floatx4 (&x)[CT]) {
+        const int at = ((16 * i + 1 + 4 * lq) * ld + c0 + l16) * 4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+                x[j][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsZ, at + r * ld * 4 + 64 * j, 0, 0));
+    };
+    auto store_tile = [&](int i, const floatx4 (&x)[CT]) {
+        const int at = ((16 * i + 1 + 4 * lq) * ld + c0 + l16) * 4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[j][r]), rsZ,
+                                                      c0 + 16 * j + l16 < n ? at + r * ld * 4 + 64 * j : int(0x80000000),
+                                                      0, 0);
+    };
+    // the operands of block (gi, k) at first, then of each next block of this
+    // wave in turn (past the last: of the last again)
+    const float4* ops = reinterpret_cast<const float4*>(Q2) +
+                        (wv < NG ? q2_block_offset(n, NG - 1 - wv) : 0) * (kQ2BlockFloats / 4);
+    auto load_ops = [&](float4 (&va)[3], float4 (&na)[3]) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            va[i] = V4[i];
-            na[i] = N4[i];
+            va[i] = ops[64 * i + lane];
+            na[i] = ops[(kQ2R * kQ2G + kQ2G) / 4 + 64 * i + lane];
         }
     };
-    // the wave's blocks in order (step by step, groups in order within a
-    // step); the next block's operands are in flight while a block runs, also
-    // across the step barrier
-    auto advance = [&](int& tt, int& g) {  // the block after (tt, g), or tt = nstep
-        if (g >= 0 && g + NW <= min(tt, NG - 1)) {
-            g += NW;
-            return;
+    constexpr size_t kSlot = 2 * 16 * S;  // floats per slot
+    int gi = wv, k = 0, K = tasks_of(gi < NG ? gi : -1), Kp = tasks_of(gi < NG ? gi - 1 : -1);
+    int in = 0, out = 0;  // slots taken from the wave before, and passed on
+    floatx4 x0[CT], xa[CT], xb[CT];  // the block's three row tiles
+    floatx4 xn[CT];        // the next group's first tile
+    // first wave: slot k of group gi from Z, once the wave of the group before
+    // has stored it
+    auto fetch = [&](int slot, floatx4 (&pa)[CT], floatx4 (&pb)[CT]) {
+        if (slot >= K) return;
+        if (slot < Kp) {
+            wait_for(&made[NW - 1], in + 1);
+            ++in;
         }
-        g = -1;
-        while (g < 0 && ++tt < nstep) g = first_of(tt);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        const int i = NG - 1 - gi + 2 * slot + 1;
+        load_tile(i, pa);
+        load_tile(i + 1, pb);
     };
-    // Blocks run in the step order without a barrier per step: block (gi,
-    // k) waits until group gi - 1 has finished position k, or all of its
-    // positions where it has no position k (done[gi - 1] >= min(k + 1, its
-    // task count)); with each wave's own earlier blocks this orders it after
-    // every block whose rows it shares and that must come first.  A wait
-    // points to a block of an earlier step and every wave takes its blocks in
-    // step order, so every wait ends.
-    int t = 0, gi = first_of(0);
-    if (gi < 0) advance(t, gi);
     // one block from operands (va, na) while the next block's are read into
     // (vn, nn); the two buffer pairs alternate, so no copy waits for a read
     // in flight
-    auto block = [&](const float4 (&va)[3], const float4 (&na)[3], float4 (&vn)[3], float4 (&nn)[3]) {
-        {
-            int t2 = t, g2 = gi;
-            advance(t2, g2);
-            // the next block's operands (this block's again after the last)
-            load_ops(t2 < nstep ? t2 : t, t2 < nstep ? g2 : gi, vn, nn);
-            __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the block
-            const int k = t - gi;
-            if (gi > 0) {
-                // (bounded: a wait that ran far past any block's time marks
-                // the slab, which is then written back as NaN, instead of
-                // holding the GPU)
-                const int need = min(k + 1, tasks_of(gi - 1));
-                for (int spin = 0;
-                     __hip_atomic_load(&done[gi - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < need; ++spin) {
-                    if (spin > (1 << 22) || stuck) {
-                        stuck = 1;
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
+    auto block = [&](const float4 (&va)[3], const float4 (&na)[3], floatx4 (&pa)[CT], floatx4 (&pb)[CT],
+                     float4 (&vn)[3], float4 (&nn)[3], floatx4 (&qa)[CT], floatx4 (&qb)[CT]) {
+        const int g = NG - 1 - gi;
+        const bool lastk = k + 1 == K;
+        if (!lastk)
+            ops += kQ2BlockFloats / 4;
+        else if (gi + NW < NG)
+            ops = reinterpret_cast<const float4*>(Q2) + q2_block_offset(n, g - NW) * (kQ2BlockFloats / 4);
+        load_ops(vn, nn);
+        if (k == 0) {
+#pragma unroll
+            for (int j = 0; j < CT; ++j) x0[j] = xn[j];
+            if (gi + NW < NG) load_tile(g - NW, xn);
+        }
+        if (wv == 0) {
+            // slot k, with slot k + 1 on its way
+            if (k == 0) {
+                fetch(0, pa, pb);
+                fetch(1, qa, qb);
             }
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                xa[j] = pa[j];
+                xb[j] = pb[j];
+            }
+            fetch(k + 2, pa, pb);
+        } else if (k < Kp) {
+            wait_for(&made[wv - 1], in + 1);
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-            const int g = NG - 1 - gi;
-            const int rb = g * kQ2G + 1 + k * kBandNB;
-            // this lane's column, from the block's first row
-            float* zc = Zs + l16 * P + rb + 3;
-            floatx4 zq[3];
+            const floatx4* slot = reinterpret_cast<const floatx4*>(q2_smem + (size_t(wv - 1) * kQ2Fifo + in % kQ2Fifo) *
+                                                                                 kSlot) + lane;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) zq[q] = *reinterpret_cast<const floatx4*>(zc + 16 * q + 4 * lq);
-            floatx4 acc[3];
-            if constexpr (BF) {
-                // split-BF16x3 (x = hi + lo, products lo*hi + hi*lo + hi*hi
-                // accumulated in FP32), the operands' parts stored by
-                // q2_prep_kernel.  Lane (lq, l16) holds k = 4 lq .. 4 lq + 3
-                // of its row (A) or column (B), so W = V^T Zb comes out as the
-                // update's B operand, W(4 lq + r, l16) in register r, with no
-                // transpose.  Two 16-deep products share one 16x16x32 MFMA
-                // (the same 16 cycles as a 16x16x16): lo*hi beside hi*lo, and
-                // two row tiles' hi*hi.  An odd product has a zero half: a
-                // 16x16x16 and a 16x16x32 one after the other on the same
-                // accumulator gave wrong sums on this device.
-                constexpr shortx4 zero4 = {0, 0, 0, 0};
-                short8 vhl[3], zlh[3];
-                shortx4 vh[3], zh[3];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    const shortx4 vl = q2_half(va[q].z, va[q].w);
-                    shortx4 zl;
-                    vh[q] = q2_half(va[q].x, va[q].y);
-                    split_bf16(zq[q][0], zq[q][1], zq[q][2], zq[q][3], zh[q], zl);
-                    vhl[q] = q2_cat(vl, vh[q]);
-                    zlh[q] = q2_cat(zh[q], zl);
-                }
-                floatx4 w = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int q = 0; q < 3; ++q) w = q2_mfma32(vhl[q], zlh[q], w);
-                w = q2_mfma32(q2_cat(vh[0], vh[1]), q2_cat(zh[0], zh[1]), w);
-                w = q2_mfma32(q2_cat(vh[2], zero4), q2_cat(zh[2], zero4), w);
-                shortx4 wh, wl;
-                split_bf16(w[0], w[1], w[2], w[3], wh, wl);
-                const short8 whl = q2_cat(wh, wl), wh0 = q2_cat(wh, zero4);
-#pragma unroll
-                for (int rt = 0; rt < 3; ++rt) {
-                    const shortx4 nh = q2_half(na[rt].x, na[rt].y), nl = q2_half(na[rt].z, na[rt].w);
-                    acc[rt] = q2_mfma32(q2_cat(nl, nh), whl, zq[rt]);
-                    acc[rt] = q2_mfma32(q2_cat(nh, zero4), wh0, acc[rt]);
-                }
-            } else {
-            const float vs[12] = {va[0].x, va[0].y, va[0].z, va[0].w, va[1].x, va[1].y,
-                                  va[1].z, va[1].w, va[2].x, va[2].y, va[2].z, va[2].w};
-            const float ns[12] = {na[0].x, na[0].y, na[0].z, na[0].w, na[1].x, na[1].y,
-                                  na[1].z, na[1].w, na[2].x, na[2].y, na[2].z, na[2].w};
-            floatx4 w0 = {0.f, 0.f, 0.f, 0.f}, w1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                w0 = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q], zq[q][0], w0, 0, 0, 0);
-                w1 = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q + 1], zq[q][1], w1, 0, 0, 0);
-                w0 = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q + 2], zq[q][2], w0, 0, 0, 0);
-                w1 = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[4 * q + 3], zq[q][3], w1, 0, 0, 0);
+            for (int j = 0; j < CT; ++j) {
+                xa[j] = slot[64 * j];
+                xb[j] = slot[64 * (CT + j)];
             }
-            // W as the next product's B operand: register s of lane (lq, l16)
-            // must hold W(4 s + lq, l16), the accumulator holds W(4 lq + r,
-            // l16) in register r, so the 4 x 4 (lq, r) blocks of each column
-            // are transposed across lanes: the off-diagonal 2 x 2 blocks by
-            // v_permlane32_swap, then each 2 x 2 block by v_permlane16_swap
-            float wb[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) wb[r] = w0[r] + w1[r];
-            {
-                auto p0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(wb[0]), __float_as_uint(wb[2]), false, false);
-                auto p1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(wb[1]), __float_as_uint(wb[3]), false, false);
-                auto q0 = __builtin_amdgcn_permlane16_swap(p0[0], p1[0], false, false);
-                auto q1 = __builtin_amdgcn_permlane16_swap(p0[1], p1[1], false, false);
-                wb[0] = __uint_as_float(q0[0]);
-                wb[1] = __uint_as_float(q0[1]);
-                wb[2] = __uint_as_float(q1[0]);
-                wb[3] = __uint_as_float(q1[1]);
-            }
-#pragma unroll
-            for (int rt = 0; rt < 3; ++rt) acc[rt] = *reinterpret_cast<const floatx4*>(zc + 16 * rt + 4 * lq);
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int rt = 0; rt < 3; ++rt)
-                    acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ns[4 * rt + s], wb[s], acc[rt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int rt = 0; rt < 3; ++rt) *reinterpret_cast<floatx4*>(zc + 16 * rt + 4 * lq) = acc[rt];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-            if (lane == 0) __hip_atomic_store(&done[gi], k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            t = t2;
-            gi = g2;
+            publish(&taken[wv], ++in);
+        } else {
+#pragma unroll
+            for (int j = 0; j < CT; ++j) xa[j] = xb[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the block
+        if constexpr (CT == 4) {
+            q2_block<2, BF>(va, na, *reinterpret_cast<floatx4(*)[2]>(&x0[0]), *reinterpret_cast<floatx4(*)[2]>(&xa[0]),
+                            *reinterpret_cast<floatx4(*)[2]>(&xb[0]));
+            q2_block<2, BF>(va, na, *reinterpret_cast<floatx4(*)[2]>(&x0[2]), *reinterpret_cast<floatx4(*)[2]>(&xa[2]),
+                            *reinterpret_cast<floatx4(*)[2]>(&xb[2]));
+        } else {
+            q2_block<CT, BF>(va, na, x0, xa, xb);
+        }
+        if (wv == NW - 1 || gi == NG - 1) {
+            // stored slots are published a block later, when their stores
+            // have long gone, or at the group's end
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            publish(&made[wv], out);
+            store_tile(g + 2 * k, x0);
+            store_tile(g + 2 * k + 1, xa);
+            ++out;
+            if (lastk) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                publish(&made[wv], out);
+            }
+        } else {
+            wait_for(&taken[wv + 1], out - kQ2Fifo + 1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            floatx4* slot = reinterpret_cast<floatx4*>(q2_smem + (size_t(wv) * kQ2Fifo + out % kQ2Fifo) * kSlot) + lane;
+#pragma unroll
+            for (int j = 0; j < CT; ++j) {
+                slot[64 * j] = x0[j];
+                slot[64 * (CT + j)] = xa[j];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            publish(&made[wv], ++out);
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j) x0[j] = xb[j];
+        ++k;
+        if (lastk) {
+            gi += NW;
+            k = 0;
+            K = tasks_of(gi < NG ? gi : -1);
+            Kp = tasks_of(gi < NG ? gi - 1 : -1);
         }
     };
-    float4 va[3], na[3], vb[3], nb[3];
-    load_ops(gi < 0 ? 0 : t, gi < 0 ? 0 : gi, va, na);  // (0, 0) is a block of every matrix
-    while (t < nstep) {
-        block(va, na, vb, nb);
-        if (t >= nstep) break;
-        block(vb, nb, va, na);
+    if (gi < NG) {
+        float4 va[3], na[3], vb[3], nb[3];
+        floatx4 pa[CT], pb[CT], qa[CT], qb[CT];  // the first wave's slots, read from Z ahead
+        load_tile(NG - 1 - gi, xn);
+        load_ops(va, na);
+        while (true) {
+            block(va, na, pa, pb, vb, nb, qa, qb);
+            if (gi >= NG) break;
+            block(vb, nb, qa, qb, va, na, pa, pb);
+            if (gi >= NG) break;
+        }
     }
     __syncthreads();
-    const bool bad = stuck != 0;
-    for (int e = tid; e < n * kQ2S; e += kQ2NT) {
-        const int r = e / kQ2S, c = e % kQ2S;
-        if (c0 + c < n) Z[size_t(r) * ld + c0 + c] = bad ? __builtin_nanf("") : Zs[c * P + r + 3];
-    }
+    if (stuck)
+        for (int e = tid; e < n * S; e += 64 * NW)
+            if (c0 + e % S < n) Z[size_t(e / S) * ld + c0 + e % S] = __builtin_nanf("");
 }
 
 int q2_prep(int batch, int n, float* Q2, hipStream_t s, bool bf16) {
@@ -1402,39 +1510,50 @@ int q2_prep(int batch, int n, float* Q2, hipStream_t s, bool bf16) {
     return CIR_OK;
 }
 
-// Workgroup width of q2_apply_kernel: 1024 threads (16 waves, candidate 0)
-// or 512, timed per size bucket on the first call (tuner.hpp) over a copy of
-// the first few matrices' eigenvectors (the kernel works in place).
-template <int NT, bool BF>
+// Waves of q2_apply_kernel's workgroup: 12 (candidate 0) or 8, timed per size
+// bucket on the first call (tuner.hpp) over a copy of the first few matrices'
+// eigenvectors (the kernel works in place).
+template <int NW, int CT, bool BF>
 static int q2_launch(int batch, int n, int ld, const float* Q2, float* Z, int64_t nblk, hipStream_t s) {
-    const size_t sm = size_t(q2_pitch(n)) * kQ2S * sizeof(float);
-    CIR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q2_apply_kernel<NT, BF>),
+    constexpr size_t sm = size_t(NW - 1) * kQ2Fifo * 2 * CT * 256 * sizeof(float);
+    CIR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&q2_apply_kernel<NW, CT, BF>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(sm)));
     // the one-dimensional grid holds at most 2^32 - 1 threads: very large
     // batches go in several launches
-    const int64_t nslab = ceil_div(n, kQ2S);
-    const int64_t most = std::max<int64_t>(1, ((int64_t(1) << 32) - 1) / (int64_t(NT) * nslab) - kXcds);
+    const int64_t nslab = ceil_div(n, 16 * CT);
+    const int64_t most = std::max<int64_t>(1, ((int64_t(1) << 32) - 1) / (int64_t(64 * NW) * nslab) - kXcds);
     for (int64_t b0 = 0; b0 < batch; b0 += most) {
         const int nb = int(std::min<int64_t>(most, batch - b0));
         dim3 grid(unsigned(ceil_div(nslab * nb, int64_t(kXcds)) * kXcds));
-        hipLaunchKernelGGL((q2_apply_kernel<NT, BF>), grid, dim3(NT), sm, s, n, ld, Q2 + size_t(b0) * nblk * kQ2BlockFloats,
-                           Z + size_t(b0) * n * ld, nblk, nb);
+        hipLaunchKernelGGL((q2_apply_kernel<NW, CT, BF>), grid, dim3(64 * NW), sm, s, n, ld,
+                           Q2 + size_t(b0) * nblk * kQ2BlockFloats, Z + size_t(b0) * n * ld, nblk, nb);
         CIR_CHECK_LAUNCH();
     }
     return CIR_OK;
 }
 
+// 32 columns per workgroup, or 16 where that leaves CUs idle.
+template <int NW, bool BF>
+static int q2_launch(int batch, int n, int ld, const float* Q2, float* Z, int64_t nblk, hipStream_t s) {
+    return ceil_div(n, 32) * batch >= 2 * kQ2Cus ? q2_launch<NW, 2, BF>(batch, n, ld, Q2, Z, nblk, s)
+                                                 : q2_launch<NW, 1, BF>(batch, n, ld, Q2, Z, nblk, s);
+}
+
 int q2_apply(int batch, int n, int ld, const float* Q2, float* Z, hipStream_t s, bool bf16) {
     const int64_t nblk = q2_blocks(n);
     if (nblk <= 0) return CIR_OK;
-    const size_t sm = size_t(q2_pitch(n)) * kQ2S * sizeof(float);
-    if (sm > 160 * 1024) return fail(CIR_ERR_ARG, "q2_apply: n too large for the LDS slab");
+    // split BF16, slabs of 64 columns for two rounds of the CUs or more: 8
+    // waves of 64 columns, each block's operands and bookkeeping serving twice
+    // the columns (256 matrices of N = 2048: 34.7 ms, 12 waves of 32 columns
+    // 39.3; a workgroup takes 1.1 ms against 0.64, so fewer than two rounds
+    // are better off with the narrower one).  FP32 is bound by its MFMAs.
+    if (bf16 && ceil_div(n, 64) * batch >= 2 * kQ2Cus) return q2_launch<8, 4, true>(batch, n, ld, Q2, Z, nblk, s);
     auto launch = [&](int cand, int nb, float* Zp) {
         if (bf16)
-            return cand == 0 ? q2_launch<1024, true>(nb, n, ld, Q2, Zp, nblk, s)
-                             : q2_launch<512, true>(nb, n, ld, Q2, Zp, nblk, s);
-        return cand == 0 ? q2_launch<1024, false>(nb, n, ld, Q2, Zp, nblk, s)
-                         : q2_launch<512, false>(nb, n, ld, Q2, Zp, nblk, s);
+            return cand == 0 ? q2_launch<12, true>(nb, n, ld, Q2, Zp, nblk, s)
+                             : q2_launch<8, true>(nb, n, ld, Q2, Zp, nblk, s);
+        return cand == 0 ? q2_launch<12, false>(nb, n, ld, Q2, Zp, nblk, s)
+                         : q2_launch<8, false>(nb, n, ld, Q2, Zp, nblk, s);
     };
     const TuneKey key{"q2_apply_threads", {size_bucket(n), bf16 ? 1 : 0, 0, 0, 0}};
     int cand = tune_lookup(key);
