@@ -12,8 +12,8 @@ constexpr int kBandW = 2 * kBandNB;   // stored band row: r - c in [0, 2 NB)
 constexpr int kQ2G = 16;              // sweeps per compact-WY block of the bulge-chasing reflectors
 constexpr int kQ2R = 48;              // rows of such a block (NB + kQ2G - 1, padded)
 
-// Largest n of the stage-1 register panel (4 rows of 512 threads below the band).
-inline int sb_max_n() { return 4 * 512 + kBandNB; }
+// Largest n of the stage-1 register panel (6 rows of 512 threads below the band).
+inline int sb_max_n() { return 6 * 512 + kBandNB; }
 
 // Tasks (block positions) of bulge-chasing sweep s: rows s+1+k NB, k < count.
 __host__ __device__ inline int sb_tasks(int n, int s) { return (s <= n - 3) ? (n - 2 - s) / kBandNB + 1 : 0; }

@@ -615,18 +615,17 @@ int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, 
     for (; j0 + NB < n - 1; j0 += NB) {
         const int r0 = j0 + NB, m = n - r0;
         const int rpt = int(ceil_div(m, kPanNT));
-        if (rpt <= 1)
-            hipLaunchKernelGGL(sb_panel_kernel<1>, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, ld, j0, A, BND, tau,
-                               P, Yh);
-        else if (rpt <= 2)
-            hipLaunchKernelGGL(sb_panel_kernel<2>, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, ld, j0, A, BND, tau,
-                               P, Yh);
-        else if (rpt <= 3)
-            hipLaunchKernelGGL(sb_panel_kernel<3>, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, ld, j0, A, BND, tau,
-                               P, Yh);
-        else
-            hipLaunchKernelGGL(sb_panel_kernel<4>, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, ld, j0, A, BND, tau,
-                               P, Yh);
+        auto panel = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, ld, j0, A, BND, tau, P, Yh);
+        };
+        switch (rpt) {
+            case 1: panel(sb_panel_kernel<1>); break;
+            case 2: panel(sb_panel_kernel<2>); break;
+            case 3: panel(sb_panel_kernel<3>); break;
+            case 4: panel(sb_panel_kernel<4>); break;
+            case 5: panel(sb_panel_kernel<5>); break;
+            default: panel(sb_panel_kernel<6>); break;
+        }
         CIR_CHECK_LAUNCH();
         const int nbt = int(ceil_div(m, 32));
         const dim3 grid = xcd_grid(int(ceil_div(nbt, 4)), batch);
@@ -1017,8 +1016,9 @@ __global__ void __launch_bounds__(kSbNT) sb2st_kernel(int n, float* __restrict__
     }
 }
 
-bool deterministic_eigh_size(int n) { return n >= 2 * kBandNB + 2 && n <= sb_max_n(); }
-int deterministic_eigh_max() { return sb_max_n(); }
+// (the documented range of the deterministic key, short of sb_max_n())
+int deterministic_eigh_max() { return 2080; }
+bool deterministic_eigh_size(int n) { return n >= 2 * kBandNB + 2 && n <= deterministic_eigh_max(); }
 
 int sb2st(int batch, int n, float* BND, float* d, float* e, float* Q2, hipStream_t s) {
     if (n < 1) return fail(CIR_ERR_ARG, "sb2st: bad size");

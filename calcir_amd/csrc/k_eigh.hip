@@ -1675,7 +1675,8 @@ inline size_t larft_smem_bytes(size_t esz) { return (size_t(kBtNB) * (kBtNB + 1)
 //   one stage, batched        one workgroup per matrix
 // The lines, from both sides measured (ms per batch): two stages against one
 // workgroup per matrix, 64 matrices, n = 320 5.1 / 4.6, n = 400 7.0 / 6.8, n =
-// 512 9.5 / 10.7, n = 640 13.4 / 17.1, 24 of n = 1000 23.8 / 43; against the
+// 512 9.5 / 10.7, n = 640 13.4 / 17.1, 24 of n = 1000 23.8 / 43, 32 of n = 2100
+// 84 / 277, 24 of n = 3072 168 / 741; against the
 // whole-GPU form, one matrix of n = 512 8.8 / 13.8, n = 1024 22.6 / 30.7, n =
 // 2048 66.5 / 73.5, 8 of n = 512 8.9 / 104.  The whole-GPU form takes a time
 // that grows with the batch (n = 1024 in FP64: 27 per matrix), the batched form
@@ -1707,13 +1708,19 @@ inline bool use_whole_gpu(int batch, int n) {
 // and D = V^T C, lambda_j += D_jj and V += V E, E_ij = D_ij / (lambda_j -
 // lambda_i).  E is antisymmetric, so V stays orthogonal to second order.
 // Only C needs FP32's full accuracy (H's diagonal, its largest entries, is
-// taken out of the product and applied in FP64 with the eigenvalue); D and E
-// are corrections, formed in split-BF16x3.  After it: eigenvalues 1.6e-7, the
-// density 4e-7.  One matrix of n = 2048: 0.8 of 66 ms; 48 of n = 766: 1.7 of 18.
-constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16;
-inline bool use_refine(int batch, int n) { return n < kRefineMaxN || batch <= kRefineMaxBatch; }
+// taken out of the product and applied in FP64 with the eigenvalue; the rest
+// is summed in runs, an FP32 MFMA chain over all rows biases the eigenvalues by
+// 4e-6); D and E are corrections, formed in split-BF16x3.  The vectors are then
+// scaled to length one (first-order rotations lengthen them by E_ij^2, 2e-7 on
+// average).  After it: eigenvalues 2e-8, the density 5e-8 .. 2e-7 (one stage:
+// 2e-7 .. 3e-7 and 1e-7 .. 4e-7).  One matrix of n = 2048: 0.9 of 42 ms; 48 of
+// n = 766: 1.7 of 13; 24 of n = 3072: 30 of 168.  Above kRefineAboveN, where
+// only the one-stage form used to run, it is always made.
+constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16, kRefineAboveN = 2080;
+inline bool use_refine(int batch, int n) { return n < kRefineMaxN || batch <= kRefineMaxBatch || n > kRefineAboveN; }
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
+constexpr int kRqRun = 128;          // rows summed in one MFMA chain
 // C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major:
 // 64 x 64 tiles, four waves of one 32x32 fragment on the FP32 MFMA.
 __global__ void __launch_bounds__(256)
@@ -1738,9 +1745,11 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
             rb[q] = (k < n) ? V[size_t(kc) * ld + cn] : 0.f;
         }
     };
-    floatx16 acc;
+    // summed in runs of kRqRun rows: each run's sum is small beside the whole,
+    // so is its rounding
+    floatx16 acc, sum;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
+    for (int q = 0; q < 16; ++q) acc[q] = sum[q] = 0.f;
     load(0);
     for (int kb = 0; kb < n; kb += kRqK) {
         __syncthreads();
@@ -1751,6 +1760,13 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
         }
         __syncthreads();
         load(kb + kRqK);
+        if (kb % kRqRun == 0) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                sum[q] += acc[q];
+                acc[q] = 0.f;
+            }
+        }
 #pragma unroll
         for (int k = 0; k < kRqK; k += 2)
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[k + h][wm + l32], Bs[k + h][wn + l32], acc, 0, 0, 0);
@@ -1762,7 +1778,7 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
         const int i = m0 + wm + 8 * (q >> 2) + 4 * h + (q & 3);
         if (i < n && k < n) {
             const double v = double(V[size_t(i) * ld + k]);
-            C[size_t(i) * ld + k] = float(double(acc[q]) + (double(H[size_t(i) * ld + i]) - lam) * v);
+            C[size_t(i) * ld + k] = float(double(sum[q] + acc[q]) + (double(H[size_t(i) * ld + i]) - lam) * v);
         }
     }
 }
@@ -1834,13 +1850,33 @@ correct_w_kernel(int n, const float* __restrict__ dlall, double* __restrict__ wa
     for (int k = threadIdx.x; k < n; k += 1024) w[k] = a[k];
 }
 
-// V += P over n rows of pitch ld (columns past n: P's are not defined)
+// dl_j = 1 / |v_j + p_j| over n rows of pitch ld: 64 columns per workgroup, the
+// rows over its waves, summed in FP64 in a fixed order.
+__global__ void __launch_bounds__(1024)
+norms_kernel(int n, int ld, const float* __restrict__ Pall, const float* __restrict__ Vall, float* __restrict__ dlall) {
+    __shared__ double red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = blockIdx.x * 64 + lane, jc = min(j, n - 1);
+    const size_t mat = size_t(blockIdx.y) * n * ld;
+    double s = 0.0;
+    for (int i = wave; i < n; i += 16) {
+        const float v = Vall[mat + size_t(i) * ld + jc] + Pall[mat + size_t(i) * ld + jc];
+        s += double(v) * double(v);
+    }
+    red[wave][lane] = s;
+    __syncthreads();
+    if (wave != 0 || j >= n) return;
+    for (int w = 1; w < 16; ++w) s += red[w][lane];
+    dlall[size_t(blockIdx.y) * n + j] = float(rsqrt(s));
+}
+
+// V = (V + P) diag(dl) over n rows of pitch ld (columns past n: P's are not
+// defined)
 __global__ void __launch_bounds__(256)
-add_rows_kernel(int n, int ld, const float* __restrict__ Pall, float* __restrict__ Vall) {
+add_rows_kernel(int n, int ld, const float* __restrict__ Pall, const float* __restrict__ dlall, float* __restrict__ Vall) {
     const int j = blockIdx.x * 256 + threadIdx.x;
     if (j >= n) return;
     const size_t o = (size_t(blockIdx.z) * n + blockIdx.y) * ld + j;
-    Vall[o] += Pall[o];
+    Vall[o] = (Vall[o] + Pall[o]) * dlall[size_t(blockIdx.z) * n + j];
 }
 
 // The matrices' copy for the refinement
@@ -2105,10 +2141,13 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
             hipLaunchKernelGGL(rotation_kernel, dim3(nr, nr, unsigned(batch)), dim3(256), 0, s, n, ld, w, H, dl);
             CIR_CHECK_LAUNCH();
             CIR_TRY(product(V, ld, 1, H, C));
-            hipLaunchKernelGGL(add_rows_kernel, dim3(nc, unsigned(n), unsigned(batch)), dim3(256), 0, s, n, ld, C, V);
-            CIR_CHECK_LAUNCH();
             hipLaunchKernelGGL(correct_w_kernel, dim3(unsigned(batch)), dim3(1024), 2 * size_t(n) * sizeof(double), s, n, dl,
                                w);
+            CIR_CHECK_LAUNCH();
+            hipLaunchKernelGGL(norms_kernel, dim3(unsigned(ceil_div(n, 64)), unsigned(batch)), dim3(1024), 0, s, n, ld, C, V,
+                               dl);
+            CIR_CHECK_LAUNCH();
+            hipLaunchKernelGGL(add_rows_kernel, dim3(nc, unsigned(n), unsigned(batch)), dim3(256), 0, s, n, ld, C, dl, V);
             CIR_CHECK_LAUNCH();
         }
     }

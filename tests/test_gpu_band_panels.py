@@ -16,7 +16,8 @@ DEV = "cuda:0"
 # the first panel has n - 32 rows, 512 per register row; 17 matrices of
 # N >= 1024 take the route without a correction of the eigenpairs
 @pytest.mark.parametrize("n,batch,band", [(544, 2, 0), (545, 2, 0), (1056, 17, 0), (1057, 17, 0), (1063, 17, 20),
-                                          (1568, 17, 0), (1569, 17, 0), (2080, 17, 0), (2079, 17, 33)])
+                                          (1568, 17, 0), (1569, 17, 0), (2080, 17, 0), (2079, 17, 33), (2081, 2, 0),
+                                          (2592, 2, 0), (2593, 2, 31), (3104, 2, 0), (3105, 2, 0)])
 def test_two_stage_at_panel_edges(n, batch, band):
     announce("band panels n=%d batch=%d band=%d" % (n, batch, band))
     rng = np.random.default_rng(n)
