@@ -656,9 +656,9 @@ constexpr int kSbG = 8;                  // sweeps per group = waves per workgro
 constexpr int kSbNT = 64 * kSbG;
 constexpr int kSbWR = 512;               // window rows (power of two)
 constexpr int kSbWP = kBandW;            // window row pitch (floats)
-// window, per-wave task scratch (v, two reduced vectors, a per-lane sink),
+// window, per-wave task scratch (v and a per-lane sink),
 // and one 16-byte sink for the read-ahead pieces of threads with no row to add
-constexpr int kSbScratch = 3 * kBandNB + 64;
+constexpr int kSbScratch = kBandNB + 64;
 constexpr size_t kSbSmemFloats = size_t(kSbWR) * kSbWP + size_t(kSbG) * kSbScratch + 4;
 static_assert(kBandNB * (kBandW / 4) <= kSbNT, "one step's new band rows must fit one 16-byte piece per thread");
 static_assert((2 * kSbG - 1) * kBandNB + kBandNB <= kSbWR, "window must hold a step's rows plus the read-ahead");
@@ -712,31 +712,38 @@ __device__ __forceinline__ float half_sum(float x) {
     return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
 }
 
+// Column of the block that register c of a lane of half h holds (the row that
+// register c of a 32x32 MFMA accumulator holds there).
+__device__ __forceinline__ constexpr int sb_col(int c, int h) { return 8 * (c >> 2) + 4 * h + (c & 3); }
+
 // One wave's share of a bulge-chasing step: task (s, k) of its sweep.
-// Lane l: row i = l & 31 of the task's block, column half h = l >> 5
-// (columns 16 h .. 16 h + 15).  pv / ptau: the sweep's previous reflector
-// (columns of the previous block, this lane's half), replaced by this task's;
-// q2val: this task's reflector as a Q2 block column.  The wave's scratch sc
-// holds v, the two reduced vectors and a per-lane sink for masked-off stores.
+// Lane l: row i = l & 31 of the task's blocks and 16 of their columns, sb_col(c,
+// l >> 5).  pv / pvi / ptau: the sweep's previous reflector (at this lane's 16
+// columns, at column i, its factor), replaced by this task's; q2val: this task's
+// reflector as a Q2 block column.  The wave's scratch sc holds v and a per-lane
+// sink for masked-off stores.
 // FULL: a block of 32 rows, every task but a sweep's last.  The last one's
 // lanes outside the block read a row inside it and discard the value.  All the
-// window's reads are issued together, the diagonal block's at the start (no
-// earlier part of the task writes it); read where they are used, the compiler
-// put each of the masked ones into a branch of its own with a wait behind it
-// (16 LDS latencies per task).  dofs: window offset of D(max(i, j), min(i, j))
-// for column j = 16 h + c, against the block's first row; rows are 64 floats,
-// so an offset past the window's end wraps with a mask.  The left application
-// to the block below and the two-sided update of the diagonal block share one
-// pass of reductions.
+// window's reads are issued together at the start; read where they are used,
+// the compiler put each of the masked ones into a branch of its own with a wait
+// behind it (16 LDS latencies per task).  dofs: window offset of D(max(i, j),
+// min(i, j)) for column j = sb_col(c, h), against the block's first row; rows
+// are 64 floats, so an offset past the window's end wraps with a mask.
+// Issue-bound (two waves per SIMD): the block below, B, is read a second time
+// by columns (tb: rows sb_col(c, h) of column i), so that v^T B is a sum within
+// the lane like the other products, with the right application's part (v . f)
+// pv taken off afterwards, and the two rank-one updates of either block are one
+// 32x32x2 MFMA.  With v^T B reduced across lanes after the right application,
+// both reduced vectors handed round through LDS and the updates on the vector
+// units: 23.4 ms for one matrix of N = 2048, 4.4 for 48 of N = 766; this takes
+// 19.7 and 3.8.
 template <bool FULL>
 __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, float* sc, const int (&dofs)[16],
-                                        float (&pv)[16], float& ptau, float& q2val, int lane) {
+                                        float (&pv)[16], float& pvi, float& ptau, float& q2val, int lane) {
     constexpr int NB = kBandNB;
     constexpr int WMASK = kSbWR * kSbWP - 1;
     float* vs = sc;
-    float* wsB = sc + NB;
-    float* wsD = sc + 2 * NB;
-    float* sink = sc + 3 * NB + lane;
+    float* sink = sc + NB + lane;
     const int i = lane & 31, h = lane >> 5;
     const int r0 = s + 1 + k * NB;
     const int len = FULL ? NB : min(NB, n - r0);
@@ -745,53 +752,71 @@ __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, 
     // this lane's row (clamped into the block): element (row, c) at wr[row - c]
     const int ic = FULL ? i : min(i, len - 1);
     float* const wr = w + ((R + ic * kSbWP) & WMASK);
-    float bk[16], dd[16];
+    floatx16 bk, dd;
+    float tb[16];
     float x = 0.f;
     if (k == 0) {
         x = wr[ic + 1];  // column s
     } else {
-        // the block below the previous one, columns r0 - NB + 16 h ..
-        const float* bp = wr + (NB + ic - 16 * h - 15);
+        // the block below the previous one
+        const float* bp = wr + (NB + ic - 4 * h - 27);
 #pragma unroll
-        for (int c = 0; c < 16; ++c) bk[c] = bp[15 - c];
+        for (int c = 0; c < 16; ++c) bk[c] = bp[27 - sb_col(c, 0)];
     }
     // the diagonal block D (rows/cols r0 .. r0+len-1), both triangles, from
-    // its lower triangle
+    // its lower triangle, and B by columns
+    if (FULL && R <= (kSbWR - NB) * kSbWP) {  // no row wraps
+        const float* base = w + R;
+        const float* tp = base + (NB - i + 4 * h * (kSbWP + 1));
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        if constexpr (FULL) {
-            dd[c] = w[(R + dofs[c]) & WMASK];
-        } else {
-            const int j = 16 * h + c, ra = min(max(i, j), len - 1), cb = min(min(i, j), ra);
-            dd[c] = w[(R + ra * kSbWP + ra - cb) & WMASK];
+        for (int c = 0; c < 16; ++c) {
+            dd[c] = base[dofs[c]];
+            tb[c] = tp[sb_col(c, 0) * (kSbWP + 1)];
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int j = sb_col(c, h), jc = FULL ? j : min(j, len - 1);
+            if constexpr (FULL) {
+                dd[c] = w[(R + dofs[c]) & WMASK];
+            } else {
+                const int ra = min(max(i, j), len - 1), cb = min(min(i, j), ra);
+                dd[c] = w[(R + ra * kSbWP + ra - cb) & WMASK];
+            }
+            tb[c] = w[((R + jc * kSbWP) & WMASK) + NB + jc - i];
         }
     }
     if constexpr (!FULL) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) asm volatile("" : "+v"(dd[c]));  // read above, masked here
-#pragma unroll
-        for (int c = 0; c < 16; ++c) dd[c] = (rowok && 16 * h + c < len) ? dd[c] : 0.f;
+        for (int c = 0; c < 16; ++c) {  // read above, masked here
+            float t = dd[c];
+            asm volatile("" : "+v"(t));
+            dd[c] = (rowok && sb_col(c, h) < len) ? t : 0.f;
+        }
         if (k == 0) {
             x = rowok ? x : 0.f;
         } else {
 #pragma unroll
-            for (int c = 0; c < 16; ++c) asm volatile("" : "+v"(bk[c]));
-#pragma unroll
-            for (int c = 0; c < 16; ++c) bk[c] = rowok ? bk[c] : 0.f;
+            for (int c = 0; c < 16; ++c) {
+                float t = bk[c];
+                asm volatile("" : "+v"(t));
+                bk[c] = rowok ? t : 0.f;
+            }
         }
     }
+    float f = 0.f;
     if (k > 0) {
-        // the previous reflector from the right (this fills the bulge)
+        // the previous reflector from the right (this fills the bulge): B -= f
+        // pv^T, applied with the new one's below; of it the first column here
+        // (pv(0) = 1), from the h = 0 lanes
         float u0 = 0.f, u1 = 0.f;
 #pragma unroll
         for (int c = 0; c < 16; c += 2) {
             u0 += bk[c] * pv[c];
             u1 += bk[c + 1] * pv[c + 1];
         }
-        const float f = ptau * half_pair_sum(u0 + u1);
-#pragma unroll
-        for (int c = 0; c < 16; ++c) bk[c] -= f * pv[c];
-        x = from_low_half(bk[0]);  // the block's first column, from the h = 0 lanes
+        f = ptau * half_pair_sum(u0 + u1);
+        x = from_low_half(bk[0]) - f;
     }
     // reflector annihilating x[1..len) (x is the same in both halves)
     const float sigma = half_sum((i >= 1 && rowok) ? x * x : 0.f);
@@ -804,7 +829,7 @@ __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, 
     float vj[16];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const float4 t = reinterpret_cast<const float4*>(vs + 16 * h)[q];
+        const float4 t = *reinterpret_cast<const float4*>(vs + 8 * q + 4 * h);
         vj[4 * q] = t.x;
         vj[4 * q + 1] = t.y;
         vj[4 * q + 2] = t.z;
@@ -819,62 +844,36 @@ __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, 
     }
     const float pp = tau * half_pair_sum(p0a + p1a);
     if (k > 0) {
-        if (h == 0) bk[0] = (i == 0) ? beta : 0.f;
-        // the new reflector from the left on the block's other columns:
-        // w(c) = v^T B(:, c), reduce-scattered over the half's 32 lanes
-        float t[16];
+        // the new reflector from the left on the block's other columns: w =
+        // B^T v - (v . f) pv in lane i for column i, B -= f pv^T + tau v w^T
+        float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) t[c] = vi * bk[c];
-        float z[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[c]), __float_as_uint(t[c + 8]), false,
-                                                             false);
-            z[c] = brow_sum16(__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
+        for (int c = 0; c < 16; c += 2) {
+            s0 += tb[c] * vj[c];
+            s1 += tb[c + 1] * vj[c + 1];
         }
-        // 16-lane row R = l >> 4 holds columns 16 h + 8 (R & 1) + c
-        const int ri = lane & 15;
-        float zz = z[0];
-#pragma unroll
-        for (int c = 1; c < 8; ++c) zz = (ri == c) ? z[c] : zz;
-        if (ri < 8) wsB[16 * h + 8 * ((lane >> 4) & 1) + ri] = zz;
+        const float vf = half_sum(vi * f);
+        const float tw = half_pair_sum(s0 + s1) - vf * pvi;
+        bk = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? pvi : tw, h == 0 ? -f : -tau * vi, bk, 0, 0, 0);
     }
     const float kk = half_sum(pp * vi);  // (pp is the same in both halves)
-    const float K = -0.5f * tau * kk;
-    const float wi = pp + K * vi;
-    if (h == 0) wsD[i] = wi;
-    wave_lds_sync();
+    const float wi = pp - 0.5f * tau * kk * vi;
+    dd = __builtin_amdgcn_mfma_f32_32x32x2f32(h == 0 ? vi : wi, h == 0 ? -wi : -vi, dd, 0, 0, 0);
     if (k > 0) {
-        const float tv = tau * vi;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 t = reinterpret_cast<const float4*>(wsB + 16 * h)[q];
-            const float tw[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int c = 4 * q + e;
-                if (!(h == 0 && c == 0)) bk[c] -= tv * tw[e];  // column 0 is the annihilated one
-            }
-        }
+        if (h == 0) bk[0] = (i == 0) ? beta : 0.f;  // the annihilated column
         if (rowok) {
-            float* bq = wr + (NB + ic - 16 * h - 15);
+            float* bq = wr + (NB + ic - 4 * h - 27);
 #pragma unroll
-            for (int c = 0; c < 16; ++c) bq[15 - c] = bk[c];
+            for (int c = 0; c < 16; ++c) bq[27 - sb_col(c, 0)] = bk[c];
         }
     } else if (h == 0 && rowok) {
         wr[ic + 1] = (i == 0) ? beta : 0.f;
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float4 t = reinterpret_cast<const float4*>(wsD + 16 * h)[q];
-        const float tw[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = 4 * q + e, j = 16 * h + c;
-            dd[c] -= vi * tw[e] + wi * vj[c];
-            float* dst = (rowok && j <= i) ? wr + (i - j) : sink;
-            *dst = dd[c];
-        }
+    for (int c = 0; c < 16; ++c) {
+        const int j = sb_col(c, h);
+        float* dst = (rowok && j <= i) ? wr + (i - j) : sink;
+        *dst = dd[c];
     }
     // the reflector as its Q2 block column (48 rows, zero outside [jq, jq +
     // len)): lane r < 48 holds row r
@@ -884,6 +883,7 @@ __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, 
     q2val = (rr >= 0 && rr < NB) ? vv : 0.f;
 #pragma unroll
     for (int c = 0; c < 16; ++c) pv[c] = vj[c];
+    pvi = vi;
     ptau = tau;
     wave_lds_sync();
 }
@@ -958,13 +958,13 @@ __global__ void __launch_bounds__(kSbNT) sb2st_kernel(int n, float* __restrict__
             enter(0, pre, x);
         }
         float4 pf = read(1, pre);
-        float pv[16], ptau = 0.f;
+        float pv[16], pvi = 0.f, ptau = 0.f;
 #pragma unroll
         for (int c = 0; c < 16; ++c) pv[c] = 0.f;
         int dofs[16];
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
-            const int i = lane & 31, j = 16 * (lane >> 5) + c;
+            const int i = lane & 31, j = sb_col(c, lane >> 5);
             dofs[c] = max(i, j) * kSbWP + abs(i - j);
         }
         SbStream my(n);
@@ -984,9 +984,9 @@ __global__ void __launch_bounds__(kSbNT) sb2st_kernel(int n, float* __restrict__
             if (act) {
                 const int off = 32 * my.st - kSbG * my.g;
                 if (s + 1 + (k + 1) * NB <= n)
-                    sb_task<true>(n, s, k, off, win, sc, dofs, pv, ptau, q2val, lane);
+                    sb_task<true>(n, s, k, off, win, sc, dofs, pv, pvi, ptau, q2val, lane);
                 else
-                    sb_task<false>(n, s, k, off, win, sc, dofs, pv, ptau, q2val, lane);
+                    sb_task<false>(n, s, k, off, win, sc, dofs, pv, pvi, ptau, q2val, lane);
             }
             __syncthreads();
             // the rows read ahead are written before this step's stores are
