@@ -772,6 +772,176 @@ tridiag_kernel(int n, int ld, T* __restrict__ Aall, T* __restrict__ dall, T* __r
     }
 }
 
+// Householder tridiagonalisation of matrices of n <= kSmallN, one workgroup per
+// matrix with the matrix in registers: thread (ri, ci) holds the elements of
+// rows ri + 32 a and columns ci + 16 b, both triangles (read from the lower
+// one), so finished rows and columns drop out of every thread's work alike.
+// The columns b < LB of FP64, which would not fit, are in LDS; they are the
+// first to finish.  Same inputs, outputs and factorisation as tridiag_kernel,
+// unblocked (LAPACK sytd2): per column its reflector from the column that its
+// owners put into LDS (every wave forms the norm and the scalars itself), p =
+// A v with the partial sums of a row in one row of 16 lanes, and A -= v w^T + w
+// v^T; two barriers.  Bound by these chains' latency and, at first, by the
+// updates' issue.  SMALLTIMES
+constexpr int kSmallN = 256;
+template <typename T, int AR, int LB, int RB>
+__global__ void __launch_bounds__(kTriNT)
+tridiag_small_kernel(int n, int ld, T* __restrict__ Aall, T* __restrict__ dall, T* __restrict__ eall,
+                     T* __restrict__ tauall) {
+    constexpr int NR = 32 * AR;  // rows held
+    static_assert(kTriNT == 512, "32 x 16 threads");
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* const el = reinterpret_cast<T*>(smem_raw);       // [b][a][thread], b < LB
+    T* const su = el + size_t(LB) * AR * kTriNT;        // column j, two buffers taking turns
+    T* const sp = su + 2 * NR;                          // A v
+    T* const red = sp + NR;                             // kTriNW: v^T A v partials
+    const int b0 = blockIdx.x, tid = threadIdx.x, lane = tid & 63, ri = tid >> 4, ci = tid & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T* const A = Aall + size_t(b0) * n * ld;
+    T* const d = dall + size_t(b0) * n;
+    T* const e = eall + size_t(b0) * n;
+    T* const tau = tauall + size_t(b0) * n;
+    auto elem = [&](int a, int b) -> T {
+        const int r = ri + 32 * a, c = ci + 16 * b;
+        return (r < n && c < n) ? A[size_t(min(r, c)) * ld + max(r, c)] : T(0);
+    };
+    T p[RB][AR];
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int a = 0; a < AR; ++a) p[b][a] = elem(a, LB + b);
+    for (int b = 0; b < LB; ++b)
+#pragma unroll
+        for (int a = 0; a < AR; ++a) el[(b * AR + a) * kTriNT + tid] = elem(a, b);
+    // column j into u, from the lanes that hold it
+    auto publish = [&](int j, T* u) {
+        const int bj = j >> 4;
+        const bool own = ci == (j & 15);
+        if (bj < LB) {
+            if (own)
+#pragma unroll
+                for (int a = 0; a < AR; ++a) u[ri + 32 * a] = el[(bj * AR + a) * kTriNT + tid];
+        } else {
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+                if (b + LB == bj && own)
+#pragma unroll
+                    for (int a = 0; a < AR; ++a) u[ri + 32 * a] = p[b][a];
+        }
+    };
+    __syncthreads();  // A has been read
+    for (int j = 0; j < n - 1; ++j) {
+        T* const u = su + (j & 1) * NR;
+        const int bj = (j + 1) >> 4;  // columns of smaller b are finished
+        publish(j, u);
+        __syncthreads();
+        T sig = T(0);
+#pragma unroll
+        for (int q = 0; q < NR / 64; ++q) {
+            const int i = lane + 64 * q;
+            const T x = u[i];
+            sig += i >= j + 2 ? x * x : T(0);  // (rows past n are zero)
+        }
+        sig = wave_sum(sig);
+        const T alpha = u[j + 1];
+        T tj = T(0), beta = alpha, scal = T(0);
+        if (sig != T(0)) {
+            const T nrm = sqrt(alpha * alpha + sig);
+            beta = (alpha >= T(0)) ? -nrm : nrm;
+            tj = (beta - alpha) / beta;
+            scal = T(1) / (alpha - beta);
+        }
+        auto vat = [&](int i) -> T { return i > j + 1 ? u[i] * scal : (i == j + 1 ? T(1) : T(0)); };
+        if (tid < n && tid < NR) A[size_t(j) * ld + tid] = vat(tid);
+        if (tid == 0) {
+            d[j] = u[j];
+            e[j] = beta;
+            tau[j] = tj;
+        }
+        if (tj == T(0)) continue;
+        const bool low = j < NR / 2 - 1;  // whether any of the first half of the rows is left
+        T va[AR], acc[AR];
+#pragma unroll
+        for (int a = 0; a < AR; ++a) {
+            va[a] = vat(ri + 32 * a);
+            acc[a] = T(0);
+        }
+#pragma unroll
+        for (int b = 0; b < LB + RB; ++b) {
+            if (b < bj) continue;
+            const T vc = vat(ci + 16 * b);
+            if (low)
+#pragma unroll
+                for (int a = 0; a < AR / 2; ++a)
+                    acc[a] += (b < LB ? el[(b * AR + a) * kTriNT + tid] : p[b < LB ? 0 : b - LB][a]) * vc;
+#pragma unroll
+            for (int a = AR / 2; a < AR; ++a)
+                acc[a] += (b < LB ? el[(b * AR + a) * kTriNT + tid] : p[b < LB ? 0 : b - LB][a]) * vc;
+        }
+        T vav = T(0), mine = T(0);
+#pragma unroll
+        for (int a = 0; a < AR; ++a) {
+            acc[a] = row_sum16(acc[a]);
+            vav += va[a] * acc[a];
+            mine = ci == a ? acc[a] : mine;
+        }
+        if (ci < AR) sp[ri + 32 * ci] = mine;
+        vav += __shfl_xor(vav, 16, 64);
+        vav += __shfl_xor(vav, 32, 64);
+        if (lane == 0) red[wave] = vav;
+        __syncthreads();
+        T vAv = T(0);
+#pragma unroll
+        for (int w = 0; w < kTriNW; ++w) vAv += red[w];
+        // w = tau A v + K v, K = -tau (tau v^T A v) / 2, on the rows and columns left
+        const T K = T(-0.5) * tj * tj * vAv;
+        T wa[AR];
+#pragma unroll
+        for (int a = 0; a < AR; ++a) wa[a] = ri + 32 * a > j ? tj * acc[a] + K * va[a] : T(0);
+#pragma unroll
+        for (int b = 0; b < LB + RB; ++b) {
+            if (b < bj) continue;
+            const int c = ci + 16 * b;
+            const T vc = vat(c), wc = c > j ? tj * sp[c] + K * vc : T(0);
+#pragma unroll
+            for (int a = 0; a < AR; ++a) {
+                if (a < AR / 2 && !low) continue;
+                T& x = b < LB ? el[(b * AR + a) * kTriNT + tid] : p[b < LB ? 0 : b - LB][a];
+                x -= va[a] * wc + wa[a] * vc;
+            }
+        }
+    }
+    publish(n - 1, su + ((n - 1) & 1) * NR);
+    __syncthreads();
+    if (tid == 0) {
+        d[n - 1] = su[((n - 1) & 1) * NR + n - 1];
+        e[n - 1] = T(0);
+        tau[n - 1] = T(0);
+        A[size_t(n - 1) * ld + (n - 1)] = T(0);
+    }
+}
+
+template <typename T, int AR, int LB, int RB>
+int tridiag_small_launch(int batch, int n, int ld, T* A, T* d, T* e, T* tau, hipStream_t s) {
+    constexpr size_t sm = (size_t(LB) * AR * kTriNT + 3 * 32 * AR + kTriNW) * sizeof(T);
+    CIR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&tridiag_small_kernel<T, AR, LB, RB>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, int(sm)));
+    hipLaunchKernelGGL((tridiag_small_kernel<T, AR, LB, RB>), dim3(unsigned(batch)), dim3(kTriNT), sm, s, n, ld, A, d, e,
+                       tau);
+    CIR_CHECK_LAUNCH();
+    return CIR_OK;
+}
+
+template <typename T>
+int tridiag_small(int batch, int n, int ld, T* A, T* d, T* e, T* tau, hipStream_t s) {
+    if (n <= 128) return tridiag_small_launch<T, 4, 0, 8>(batch, n, ld, A, d, e, tau, s);
+    if constexpr (sizeof(T) == 4)
+        return tridiag_small_launch<T, 8, 0, 16>(batch, n, ld, A, d, e, tau, s);
+    else  // (12 of the 16 column registers are what FP64 has room for)
+        return n <= 192 ? tridiag_small_launch<T, 8, 0, 12>(batch, n, ld, A, d, e, tau, s)
+                        : tridiag_small_launch<T, 8, 4, 12>(batch, n, ld, A, d, e, tau, s);
+}
+
 // ---------------------------------------------------------------------------
 // Single-matrix tridiagonalisation across the whole GPU (batch == 1: the
 // reference control flow diagonalises one Hamiltonian at a time).  Same
@@ -1600,46 +1770,95 @@ invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ ea
     }
 }
 
-// T factor of a compact-WY block of kb <= kBtNB reflectors from its Gram
-// matrix G = Y^T Y: T(l,l) = tau_l, T(0:l, l) = -tau_l T(0:l, 0:l) G(0:l, l).
-// G and T are kBtNB x kBtNB blocks with row pitch ldt inside per-matrix
-// arrays of bstride elements.  Column l's triangular product takes four
-// lanes per row (each a quarter of the terms, summed by two shuffles), so
-// the longest chain per column is l / 4 products instead of l.
+// T factors of a pass's compact-WY blocks of kBtNB reflectors (blockIdx.y; the
+// pass has kb in all) from its Gram matrix G = Y^T Y: T(l,l) = tau_l, T(0:l, l)
+// = -tau_l T(0:l, 0:l) G(0:l, l).  G and T are blocks with row pitch ldt on the
+// diagonal of per-matrix arrays of bstride elements.
+//
+// The recursion over 128 columns is a chain of 128 products and barriers
+// (150 us for any number of matrices up to a few per CU); here a wave runs it
+// on each of eight 16-column blocks, and blocks are joined pairwise, T = [T1
+// T12; 0 T2] with T12 = -T1 (G12 T2), three times: LARFTTIMES.
+// One LDS array holds G above the diagonal, T in its place as blocks are
+// finished, and the products G12 T2 in the mirror image of T12's place.
+constexpr int kLtB = 16;         // columns of a recursion
+constexpr int kLtP = kBtNB + 1;  // odd pitch: rows and columns without bank conflicts
+constexpr int kLtNT = 4 * kBtNB;
+static_assert(kBtNB == 8 * kLtB && kLtNT == 512, "eight blocks, one per wave, and three joins");
+
+template <int S, typename T>
+__device__ __forceinline__ void larft_join(T* t, int tid) {
+    constexpr int R = S / 8;  // rows per thread: kBtNB / (2 S) pairs of S x S outputs
+    const int d1 = tid / (8 * S) * 2 * S, d2 = d1 + S, j = tid % S, i0 = tid / S % 8 * R;
+    T acc[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = T(0);
+    // G12 T2, T2(k, j) for k <= j
+    for (int k = 0; k <= j; ++k) {
+        const T x = t[(d2 + k) * kLtP + d2 + j];
+#pragma unroll
+        for (int i = 0; i < R; ++i) acc[i] += t[(d1 + i0 + i) * kLtP + d2 + k] * x;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) t[(d2 + i0 + i) * kLtP + d1 + j] = acc[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = T(0);
+    // T12, T1(i, k) for k >= i
+    for (int k = i0; k < S; ++k) {
+        const T x = t[(d2 + k) * kLtP + d1 + j];
+#pragma unroll
+        for (int i = 0; i < R; ++i) acc[i] += (k >= i0 + i ? t[(d1 + i0 + i) * kLtP + d1 + k] : T(0)) * x;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) t[(d1 + i0 + i) * kLtP + d2 + j] = -acc[i];
+    __syncthreads();
+}
+
 template <typename T>
-__global__ void __launch_bounds__(4 * kBtNB)
+__global__ void __launch_bounds__(kLtNT)
 larft_kernel(int n, int kb, int j0, const T* __restrict__ tauall, const T* __restrict__ Gall,
              T* __restrict__ Tall, int ldt, int bstride) {
-    // T is built in LDS, transposed with a padded pitch (Tt[c*kLtP + r] =
-    // T(r, c)): the column step reads a row of T with lanes along r and the
-    // final copy reads it with lanes along c, both without bank conflicts
-    constexpr int kLtP = kBtNB + 1;
     extern __shared__ __align__(16) unsigned char lsm[];
-    T* const Tt = reinterpret_cast<T*>(lsm);
-    T* const col = Tt + kBtNB * kLtP;
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const int row = tid >> 2, part = tid & 3;
-    const T* tau = tauall + size_t(b) * n + j0;
-    const T* G = Gall + size_t(b) * bstride;
-    T* Tm = Tall + size_t(b) * bstride;
-    for (int q = tid; q < kBtNB * kLtP; q += 4 * kBtNB) Tt[q] = T(0);
-    __syncthreads();
-    for (int l = 0; l < kb; ++l) {
-        const T tl = tau[l];
-        if (tid < l) col[tid] = -tl * G[tid * ldt + l];
-        __syncthreads();
-        T acc = T(0);
-        if (row < l)
-            for (int q = row + part; q < l; q += 4) acc += Tt[q * kLtP + row] * col[q];
-        acc += __shfl_xor(acc, 1, 64);
-        acc += __shfl_xor(acc, 2, 64);
-        if (row < l && part == 0) Tt[l * kLtP + row] = acc;
-        if (tid == 0) Tt[l * kLtP + l] = tl;
-        __syncthreads();
-    }
-    for (int q = tid; q < kBtNB * kBtNB; q += 4 * kBtNB) {
+    T* const t = reinterpret_cast<T*>(lsm);
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, first = blockIdx.y * kBtNB;
+    const int kn = min(kBtNB, kb - first);  // reflectors of this block; past them tau = 0 and G = 0
+    const T* tau = tauall + size_t(b) * n + j0 + first;
+    const T* G = Gall + size_t(b) * bstride + size_t(first) * (ldt + 1);
+    T* Tm = Tall + size_t(b) * bstride + size_t(first) * (ldt + 1);
+#pragma unroll 8
+    for (int q = tid; q < kBtNB * kBtNB; q += kLtNT) {
         const int r = q / kBtNB, c = q % kBtNB;
-        Tm[r * ldt + c] = Tt[c * kLtP + r];
+        t[r * kLtP + c] = (r < c && c < kn) ? G[r * ldt + c] : T(0);
+    }
+    const int d0 = tid / 64 * kLtB, row = lane & (kLtB - 1);
+    T tl[kLtB];
+#pragma unroll
+    for (int l = 0; l < kLtB; ++l) tl[l] = (d0 + l < kn) ? tau[d0 + l] : T(0);
+    __syncthreads();
+    {
+        // lane r (of each 16) the row r of T
+        T Tr[kLtB];
+#pragma unroll
+        for (int l = 0; l < kLtB; ++l) {
+            T acc = T(0);
+#pragma unroll
+            for (int q = 0; q < l; ++q) acc += Tr[q] * t[(d0 + q) * kLtP + d0 + l];
+            Tr[l] = (row == l) ? tl[l] : (row < l ? -tl[l] * acc : T(0));
+        }
+        wave_lds_sync();
+        if (lane < kLtB)
+#pragma unroll
+            for (int l = 0; l < kLtB; ++l)
+                if (row <= l) t[(d0 + row) * kLtP + d0 + l] = Tr[l];
+    }
+    __syncthreads();
+    larft_join<16>(t, tid);
+    larft_join<32>(t, tid);
+    larft_join<64>(t, tid);
+    for (int q = tid; q < kBtNB * kBtNB; q += kLtNT) {
+        const int r = q / kBtNB, c = q % kBtNB;
+        Tm[r * ldt + c] = r <= c ? t[r * kLtP + c] : T(0);
     }
 }
 
@@ -1667,24 +1886,25 @@ yt_kernel(int n, int ld, int j0, int off, int kb, int mrows, const T* __restrict
     }
 }
 
-inline size_t larft_smem_bytes(size_t esz) { return (size_t(kBtNB) * (kBtNB + 1) + kBtNB) * esz; }
+inline size_t larft_smem_bytes(size_t esz) { return size_t(kBtNB) * kLtP * esz; }
 
 // How a batch is reduced to tridiagonal form:
-//   two stages (k_band.hip)   FP32 up to sb_max_n(), from kTwoStageMinN on
+//   one stage, in registers   n <= kSmallN, one workgroup per matrix
+//   two stages (k_band.hip)   FP32 from there to sb_max_n()
 //   one stage, whole GPU      a few matrices, one at a time, a grid per step
 //   one stage, batched        one workgroup per matrix
-// The lines, from both sides measured (ms per batch): two stages against one
-// workgroup per matrix, 64 matrices, n = 320 5.1 / 4.6, n = 400 7.0 / 6.8, n =
-// 512 9.5 / 10.7, n = 640 13.4 / 17.1, 24 of n = 1000 23.8 / 43, 32 of n = 2100
-// 84 / 277, 24 of n = 3072 168 / 741; against the
-// whole-GPU form, one matrix of n = 512 8.8 / 13.8, n = 1024 22.6 / 30.7, n =
-// 2048 66.5 / 73.5, 8 of n = 512 8.9 / 104.  The whole-GPU form takes a time
+// The lines, from both sides measured (ms per batch): two stages against
+// registers, 64 matrices of n = 256 2.3 / 1.9 (FP32, with the corrections
+// below); against one workgroup per matrix without them, 64 of n = 300 3.1 /
+// 3.9, one 2.6 / 3.7, 64 of n = 384 4.1 / 5.9, 48 of n = 448 4.8 / 7.8, 64 of n
+// = 640 8.9 / 16.5, 32 of n = 2100 84 / 277, 24 of n = 3072 168 / 741; against
+// the whole-GPU form, one matrix of n = 512 8.8 / 13.8, n = 1024 22.6 / 30.7, n
+// = 2048 41 / 73.5, 8 of n = 512 8.9 / 104.  The whole-GPU form takes a time
 // that grows with the batch (n = 1024 in FP64: 27 per matrix), the batched form
 // one that does not up to a matrix per CU (76), and the ratio of the two grows
 // with n: the whole-GPU form runs batches of up to n / kSinglePer matrices.
 // CIR_EIGH_STAGES=1 or 2 in the environment forces one or two stages where
 // both apply (tests compare them).
-constexpr int kTwoStageMinN = 448;
 inline bool use_two_stage(size_t esz, int n) {
     if (esz != sizeof(float) || n > sb_max_n() || n < 2 * kBandNB + 2) return false;
     if (deterministic_mode()) return true;  // the form without float atomics
@@ -1692,7 +1912,7 @@ inline bool use_two_stage(size_t esz, int n) {
     const int forced = fv ? std::atoi(fv) : 0;
     if (forced == 1) return false;
     if (forced == 2) return true;
-    return n >= kTwoStageMinN;
+    return n > kSmallN;
 }
 inline bool use_whole_gpu(int batch, int n) {
     return n >= kSingleMinN && batch <= kSingleMaxBatch && int64_t(batch) * kSinglePer <= n;
@@ -1701,7 +1921,9 @@ inline bool use_whole_gpu(int batch, int n) {
 // The two-stage form's T carries the rounding of N bulge-chasing sweeps over
 // every element of the band: in FP32 about three times the one-stage form's
 // backward error (2048-OH Hamiltonians: eigenvalues 6.5e-7 against 2.1e-7 of
-// the spectrum, spectral density 1.7e-6 against 4e-7).  Where the reduction is
+// the spectrum, spectral density 1.7e-6 against 4e-7), and that of the unblocked
+// reduction in registers the rounding of N rank-two updates (N = 256: 2.2e-7
+// against 1.3e-7 by panels).  Where the reduction is
 // bound by its chains rather than by its arithmetic (small matrices, small
 // batches) three N^3 products cost little, and the eigenpairs get one step of
 // first-order correction from a copy of H: with the residuals C = H V - V L
@@ -1717,7 +1939,10 @@ inline bool use_whole_gpu(int batch, int n) {
 // n = 766: 1.7 of 13; 24 of n = 3072: 30 of 168.  Above kRefineAboveN, where
 // only the one-stage form used to run, it is always made.
 constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16, kRefineAboveN = 2080;
-inline bool use_refine(int batch, int n) { return n < kRefineMaxN || batch <= kRefineMaxBatch || n > kRefineAboveN; }
+inline bool use_refine(size_t esz, bool two, int batch, int n) {
+    if (esz != sizeof(float) || !(two || n <= kSmallN)) return false;
+    return n < kRefineMaxN || batch <= kRefineMaxBatch || n > kRefineAboveN;
+}
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
 constexpr int kRqRun = 128;          // rows summed in one MFMA chain
@@ -1879,15 +2104,32 @@ add_rows_kernel(int n, int ld, const float* __restrict__ Pall, const float* __re
     Vall[o] = (Vall[o] + Pall[o]) * dlall[size_t(blockIdx.z) * n + j];
 }
 
-// The matrices' copy for the refinement
+// The matrices' copy for the correction, both triangles from the one that the
+// reductions read (row-major, column >= row): one workgroup per 32 x 32 tile
+// on or above the diagonal and its mirror image.
 __global__ void __launch_bounds__(256)
-copy4_kernel(int64_t cnt, const float4* __restrict__ src, float4* __restrict__ dst) {
-    for (int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x; q < cnt; q += int64_t(gridDim.x) * 256) dst[q] = src[q];
+mirror_copy_kernel(int n, int ld, const float* __restrict__ Aall, float* __restrict__ Hall) {
+    __shared__ float t[kRotT][kRotT + 1];
+    const int I = blockIdx.y * kRotT, J = blockIdx.x * kRotT;
+    if (I > J) return;
+    const float* A = Aall + size_t(blockIdx.z) * n * ld;
+    float* H = Hall + size_t(blockIdx.z) * n * ld;
+    const int c = threadIdx.x % kRotT, r0 = threadIdx.x / kRotT;
+#pragma unroll
+    for (int r = r0; r < kRotT; r += 256 / kRotT)
+        if (I + r <= J + c && J + c < n) t[r][c] = A[size_t(I + r) * ld + J + c];
+    __syncthreads();
+#pragma unroll
+    for (int r = r0; r < kRotT; r += 256 / kRotT) {
+        if (I + r < n && J + c < n && I + r <= J + c) H[size_t(I + r) * ld + J + c] = t[r][c];
+        if (J + r < n && I + c < n && I + c <= J + r) H[size_t(J + r) * ld + I + c] = t[c][r];
+    }
 }
 
 struct EighWork {
     size_t off_d, off_e, off_tau, off_vw, off_g, off_t, off_w1, off_w2, off_s1, off_scr, total;
-    size_t off_bnd, off_p1, off_yh, off_q2, off_h, off_r;  // two-stage buffers
+    size_t off_bnd, off_p1, off_yh, off_q2;  // two-stage buffers
+    size_t off_h, off_r;                     // the correction's
     bool two, refine;
     int sub;  // matrices per inverse-iteration pass
 };
@@ -1906,11 +2148,13 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
         o = al(o + esz * batch * size_t(n) * kBandNB);
         L.off_q2 = o;
         o = al(o + esz * batch * size_t(q2_blocks(n)) * kQ2BlockFloats);
-        L.refine = use_refine(batch, n);
+    }
+    L.refine = use_refine(esz, L.two, batch, n);
+    if (L.refine) {
         L.off_h = o;
-        if (L.refine) o = al(o + esz * batch * size_t(n) * ld);
+        o = al(o + esz * batch * size_t(n) * ld);
         L.off_r = o;
-        if (L.refine) o = al(o + esz * batch * size_t(n) * ld);
+        o = al(o + esz * batch * size_t(n) * ld);
     }
     L.off_d = o;
     o = al(o + esz * batch * n);
@@ -1959,18 +2203,18 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
     // across the whole GPU
     if (ld % 4 != 0) return fail(CIR_ERR_ARG, "eigh: the leading dimension must be a multiple of 4");
     if constexpr (sizeof(T) == sizeof(float)) {
+        if (L.refine) {
+            ProfScope ps(prof, CIR_PH_TRIDIAG, s);
+            const unsigned nr = unsigned(ceil_div(n, kRotT));
+            hipLaunchKernelGGL(mirror_copy_kernel, dim3(nr, nr, unsigned(batch)), dim3(256), 0, s, n, ld,
+                               reinterpret_cast<const float*>(A), reinterpret_cast<float*>(work + L.off_h));
+            CIR_CHECK_LAUNCH();
+        }
         if (L.two) {
             float* bnd = reinterpret_cast<float*>(work + L.off_bnd);
             float* q2 = reinterpret_cast<float*>(work + L.off_q2);
             {
                 ProfScope ps(prof, CIR_PH_TRIDIAG, s);
-                if (L.refine) {
-                    const int64_t cnt = int64_t(batch) * n * ld / 4;
-                    hipLaunchKernelGGL(copy4_kernel, dim3(unsigned(std::min<int64_t>(ceil_div(cnt, 256), 8192))), dim3(256),
-                                       0, s, cnt, reinterpret_cast<const float4*>(A),
-                                       reinterpret_cast<float4*>(work + L.off_h));
-                    CIR_CHECK_LAUNCH();
-                }
                 CIR_TRY(sy2sb(batch, n, ld, A, bnd, tau, reinterpret_cast<float*>(work + L.off_p1),
                               reinterpret_cast<float*>(work + L.off_yh), s));
             }
@@ -1986,6 +2230,9 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
         for (int b = 0; b < batch; ++b)
             CIR_TRY(tridiag_single<T>(n, ld, A + size_t(b) * n * ld, dd + size_t(b) * n, ee + size_t(b) * n,
                                       tau + size_t(b) * n, vw + size_t(b) * 2 * kTriNB * ld, s1, s));
+    } else if (n <= kSmallN) {
+        ProfScope ps(prof, CIR_PH_TRIDIAG, s);
+        CIR_TRY(tridiag_small<T>(batch, n, ld, A, dd, ee, tau, s));
     } else {
         const int rl = tridiag_panel_rows<T>(n);
         const size_t sm = (tridiag_smem_elems<T>(n) + size_t(rl) * 2 * kTriNB) * sizeof(T);
@@ -2082,13 +2329,10 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
         CIR_TRY(mm(kb, kb, mrows, Y, ld, 1, mat, Y, 1, ld, mat, G, P, 1, pp, 1.0, 0.0));
         // T1, T2 from the diagonal blocks of G; T12 = -T1 (G12 T2), with
         // G12 T2 staged in W2
-        hipLaunchKernelGGL(larft_kernel<T>, dim3(batch), dim3(4 * kBtNB), larft_smem_bytes(sizeof(T)), s, n, kb1, j0, tau,
-                           G, Tm, P, int(pp));
+        hipLaunchKernelGGL(larft_kernel<T>, dim3(batch, kb2 > 0 ? 2 : 1), dim3(kLtNT), larft_smem_bytes(sizeof(T)), s, n,
+                           kb, j0, tau, G, Tm, P, int(pp));
         CIR_CHECK_LAUNCH();
         if (kb2 > 0) {
-            hipLaunchKernelGGL(larft_kernel<T>, dim3(batch), dim3(4 * kBtNB), larft_smem_bytes(sizeof(T)), s, n, kb2,
-                               j0 + kb1, tau, G + int64_t(kb1) * P + kb1, Tm + int64_t(kb1) * P + kb1, P, int(pp));
-            CIR_CHECK_LAUNCH();
             CIR_TRY(mm(kb1, kb2, kb2, G + kb1, P, 1, pp, Tm + int64_t(kb1) * P + kb1, P, 1, pp, W2, P, 1, pn, 1.0,
                        0.0));
             CIR_TRY(mm(kb1, kb2, kb1, Tm, P, 1, pp, W2, P, 1, pn, Tm + kb1, P, 1, pp, -1.0, 0.0));

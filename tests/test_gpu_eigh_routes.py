@@ -36,6 +36,8 @@ def test_corrected_two_stage_eigenpairs(n, batch, prec):
     ld = (n + 3) // 4 * 4 + 4
     Hd = np.zeros((batch, n, ld), np.float32)
     Hd[:, :, :n] = H
+    for b in range(batch):  # the triangle below the diagonal is not read
+        Hd[b, :, :n][np.tril_indices(n, -1)] = 5.0e3
     w, V = S.eigh(torch.from_numpy(Hd).to(DEV), n, prec=prec)
     w, V = w.cpu().numpy(), V.cpu().double().numpy()[:, :, :n]
     eps = 6e-8
