@@ -421,6 +421,7 @@ int forward_impl(cir_ctx* c, int nframes, const float* xyz_d, const float* box_d
     const size_t eig_all = size_t(nu) * (size_t(N) * ld * esz + size_t(N) * 8);
     size_t fr = 0, tot = 0;
     CIR_HIP(hipMemGetInfo(&fr, &tot));
+    fr += dev_cache_bytes();
     const bool fits = double(base + eig_all) <= 0.8 * double(fr);
     if (p.adj_store == 1 && !fits)
         return fail(CIR_ERR_NOMEM, "forward_ls: the eigensystems of all frames do not fit in device memory");
@@ -690,6 +691,7 @@ extern "C" int cir_forward_ls(cir_ctx* c, int nframes, const float* xyz, const f
                               double* ftcf_ir) try {
     if (!c || !xyz || !box || !times || !ftcf_ir || nframes <= 0)
         return fail(CIR_ERR_ARG, "cir_forward_ls: bad arguments");
+    KeepScope keep(c->stream);
     if (c->p.adj_store < 0 || c->p.adj_store > 2) return fail(CIR_ERR_ARG, "adjoint_store must be 0, 1 or 2");
     if (c->p.reunit_every > 0)
         return fail(CIR_ERR_ARG, "the lineshape adjoint propagates without re-unitarisation: set reunitarise_every 0");
@@ -713,6 +715,7 @@ extern "C" int cir_forward_ls(cir_ctx* c, int nframes, const float* xyz, const f
 
 extern "C" int cir_backward_ls(cir_ctx* c, const double* dL_dftcf_ir, double* dL_dcoef) try {
     if (!c || !dL_dftcf_ir || !dL_dcoef) return fail(CIR_ERR_ARG, "cir_backward_ls: bad arguments");
+    KeepScope keep(c->stream);
     if (!c->adj || !c->adj->have) return fail(CIR_ERR_ARG, "cir_backward_ls: call cir_forward_ls first");
     if (c->real_prec == CIR_PREC_FP64) return backward_impl<double>(c, dL_dftcf_ir, dL_dcoef);
     return backward_impl<float>(c, dL_dftcf_ir, dL_dcoef);

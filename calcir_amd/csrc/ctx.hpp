@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "dev_cache.hpp"
 
 namespace cir {
 
@@ -21,11 +22,27 @@ struct PoolStream {
 };
 inline thread_local const PoolStream* tl_pool = nullptr;
 
+// While a thread is in a KeepScope, the buffers that it takes (outside a
+// PoolStream) come from the memory kept between runs (dev_cache.hpp) and go
+// back to it once the work queued on the scope's stream, the only one that
+// uses them, is done.
+inline thread_local const hipStream_t* tl_keep = nullptr;
+struct KeepScope {
+    const hipStream_t s;
+    const hipStream_t* const prev;
+    explicit KeepScope(hipStream_t stream) : s(stream), prev(tl_keep) { tl_keep = &s; }
+    ~KeepScope() { tl_keep = prev; }
+    KeepScope(const KeepScope&) = delete;
+    KeepScope& operator=(const KeepScope&) = delete;
+};
+
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
-    hipStream_t fs = nullptr;  // stream a pooled buffer is freed on
-    bool pooled = false;
+    size_t cap = 0;            // a kept buffer's block and its device
+    int dev = 0;
+    hipStream_t fs = nullptr;  // stream a pooled or kept buffer is freed on
+    bool pooled = false, kept = false;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
@@ -34,19 +51,23 @@ struct DevBuf {
         if (p) {
             if (pooled)
                 (void)hipFreeAsync(p, fs);
+            else if (kept && hipStreamSynchronize(fs) == hipSuccess)
+                dev_cache_free(p, cap, dev);
             else
                 (void)hipFree(p);
         }
         p = nullptr;
-        bytes = 0;
+        bytes = cap = 0;
         fs = nullptr;
-        pooled = false;
+        pooled = kept = false;
     }
     int alloc(size_t n) {
         release();
         if (n == 0) n = 256;
         const PoolStream* ps = tl_pool;
-        const hipError_t e = ps ? hipMallocFromPoolAsync(&p, n, ps->pool, ps->stream) : hipMalloc(&p, n);
+        const hipError_t e = ps ? hipMallocFromPoolAsync(&p, n, ps->pool, ps->stream)
+                             : tl_keep ? hipError_t(dev_cache_alloc(&p, n, &cap, &dev))
+                                       : hipMalloc(&p, n);
         if (e != hipSuccess) {
             p = nullptr;
             return hip_fail(e, ps ? "hipMallocFromPoolAsync" : "hipMalloc", __FILE__, __LINE__);
@@ -55,6 +76,9 @@ struct DevBuf {
         if (ps) {
             pooled = true;
             fs = ps->stream;
+        } else if (tl_keep) {
+            kept = true;
+            fs = *tl_keep;
         }
         return CIR_OK;
     }

@@ -268,7 +268,7 @@ int auto_chunk(const cir_ctx* c, int nuniq) {
     auto need = [&](int B) { return double(B) * hv + double(eigh_workspace(c->real_prec, B, c->N, c->ld)); };
     size_t fr = 0, tot = 0;
     double budget = 24.0 * (1 << 30);
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess) budget = std::max(budget, 0.5 * double(fr));
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess) budget = std::max(budget, 0.5 * double(fr + dev_cache_bytes()));
     budget /= std::max(1, c->mem_share);
     int B = std::max(1, std::min(512, nuniq));
     while (B > 1 && need(B) > budget) B = std::max(1, std::min(B - 1, int(double(B) * budget / need(B))));
@@ -932,6 +932,7 @@ void reset_phases(cir_ctx* c) {
 
 extern "C" int cir_run_device(cir_ctx* c, int nframes, const float* xyz_d, const float* box_d, const float* times) try {
     if (!c || !xyz_d || !box_d || !times || nframes <= 0) return fail(CIR_ERR_ARG, "cir_run_device: bad arguments");
+    KeepScope keep(c->stream);
     {
         // the boxes are few bytes: check them on the host
         std::vector<float> hb(size_t(nframes) * box_floats(c));
@@ -959,6 +960,7 @@ extern "C" int cir_run_device(cir_ctx* c, int nframes, const float* xyz_d, const
 
 extern "C" int cir_stream_begin(cir_ctx* c, int nframes, const float* times) try {
     if (!c || !times || nframes <= 0) return fail(CIR_ERR_ARG, "cir_stream_begin: bad arguments");
+    KeepScope keep(c->stream);
     c->streamed.reset();
     if (c->p.mode == CIR_MODE_PLAIN) return fail(CIR_ERR_ARG, "cir_stream_begin: streaming needs mode batched");
     if (c->p.ckpt_every > 0 || c->p.resume != 0 || c->p.max_frames > 0)
@@ -1023,6 +1025,7 @@ int stream_push(cir_ctx* c, int first, int count, const float* xyz, const float*
 
 extern "C" int cir_stream_push(cir_ctx* c, int first, int count, const float* xyz, const float* box) try {
     if (!c) return fail(CIR_ERR_ARG, "cir_stream_push: null context");
+    KeepScope keep(c->stream);
     const int st = stream_push(c, first, count, xyz, box);
     if (st != CIR_OK) c->streamed.reset();  // a failed push closes the stream
     return st;
@@ -1033,6 +1036,7 @@ extern "C" int cir_stream_push(cir_ctx* c, int first, int count, const float* xy
 
 extern "C" int cir_stream_end(cir_ctx* c) try {
     if (!c) return fail(CIR_ERR_ARG, "cir_stream_end: null context");
+    KeepScope keep(c->stream);
     std::unique_ptr<StreamRun, StreamDeleter> s = std::move(c->streamed);
     if (!s) return fail(CIR_ERR_ARG, "cir_stream_end: no stream is open (cir_stream_begin)");
     if (s->c0 < s->run.nu)
@@ -1080,6 +1084,7 @@ extern "C" int cir_phase_times(cir_ctx* c, double* seconds, long long* groups, i
 
 extern "C" int cir_run(cir_ctx* c, int nframes, const float* xyz, const float* box, const float* times) try {
     if (!c || !xyz || !box || !times || nframes <= 0) return fail(CIR_ERR_ARG, "cir_run: bad arguments");
+    KeepScope keep(c->stream);
     const size_t nx = size_t(nframes) * c->natoms * 3;
     for (size_t i = 0; i < nx; ++i)
         if (!std::isfinite(xyz[i])) return fail(CIR_ERR_NONFINITE, "non-finite coordinate in the trajectory");
@@ -1195,6 +1200,7 @@ extern "C" int cir_run_many(int njob, cir_ctx* const* ctxs, const int* nframes, 
         (void)hipMemPoolTrimTo(pool, 0);
         (void)hipGetLastError();
     }
+    dev_cache_release();
     for (int j = 0; j < njob; ++j) {
         ctxs[j]->stream = saved[j];
         ctxs[j]->mem_share = saved_share[j];
