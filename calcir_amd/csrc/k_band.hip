@@ -320,27 +320,33 @@ __device__ __forceinline__ bool xcd_slot(int gx, int batch, int& x, int& b) {
 }
 inline dim3 xcd_grid(int gx, int batch) { return dim3(unsigned(ceil_div(int64_t(gx) * batch, int64_t(kXcds)) * kXcds)); }
 
+constexpr int kSyWaves = 4;  // waves per block row of the trailing matrix
+
 // X = A22 Yh on the lower triangle of A22 (m x m, column-major, pitch ld,
 // first row and column r0), X row-major with pitch 2 NB in the W half of the
 // row-major panel P (rows r0.., P[r * 2NB + NB + p]); Yh row-major, pitch NB
-// (panel rows).  Wave w of workgroup x owns block row I = 4 x + w and reads
-// every tile once from its own side: the row tiles (I, J < I) go straight
-// into the MFMA A operand (lanes along rows, coalesced), the column tiles
-// (J >= I, I) are read along their rows too and transposed through the
-// wave's LDS tile.  The next tile's loads are in flight while a tile's MFMA
-// chain runs.  32x32x2 FP32 MFMA, K = 32 per tile.
-__global__ void __launch_bounds__(256) sb_symm_kernel(int n, int ld, int r0, const float* __restrict__ Aall,
+// (panel rows).  Workgroup x owns block row I = x, wave w its tiles J = w, w +
+// WV, ..., summed in wave order at the end.  Every tile is read from its own
+// side: the row tiles (I, J < I) go straight into the MFMA A operand (lanes
+// along rows, coalesced), the column tiles (J >= I, I) are read along their
+// rows too and transposed through the wave's LDS tile.  The next tile's loads
+// are in flight while a tile's MFMA chain runs.  32x32x2 FP32 MFMA, K = 32 per
+// tile.  Bound by latency where there are few matrices, by memory (4 TB/s) where
+// there are many.  With a block row per wave, up to nbt tiles one after the
+// other: 63 calls for one matrix of N = 2048 2.78 ms, 128 matrices 12.6, 48 of N
+// = 768 0.52; with 4 waves to a row 0.90, 11.4, 0.37; with 8 0.77 for the one
+// matrix, but 0.45 for the 48 (the sums cost more than the shorter chains give).
+__global__ void __launch_bounds__(64 * kSyWaves) sb_symm_kernel(int n, int ld, int r0, const float* __restrict__ Aall,
                                                       const float* __restrict__ Yhall, float* __restrict__ Pall,
                                                       int batch) {
-    constexpr int NB = kBandNB;
-    __shared__ float tl[4][32][33];
+    constexpr int NB = kBandNB, WV = kSyWaves;
+    __shared__ float tl[WV][32][33];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = n - r0, nbt = (m + 31) / 32;
     int x, b;
-    if (!xcd_slot((nbt + 3) / 4, batch, x, b)) return;
-    const int I = x * 4 + wave;
-    if (I >= nbt) return;
+    if (!xcd_slot(nbt, batch, x, b)) return;
+    const int I = x;
     const float* A = Aall + size_t(b) * n * ld + size_t(r0) * ld + r0;
     const float* Yh = Yhall + size_t(b) * n * NB;
     float* P = Pall + size_t(b) * n * 2 * NB + size_t(r0) * 2 * NB;
@@ -369,11 +375,11 @@ __global__ void __launch_bounds__(256) sb_symm_kernel(int n, int ld, int r0, con
     floatx16 acc;
 #pragma unroll
     for (int q = 0; q < 16; ++q) acc[q] = 0.f;
-    // tile J from (bv, raw) while tile J + 1 is read into (bn, rn) (past the
+    // tile J from (bv, raw) while the next one is read into (bn, rn) (past the
     // last tile: clamped reads, never used); the two buffer pairs alternate,
     // so no copy waits for a read in flight
     auto tile = [&](int J, float (&bv)[16], float (&raw)[16], float (&bn)[16], float (&rn)[16]) {
-        load(J + 1, bn, rn);
+        load(J + WV, bn, rn);
         __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the products
 #pragma unroll
         for (int q = 0; q < 16; ++q) bv[q] = (J * 32 + 2 * q + h < m) ? bv[q] : 0.f;
@@ -398,17 +404,23 @@ __global__ void __launch_bounds__(256) sb_symm_kernel(int n, int ld, int r0, con
         for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[q], bv[q], acc, 0, 0, 0);
     };
     float b0[16], r0v[16], b1[16], r1v[16];
-    load(0, b0, r0v);
-    for (int J = 0; J < nbt; J += 2) {
+    load(wave, b0, r0v);
+    for (int J = wave; J < nbt; J += 2 * WV) {
         tile(J, b0, r0v, b1, r1v);
-        if (J + 1 >= nbt) break;
-        tile(J + 1, b1, r1v, b0, r0v);
+        if (J + WV >= nbt) break;
+        tile(J + WV, b1, r1v, b0, r0v);
     }
     // acc(i, p): lane l holds column p = l32, rows 8 a + 4 h + c
+    wave_lds_sync();
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int r = I * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-        if (r < m) P[size_t(r) * 2 * NB + NB + l32] = acc[q];
+    for (int q = 0; q < 16; ++q) T[8 * (q >> 2) + 4 * h + (q & 3)][l32] = acc[q];
+    __syncthreads();
+    for (int e = tid; e < 32 * 32; e += 64 * WV) {
+        const int i = e / 32, p = e % 32, r = I * 32 + i;
+        float t = tl[0][i][p];
+#pragma unroll
+        for (int w = 1; w < WV; ++w) t += tl[w][i][p];
+        if (r < m) P[size_t(r) * 2 * NB + NB + p] = t;
     }
 }
 
@@ -500,25 +512,29 @@ __global__ void __launch_bounds__(kPanNT) sb_w_kernel(int n, int r0, const float
 constexpr int kBufferWord3 = 0x00020000;
 
 // A22 -= W Y^T + Y W^T on the lower triangle, from the row-major panel P
-// (P[r * 2NB + k]: Y(r, k) for k < NB, W(r, k - NB) after).  Wave w of
-// workgroup x owns block row br = 4 x + w and every block column bc <= br.
+// (P[r * 2NB + k]: Y(r, k) for k < NB, W(r, k - NB) after).  Workgroup x owns
+// block row br = x, wave w its block columns bc = w, w + 4, ... <= br.
 // The tile is formed transposed (MFMA row = column of A, MFMA column = row
 // of A) so that lanes run along rows of the column-major A; step s of the
 // K = 2NB sum takes panel position 32 h + s from lane half h, the A operand
 // from the panel row of the tile's column at that position, the B operand
 // from the panel row of the tile's row at the swapped half (k ^ NB).  The
 // next tile's A values and operand are in flight while a tile's MFMA chain
-// runs.
-__global__ void __launch_bounds__(256) sb_syr2k_kernel(int n, int ld, int r0, float* __restrict__ Aall,
+// runs.  Bound by
+// memory (each element of A22 read and written, 3.3 TB/s) where there are many
+// matrices.  With a block row per wave 63 calls for one matrix of N = 2048 took
+// 3.48 ms, 24 matrices of N = 3072 12.6, 48 of N = 768 0.62; with 4 waves to a row
+// 1.20, 10.0, 0.50.
+__global__ void __launch_bounds__(64 * kSyWaves) sb_syr2k_kernel(int n, int ld, int r0, float* __restrict__ Aall,
                                                        const float* __restrict__ Pall, int batch) {
-    constexpr int NB = kBandNB, PW = 2 * kBandNB;
+    constexpr int NB = kBandNB, PW = 2 * kBandNB, WV = kSyWaves;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = n - r0, nbt = (m + 31) / 32;
     int x, b;
-    if (!xcd_slot((nbt + 3) / 4, batch, x, b)) return;
-    const int br = x * 4 + wave;
-    if (br >= nbt) return;
+    if (!xcd_slot(nbt, batch, x, b)) return;
+    const int br = x;
+    if (br >= nbt || wave > br) return;
     float* A = Aall + size_t(b) * n * ld + size_t(r0) * ld + r0;
     const float* P = Pall + size_t(b) * n * PW + size_t(r0) * PW;
     const int h = lane >> 5, l32 = lane & 31;
@@ -549,12 +565,12 @@ __global__ void __launch_bounds__(256) sb_syr2k_kernel(int n, int ld, int r0, fl
     };
     float bv[32];
     panel_row(r, 1 - h, bv);
-    // tile bc from (av, old) while tile bc + 1's operand and old values are
+    // tile bc from (av, old) while the next tile's operand and old values are
     // read into (an, on) (past the last tile: clamped reads, never used); the
     // two buffer pairs alternate, so no copy waits for a read in flight
     auto tile = [&](int bc, float (&av)[32], float (&old)[16], float (&an)[32], float (&on)[16]) {
-        panel_row((bc + 1) * 32 + l32, h, an);
-        load_old(bc + 1, on);
+        panel_row((bc + WV) * 32 + l32, h, an);
+        load_old(bc + WV, on);
         __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the products
         floatx16 acc;
 #pragma unroll
@@ -574,12 +590,12 @@ __global__ void __launch_bounds__(256) sb_syr2k_kernel(int n, int ld, int r0, fl
         }
     };
     float a0[32], o0[16], a1[32], o1[16];
-    panel_row(l32, h, a0);
-    load_old(0, o0);
-    for (int bc = 0; bc <= br; bc += 2) {
+    panel_row(wave * 32 + l32, h, a0);
+    load_old(wave, o0);
+    for (int bc = wave; bc <= br; bc += 2 * WV) {
         tile(bc, a0, o0, a1, o1);
-        if (bc + 1 > br) break;
-        tile(bc + 1, a1, o1, a0, o0);
+        if (bc + WV > br) break;
+        tile(bc + WV, a1, o1, a0, o0);
     }
 }
 
@@ -628,15 +644,17 @@ int sy2sb(int batch, int n, int ld, float* A, float* BND, float* tau, float* P, 
         }
         CIR_CHECK_LAUNCH();
         const int nbt = int(ceil_div(m, 32));
-        const dim3 grid = xcd_grid(int(ceil_div(nbt, 4)), batch);
+        const dim3 grid = xcd_grid(nbt, batch);
         // X = A22 Yh into the W half of P
-        hipLaunchKernelGGL(sb_symm_kernel, grid, dim3(256), 0, s, n, ld, r0, A, Yh, P, batch);
+        hipLaunchKernelGGL(sb_symm_kernel, grid, dim3(64 * kSyWaves), 0, s, n, ld, r0, A,
+                           Yh, P, batch);
         CIR_CHECK_LAUNCH();
         // W = X - Y (Yh^T X) / 2 in place of X
         hipLaunchKernelGGL(sb_w_kernel, dim3(unsigned(batch)), dim3(kPanNT), 0, s, n, r0, Yh, P);
         CIR_CHECK_LAUNCH();
         // A22 -= W Y^T + Y W^T (lower triangle)
-        hipLaunchKernelGGL(sb_syr2k_kernel, grid, dim3(256), 0, s, n, ld, r0, A, P, batch);
+        hipLaunchKernelGGL(sb_syr2k_kernel, grid, dim3(64 * kSyWaves), 0, s, n, ld, r0, A, P,
+                           batch);
         CIR_CHECK_LAUNCH();
     }
     // the last diagonal block (n - j0 <= NB + 1 rows) is already banded
