@@ -218,6 +218,18 @@ adj_gmu_kernel(int N, int m, const int* __restrict__ trip, const double* __restr
     for (int a = 0; a < 3; ++a) gmu[size_t(a) * N + i] = g[a];
 }
 
+// Rows [fr | fi] of phi: [fi | fr] into out, [fr | -fi] in place.
+template <typename T>
+__global__ void __launch_bounds__(kAdjNT) adj_turn_kernel(int n, int w3, T* __restrict__ phi, T* __restrict__ out) {
+    const int64_t e = int64_t(blockIdx.x) * kAdjNT + threadIdx.x;
+    if (e >= int64_t(n) * w3) return;
+    const size_t o = size_t(e / w3) * 2 * w3 + size_t(e % w3);
+    const T fr = phi[o], fi = phi[o + w3];
+    out[o] = fi;
+    out[o + w3] = fr;
+    phi[o + w3] = -fi;
+}
+
 // R = Re(D o (P + P^T)) with P = Pr + i Pi (row-major, ld), tiles of 32x32
 // staged through LDS for the transposed reads.
 template <typename T>
@@ -602,16 +614,22 @@ int backward_impl(cir_ctx* c, const double* dL_dy, double* grad) {
             }
             CIR_TRY(pack_any(rp, true, N, np, trip + 3 * p0, 1, A->fv.p, Fp.p, st));
             // beta = V^T b, phi = V^T f (V(i,k) at V[i*ld+k])
-            CIR_TRY(gemm(gp, rowmajor(N, w6, N, Vu, 1, ld, Bp.p, w6, 1, beta.p, w6, 1.0, 0.0), st));
-            CIR_TRY(gemm(gp, rowmajor(N, w6, N, Vu, 1, ld, Fp.p, w6, 1, phi.p, w6, 1.0, 0.0), st));
-            const char* be = beta.as<char>();
-            const char* ph = phi.as<char>();
-            const size_t im = size_t(w3) * esz;
-            // Pr = br fr^T - bi fi^T, Pi = br fi^T + bi fr^T (X1, X2)
-            CIR_TRY(gemm(gp, rowmajor(N, N, w3, be, w6, 1, ph, 1, w6, X1.p, ld, 1.0, 0.0), st));
-            CIR_TRY(gemm(gp, rowmajor(N, N, w3, be + im, w6, 1, ph + im, 1, w6, X1.p, ld, -1.0, 1.0), st));
-            CIR_TRY(gemm(gp, rowmajor(N, N, w3, be, w6, 1, ph + im, 1, w6, X2.p, ld, 1.0, 0.0), st));
-            CIR_TRY(gemm(gp, rowmajor(N, N, w3, be + im, w6, 1, ph, 1, w6, X2.p, ld, 1.0, 1.0), st));
+            const bool narrow = rp != CIR_PREC_FP64 && w3 <= propagate_max_cols();
+            const float* Vf = static_cast<const float*>(Vu);
+            if (narrow) {
+                CIR_TRY(propagate_project(N, ld, w3, Vf, Bp.as<float>(), w6, beta.as<float>(), w6, st));
+                CIR_TRY(propagate_project(N, ld, w3, Vf, Fp.as<float>(), w6, phi.as<float>(), w6, st));
+            } else {
+                CIR_TRY(gemm(gp, rowmajor(N, w6, N, Vu, 1, ld, Bp.p, w6, 1, beta.p, w6, 1.0, 0.0), st));
+                CIR_TRY(gemm(gp, rowmajor(N, w6, N, Vu, 1, ld, Fp.p, w6, 1, phi.p, w6, 1.0, 0.0), st));
+            }
+            // Pr = br fr^T - bi fi^T, Pi = br fi^T + bi fr^T (X1, X2), each one
+            // product [br | bi] [fr | -fi]^T, [br | bi] [fi | fr]^T
+            hipLaunchKernelGGL(adj_turn_kernel<T>, dim3(unsigned(ceil_div(int64_t(N) * w3, int64_t(kAdjNT)))), dim3(kAdjNT), 0,
+                               st, N, w3, phi.as<T>(), Fp.as<T>());
+            CIR_CHECK_LAUNCH();
+            CIR_TRY(gemm(gp, rowmajor(N, N, w6, beta.p, w6, 1, phi.p, 1, w6, X1.p, ld, 1.0, 0.0), st));
+            CIR_TRY(gemm(gp, rowmajor(N, N, w6, beta.p, w6, 1, Fp.p, 1, w6, X2.p, ld, 1.0, 0.0), st));
             hipLaunchKernelGGL(adj_rsym_kernel<T>, dim3(unsigned(ceil_div(N, 32)), unsigned(ceil_div(N, 32))),
                                dim3(256), 0, st, N, ld, tau, wu, X1.as<T>(), X2.as<T>(), X3.as<T>());
             CIR_CHECK_LAUNCH();
@@ -619,8 +637,12 @@ int backward_impl(cir_ctx* c, const double* dL_dy, double* grad) {
             CIR_TRY(gemm(gp, rowmajor(N, N, N, Vu, ld, 1, X3.p, ld, 1, X1.p, ld, 1.0, 0.0), st));
             CIR_TRY(gemm(gp, rowmajor(N, N, N, X1.p, ld, 1, Vu, 1, ld, X2.p, ld, 1.0, 0.0), st));
             Gs = X2.as<T>();
-            // b <- U(t) b for the next (earlier) frame
-            CIR_TRY(propagate(rp, c->prop_prec, N, ld, w3, w6, double(p.dt), Vu, wu, Bp.p, Bo.p, G.p, st));
+            // b <- U(t) b = V (phases) beta for the next (earlier) frame; in
+            // split BF16 the propagation's own products, as the forward has them
+            if (narrow && c->prop_prec != CIR_PREC_BF16X3)
+                CIR_TRY(propagate_expand(N, ld, w3, double(p.dt), Vf, wu, beta.as<float>(), w6, Bo.as<float>(), w6, st));
+            else
+                CIR_TRY(propagate(rp, c->prop_prec, N, ld, w3, w6, double(p.dt), Vu, wu, Bp.p, Bo.p, G.p, st));
             {
                 const int64_t tot = int64_t(N) * w6;
                 const unsigned g = unsigned((tot + kAdjNT - 1) / kAdjNT);

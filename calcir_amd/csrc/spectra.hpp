@@ -47,6 +47,15 @@ int spectral_density(int prec, int batch, int n, int ld, float t1, float avef, f
 size_t propagate_work_elems(int n, int ncols);
 int propagate(int prec, int gemm_prec, int n, int ld, int ncols, int ldy, double dt, const void* V,
               const double* w, const void* Yin, void* Yout, void* G, hipStream_t s, bool may_tune = true);
+// The two products of an FP32 propagation on their own, for up to
+// propagate_max_cols() complex columns (rows of [Re | Im]): C = V^T B, and C =
+// V diag(exp(i w dt / hbar)) G with G overwritten by the phased columns.  One
+// K segment, no workspace, a fixed order of sums.
+int propagate_max_cols();
+int propagate_project(int n, int ld, int ncols, const float* V, const float* B, int ldb, float* C, int ldc,
+                      hipStream_t s);
+int propagate_expand(int n, int ld, int ncols, double dt, const float* V, const double* w, float* G, int ldg, float* C,
+                     int ldc, hipStream_t s);
 // Whether propagate() of this shape would time candidates (false: its split is
 // settled, or the shape has none to choose), so that calls of it can be
 // captured into a graph.
