@@ -1,6 +1,6 @@
 // k_band.hip -- two-stage reduction of the batched FP32 eigensolver (gfx950),
 // replacing the one-stage Householder tridiagonalisation of magma_ssyevd_gpu
-// (calcIR.cu:420-448) for batches of mid-size Hamiltonians.
+// (calcIR.cu:420-448) for Hamiltonians of up to sb_max_n().
 //
 //   Stage 1, dense -> band of half-width kBandNB (LAPACK sytrd_sy2sb form):
 //     for each panel of kBandNB columns, sb_panel_kernel factors the panel
@@ -11,14 +11,15 @@
 //     Y (Yh^T X)/2 (sb_w_kernel), A22 -= W Y^T + Y W^T
 //     (sb_syr2k_kernel), on 32x32x2 FP32 MFMA.
 //   Stage 2, band -> tridiagonal (sb2st_kernel): bulge chasing, one workgroup
-//     per matrix, sweeps in groups of kSbG run by the group's waves in
-//     lock-step with a lag of two tasks (the tasks of one step touch disjoint
-//     elements); the band rows the group touches live in a circular LDS
-//     window that slides down the matrix.
+//     per matrix, sweeps in groups of kSbG run by the group's waves with a
+//     lag of two tasks (the tasks of one step touch disjoint elements), the
+//     groups one after the other as a stream of steps (SbStream); the band rows
+//     that the waves touch live in a circular LDS window over the stream.
 //   Q2 back-transform (q2_*): the bulge-chasing reflectors of kQ2G
-//     consecutive sweeps at one block position form a compact-WY block;
-//     blocks are applied to column slabs of the eigenvector matrix held in
-//     LDS, groups last to first, block positions in ascending order.
+//     consecutive sweeps at one block position form a compact-WY block; the
+//     rows of a column slab of the eigenvectors stream through a workgroup's
+//     waves, each applying its groups' blocks; groups last to first, block
+//     positions in ascending order.
 //
 // Storage (per matrix):
 //   BND   band rows: element (r, c), 0 <= r - c < 2 NB, at BND[r * 2NB + r - c]
@@ -520,9 +521,8 @@ constexpr int kBufferWord3 = 0x00020000;
 // from the panel row of the tile's column at that position, the B operand
 // from the panel row of the tile's row at the swapped half (k ^ NB).  The
 // next tile's A values and operand are in flight while a tile's MFMA chain
-// runs.  Bound by
-// memory (each element of A22 read and written, 3.3 TB/s) where there are many
-// matrices.  With a block row per wave 63 calls for one matrix of N = 2048 took
+// runs.  Bound by memory (each element of A22 read and written, 3.3 TB/s) where
+// there are many matrices.  With a block row per wave 63 calls for one matrix of N = 2048 took
 // 3.48 ms, 24 matrices of N = 3072 12.6, 48 of N = 768 0.62; with 4 waves to a row
 // 1.20, 10.0, 0.50.
 __global__ void __launch_bounds__(64 * kSyWaves) sb_syr2k_kernel(int n, int ld, int r0, float* __restrict__ Aall,
@@ -1082,14 +1082,23 @@ __device__ __forceinline__ float4 q2_split4(const float (&v)[4]) {
 
 // Per block (one wave): reflectors that do not exist (sweeps past n - 3, or
 // past their last task) are zeroed; T is formed (forward, columnwise), and V
-// and -V T are stored in the operand order of the 16x16x4 MFMA products that
-// apply the block (Z <- Z + (-V T) (V^T Z)): lane l's 12 values of each
-// contiguous, V_op[l][s] = V(4 s + l/16, l%16) and NVT_op[l][4 rt + s] =
-// (-V T)(16 rt + l%16, 4 s + l/16).  V_op replaces V in place.
+// and -V T are stored in the operand order of the MFMA products that apply the
+// block (Z <- Z + (-V T) (V^T Z)), 16 bytes a lane and load: register 4 q + e of
+// lane (lq, l16) holds V(16 q + 4 lq + e, l16), V^T as the A operand of the W
+// product, and of -V T, as the A operand of the update, NV(16 q + l16, 4 e + lq)
+// for FP32 16x16x4 steps and NV(16 q + l16, 4 lq + e) for split-BF16 products.
+// The split-BF16 operands are split here, once per block instead of once per
+// block and slab: each 16 bytes hold the hi and lo parts of 4 values.  V_op
+// replaces V in place.
+// V^T V and (-V T)^T are FP32 MFMA products, the second with T's columns in the
+// order that leaves the result in that layout; T's rows are a recursion in one
+// lane each.  With every product a sum over LDS, a thousand LDS instructions a
+// block, 256 matrices of N = 2048 took 6.2 ms; this takes 2.4, half of it memory.
 __global__ void __launch_bounds__(64) q2_prep_kernel(int n, int64_t nblk, float* __restrict__ Q2all, int bf16) {
-    __shared__ float sv[kQ2R][kQ2G + 1], st[kQ2G][kQ2G + 1], snv[kQ2R][kQ2G + 1], sgm[kQ2G][kQ2G + 1], stau[kQ2G];
+    __shared__ float sv[kQ2R][kQ2G + 1], st[kQ2G][kQ2G + 1], stau[kQ2G];
+    __shared__ __align__(16) float sgm[kQ2G][kQ2G + 4];
     const int64_t q = blockIdx.x;
-    const int b = blockIdx.y, lane = threadIdx.x;
+    const int b = blockIdx.y, lane = threadIdx.x, l16 = lane & 15, lq = lane >> 4;
     if (q >= nblk) return;
     float* blk = Q2all + (size_t(b) * nblk + q) * kQ2BlockFloats;
     float* V = blk;
@@ -1097,63 +1106,58 @@ __global__ void __launch_bounds__(64) q2_prep_kernel(int n, int64_t nblk, float*
     float* NVT = tau + kQ2G;
     int g, k;
     q2_block_gk(n, q, &g, &k);
-    for (int e = lane; e < kQ2R * kQ2G; e += 64) {
-        const int j = e / kQ2R, r = e % kQ2R;
-        const bool ex = k < sb_tasks(n, g * kQ2G + j);
-        sv[r][j] = ex ? V[e] : 0.f;
+#pragma unroll
+    for (int u = 0; u < kQ2R * kQ2G / 64; ++u) {
+        const int e = lane + 64 * u, j = e / kQ2R, r = e % kQ2R;
+        const float v = V[e];
+        sv[r][j] = k < sb_tasks(n, g * kQ2G + j) ? v : 0.f;
     }
-    if (lane < kQ2G) stau[lane] = (k < sb_tasks(n, g * kQ2G + lane)) ? tau[lane] : 0.f;
-    __syncthreads();
-    // the Gram matrix V^T V above its diagonal, all entries at once (4 per
-    // lane, each a 48-term dot product), then T column by column from it
-    for (int e = lane; e < kQ2G * kQ2G; e += 64) {
-        const int i = e / kQ2G, j = e % kQ2G;
-        if (i < j) {
-            float acc = 0.f;
-            for (int r = 0; r < kQ2R; ++r) acc += sv[r][i] * sv[r][j];
-            sgm[i][j] = acc;
-        }
+    if (lane < kQ2G) {
+        const float t = tau[lane];
+        stau[lane] = k < sb_tasks(n, g * kQ2G + lane) ? t : 0.f;
     }
     __syncthreads();
-    for (int j = 0; j < kQ2G; ++j) {
-        if (lane < j) {
-            float acc = 0.f;
-            for (int q2 = lane; q2 < j; ++q2) acc += st[lane][q2] * sgm[q2][j];
-            st[lane][j] = -stau[j] * acc;
-        } else if (lane == j) {
-            st[j][j] = stau[j];
-        } else if (lane < kQ2G) {
-            st[lane][j] = 0.f;
-        }
-        __syncthreads();
-    }
-    for (int e = lane; e < kQ2R * kQ2G; e += 64) {
-        const int j = e / kQ2R, r = e % kQ2R;
+    float vs[12];
+#pragma unroll
+    for (int e = 0; e < 12; ++e) vs[e] = sv[16 * (e / 4) + 4 * lq + e % 4][l16];
+    floatx4 gm = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 12; ++e) gm = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[e], vs[e], gm, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sgm[4 * lq + r][l16] = gm[r];
+    __syncthreads();
+    // T(0:l, l) = -tau_l T(0:l, 0:l) G(0:l, l), lane l16 the row l16 (G is
+    // symmetric: its column l is row l)
+    float Tr[kQ2G];
+#pragma unroll
+    for (int l = 0; l < kQ2G; ++l) {
         float acc = 0.f;
-        for (int q2 = 0; q2 <= j; ++q2) acc += sv[r][q2] * st[q2][j];
-        snv[r][j] = -acc;
+#pragma unroll
+        for (int c = 0; c < l; ++c) acc += Tr[c] * sgm[l][c];
+        const float tl = stau[l];
+        Tr[l] = l16 == l ? tl : (l16 < l ? -tl * acc : 0.f);
     }
+#pragma unroll
+    for (int l = 0; l < kQ2G; ++l)
+        if (lq == l / 4) st[l16][l] = Tr[l];
     __syncthreads();
-    const int l16 = lane & 15, lq = lane >> 4;
-    // V^T as the A operand of the W product: register 4 q + e of lane (lq,
-    // l16) holds V(16 q + 4 lq + e, l16); -V T as the A operand of the update,
-    // register 4 rt + s of lane (lq, l16): FP32 16x16x4 steps take NV(16 rt +
-    // l16, 4 s + lq), split-BF16 products NV(16 rt + l16, 4 lq + s).  The
-    // split-BF16 operands are split here, once per block instead of once per
-    // block and slab: each 16 bytes hold the hi and lo parts of 4 values.
+    const int jt = bf16 ? l16 : 4 * (l16 & 3) + (l16 >> 2);
+    float tt[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) tt[s] = -st[4 * s + lq][jt];
     float4 vp[3];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        float v[4], w[4];
+    for (int rt = 0; rt < 3; ++rt) {
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = sv[16 * q + 4 * lq + e][l16];
-            w[e] = bf16 ? snv[16 * q + l16][4 * lq + e] : snv[16 * q + l16][4 * e + lq];
-        }
-        float4* vo = reinterpret_cast<float4*>(V) + 64 * q + lane;
-        float4* wo = reinterpret_cast<float4*>(NVT) + 64 * q + lane;
+        for (int s = 0; s < 4; ++s)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(tt[s], sv[16 * rt + l16][4 * s + lq], acc, 0, 0, 0);
+        const float v[4] = {vs[4 * rt], vs[4 * rt + 1], vs[4 * rt + 2], vs[4 * rt + 3]};
+        const float w[4] = {acc[0], acc[1], acc[2], acc[3]};
+        float4* vo = reinterpret_cast<float4*>(V) + 64 * rt + lane;
+        float4* wo = reinterpret_cast<float4*>(NVT) + 64 * rt + lane;
         if (bf16) {
-            vp[q] = q2_split4(v);
+            vp[rt] = q2_split4(v);
             *wo = q2_split4(w);
         } else {
             *vo = float4{v[0], v[1], v[2], v[3]};

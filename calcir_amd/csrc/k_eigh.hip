@@ -1,8 +1,11 @@
 // k_eigh.hip -- batched symmetric eigensolver for gfx950, replacing
 // magma_ssyevd_gpu (calcIR.cu:420-448).
 //
-//   1. tridiag_kernel: Householder reduction A = Q T Q^T, one workgroup per
-//      matrix (a frame's Hamiltonian), panel-blocked: within a panel of
+//   1. Householder reduction A = Q T Q^T.  In FP32 mostly in two stages
+//      (k_band.hip); matrices of N <= kSmallN with the matrix in registers
+//      (tridiag_small_kernel); the rest by tridiag_kernel, one workgroup per
+//      matrix (a frame's Hamiltonian), or a grid per step (tri1_*).
+//      tridiag_kernel is panel-blocked: within a panel of
 //      kTriNB columns the two-sided update is deferred and folded into each
 //      column and each symmetric matrix-vector product through the panel's
 //      V and W (A_now = A_panel - V W^T - W V^T); the trailing matrix is
@@ -18,10 +21,12 @@
 //      FP32 trailing update runs on MFMA 32x32x2 straight from it.
 //      The reflector v_j (v_j[j+1] = 1) replaces column j of A below the
 //      diagonal; rows 0..j of column j are zeroed.
-//   2. bisect_kernel: every eigenvalue of T by FP64 Sturm-sequence
-//      bisection, one lane per eigenvalue (eigenvalues come out ascending).
+//   2. bisect_kernel: every eigenvalue of T by FP64 bisection on the sign
+//      changes of the leading principal minors (rescaled in runs of rows), one
+//      lane per eigenvalue (eigenvalues come out ascending).
 //   3. invit_kernel: eigenvectors of T by FP64 inverse iteration with
-//      partial pivoting, one lane per eigenvalue; neighbours closer than
+//      partial pivoting, one lane per eigenvalue, its LU factors recomputed
+//      from checkpoints rather than kept; neighbours closer than
 //      1e-7 * max(|lambda|, 1) form a cluster (at most kMaxCluster members)
 //      that its first lane solves sequentially with modified Gram-Schmidt
 //      against the cluster's earlier vectors.  Both this tolerance and the
@@ -33,6 +38,8 @@
 //      A pass joins two blocks of kBtNB reflectors, T = [T1 T12; 0 T2] with
 //      T12 = -T1 (Y1^T Y2) T2, so Z is read and written once per 256
 //      reflectors.
+//   5. FP32, where use_refine() says so: one first-order correction of the
+//      eigenpairs from a copy of H.
 
 #include <cfloat>
 #include <cstdlib>
@@ -782,7 +789,8 @@ tridiag_kernel(int n, int ld, T* __restrict__ Aall, T* __restrict__ dall, T* __r
 // owners put into LDS (every wave forms the norm and the scalars itself), p =
 // A v with the partial sums of a row in one row of 16 lanes, and A -= v w^T + w
 // v^T; two barriers.  Bound by these chains' latency and, at first, by the
-// updates' issue.  SMALLTIMES
+// updates' issue: 4.4 us a column at N = 256 (FP64 6.9) against 10 (12.5) in the
+// panel form; 205 matrices in FP32 2.50 -> 1.13 ms, 64 in FP64 3.19 -> 1.78.
 constexpr int kSmallN = 256;
 template <typename T, int AR, int LB, int RB>
 __global__ void __launch_bounds__(kTriNT)
@@ -1778,7 +1786,8 @@ invit_kernel(int n, int ld, const T* __restrict__ dall, const T* __restrict__ ea
 // The recursion over 128 columns is a chain of 128 products and barriers
 // (150 us for any number of matrices up to a few per CU); here a wave runs it
 // on each of eight 16-column blocks, and blocks are joined pairwise, T = [T1
-// T12; 0 T2] with T12 = -T1 (G12 T2), three times: LARFTTIMES.
+// T12; 0 T2] with T12 = -T1 (G12 T2), three times: 70 us for both blocks of
+// a pass together.
 // One LDS array holds G above the diagonal, T in its place as blocks are
 // finished, and the products G12 T2 in the mirror image of T12's place.
 constexpr int kLtB = 16;         // columns of a recursion
@@ -1905,8 +1914,9 @@ inline size_t larft_smem_bytes(size_t esz) { return size_t(kBtNB) * kLtP * esz; 
 // with n: the whole-GPU form runs batches of up to n / kSinglePer matrices.
 // CIR_EIGH_STAGES=1 or 2 in the environment forces one or two stages where
 // both apply (tests compare them).
-inline bool use_two_stage(size_t esz, int n) {
+inline bool use_two_stage(size_t esz, int n, int ld) {
     if (esz != sizeof(float) || n > sb_max_n() || n < 2 * kBandNB + 2) return false;
+    if (int64_t(n) * ld * 4 > 0x7fffffff) return false;  // byte offsets within a matrix are 32-bit
     if (deterministic_mode()) return true;  // the form without float atomics
     const char* fv = std::getenv("CIR_EIGH_STAGES");
     const int forced = fv ? std::atoi(fv) : 0;
@@ -2138,7 +2148,7 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
     EighWork L{};
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t o = 0;
-    L.two = use_two_stage(esz, n);
+    L.two = use_two_stage(esz, n, ld);
     if (L.two) {
         L.off_bnd = o;
         o = al(o + esz * batch * size_t(n) * kBandW);

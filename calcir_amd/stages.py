@@ -132,7 +132,7 @@ def correlate(sites, Y, nslot=1):
     [nslot, 3]."""
     n = sites.shape[-1]
     _need(sites.shape[-2] == NSITE and Y.shape[0] == n and Y.shape[1] >= 18 * nslot, "bad shapes")
-    out = torch.zeros((nslot, 6), dtype=torch.float64, device=Y.device)
+    out = torch.empty((nslot, 6), dtype=torch.float64, device=Y.device)  # every slot is written
     target = torch.arange(nslot, dtype=torch.int32, device=Y.device)
     check(lib().cir_correlate(_prec_of(Y.dtype), n, nslot, Y.shape[1], None, _p(target), _p(sites.contiguous()),
                               _p(Y), _p(out), _stream()))
