@@ -234,6 +234,16 @@ __device__ __forceinline__ void minimage3(T& dx, T& dy, T& dz, const PBox<T>& B)
     dx = dx - s * B.a0;
 }
 
+// Square of the length of a minimum image.  Written out, so that every kernel
+// that forms it rounds alike: left to the compiler, which of the squares is
+// rounded by itself depends on the code around it, and where two molecules
+// nearly overlap (H of 1e5 cm^-1 and more) an ulp of a distance turns the phase
+// of their modes by 1e-3 .. 1e-2 over a run.
+template <typename T>
+__device__ __forceinline__ T image_square(T dx, T dy, T dz) {
+    return fma(dz, dz, fma(dy, dy, dx * dx));
+}
+
 // Neumaier-compensated accumulation.
 template <typename T>
 struct Compensated {

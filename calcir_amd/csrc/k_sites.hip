@@ -14,9 +14,9 @@
 // Hamiltonian (calcIR.cu:1306-1404): a 64x64 tile on or below the diagonal per
 // workgroup over the site records; every element is computed once and written
 // to both triangles, lanes along the rows of each (the mirrored tile through
-// LDS), so H(i,j) == H(j,i) bit for bit.  Bound by its arithmetic (about 60
-// instructions an element).  32 frames of 2048 OH in FP32: 0.44
-// ms with every element of both triangles computed, 0.26 ms here, against 0.105
+// LDS), so H(i,j) == H(j,i) bit for bit.  Bound by its arithmetic (an IEEE root
+// and two quotients an element among it).  32 frames of 2048 OH in FP32: 0.44
+// ms with every element of both triangles computed, 0.34 ms here, against 0.105
 // ms for writing H at the rate of a large copy.
 
 #include <algorithm>
@@ -155,8 +155,8 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
                 T h2[3] = {a[3] - o[0], a[4] - o[1], a[5] - o[2]};
                 minimage3<T>(h1[0], h1[1], h1[2], Bt);
                 minimage3<T>(h2[0], h2[1], h2[2], Bt);
-                const T r1 = sqrt(h1[0] * h1[0] + h1[1] * h1[1] + h1[2] * h1[2]);
-                const T r2 = sqrt(h2[0] * h2[0] + h2[1] * h2[1] + h2[2] * h2[2]);
+                const T r1 = sqrt(image_square<T>(h1[0], h1[1], h1[2]));
+                const T r2 = sqrt(image_square<T>(h2[0], h2[1], h2[2]));
                 T bi[3];
                 for (int c = 0; c < 3; ++c) bi[c] = h1[c] / r1 + h2[c] / r2;
                 const T rb = sqrt(bi[0] * bi[0] + bi[1] * bi[1] + bi[2] * bi[2]);
@@ -167,7 +167,7 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
                     // calcIR.cu:1124-1140: M moved to 0.015 nm along O->M
                     T om[3] = {ms[0] - o[0], ms[1] - o[1], ms[2] - o[2]};
                     minimage3<T>(om[0], om[1], om[2], Bt);
-                    const T rom = sqrt(om[0] * om[0] + om[1] * om[1] + om[2] * om[2]);
+                    const T rom = sqrt(image_square<T>(om[0], om[1], om[2]));
                     for (int c = 0; c < 3; ++c) ms[c] = o[c] + T(kOMTip4p) * om[c] / rom;
                 }
             }
@@ -180,7 +180,7 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
                 dx = dx * bohr;
                 dy = dy * bohr;
                 dz = dz * bohr;
-                const T r = sqrt(dx * dx + dy * dy + dz * dz);
+                const T r = sqrt(image_square<T>(dx, dy, dz));
                 const T qc = (s < 2) ? T(kQH) : T(-kQM);
                 const T qr3 = qc / (r * r * r);
                 ex.add(qr3 * dx);
@@ -235,7 +235,7 @@ eproj_sites_kernel(int natoms, int natom_mol, int nchrom_mol, int imodel, int ru
     const T ox = T(no[0]), oy = T(no[1]), oz = T(no[2]);
     T ux = T(nh[0]) - ox, uy = T(nh[1]) - oy, uz = T(nh[2]) - oz;
     minimage3<T>(ux, uy, uz, Bt);
-    const T r = sqrt(ux * ux + uy * uy + uz * uz);
+    const T r = sqrt(image_square<T>(ux, uy, uz));
     ux /= r;
     uy /= r;
     uz /= r;

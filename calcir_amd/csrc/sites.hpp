@@ -22,25 +22,25 @@ MapT<T> map_t(const MapCoef& c) {
 // d the unit min-image separation of the TDM positions.  The coupling is
 // this times (x_i mu'_i)(x_j mu'_j) times the hartree -> cm^-1 factor.  The
 // operation order is symmetric in i and j, so H(i,j) == H(j,i) bit for bit.
+// Root and quotients are IEEE and the fused operations written out: with 1 / r
+// from the hardware's reciprocal root (one ulp), cubed, the FP32 couplings of
+// nearly overlapping molecules were twice as far from FP64's (5.8e-7 of H
+// against 3.0e-7), for 0.08 ms less of 32 frames of 2048 OH.
 template <typename T>
 __device__ __forceinline__ T tdc_geometry(T uix, T uiy, T uiz, T rix, T riy, T riz, T ujx, T ujy, T ujz, T rjx,
                                           T rjy, T rjz, const PBox<T>& bb) {
     T dr[3] = {rix - rjx, riy - rjy, riz - rjz};
     minimage3<T>(dr[0], dr[1], dr[2], bb);
-    const T r2 = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
-    // 1 / r: the hardware's reciprocal root is within one ulp in FP32
-    T inv;
-    if constexpr (sizeof(T) == 4)
-        inv = __builtin_amdgcn_rsqf(r2);
-    else
-        inv = T(1) / sqrt(r2);
+    const T r = sqrt(image_square<T>(dr[0], dr[1], dr[2]));
+    const T inv = T(1) / r;
     const T d0 = dr[0] * inv, d1 = dr[1] * inv, d2 = dr[2] * inv;
-    const T uu = uix * ujx + uiy * ujy + uiz * ujz;
-    const T ur = uix * d0 + uiy * d1 + uiz * d2;
-    const T vr = ujx * d0 + ujy * d1 + ujz * d2;
-    const T ib = inv * T(1.0 / kBohrPerNm);
+    auto dot = [](T ax, T ay, T az, T bx, T by, T bz) { return fma(az, bz, fma(ax, bx, ay * by)); };
+    const T uu = dot(uix, uiy, uiz, ujx, ujy, ujz);
+    const T ur = dot(uix, uiy, uiz, d0, d1, d2);
+    const T vr = dot(ujx, ujy, ujz, d0, d1, d2);
+    const T rb = r * T(kBohrPerNm);
     const T t = ur * vr;
-    return (uu - T(3) * t) * (ib * ib * ib);
+    return fma(T(-3), t, uu) / (rb * rb * rb);
 }
 
 }  // namespace cir
