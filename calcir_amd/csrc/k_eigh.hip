@@ -1956,15 +1956,19 @@ inline bool use_refine(size_t esz, bool two, int batch, int n) {
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
 constexpr int kRqRun = 128;          // rows summed in one MFMA chain
-// C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major:
-// 64 x 64 tiles, four waves of one 32x32 fragment on the FP32 MFMA.
+// C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major;
+// GRAM: C = (I - V^T V) / 2 on the tiles on and above the diagonal (Hall and
+// wall are not read).  64 x 64 tiles, four waves of one 32x32 fragment on the
+// FP32 MFMA.
+template <bool GRAM>
 __global__ void __launch_bounds__(256)
 residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __restrict__ Vall,
                 const double* __restrict__ wall, float* __restrict__ Call) {
     __shared__ float As[kRqK][kRqT + 4], Bs[kRqK][kRqT + 4];
     const int b = blockIdx.z, m0 = blockIdx.y * kRqT, n0 = blockIdx.x * kRqT;
-    const float* H = Hall + size_t(b) * n * ld;
+    if (GRAM && m0 > n0) return;
     const float* V = Vall + size_t(b) * n * ld;
+    const float* H = GRAM ? V : Hall + size_t(b) * n * ld;
     float* C = Call + size_t(b) * n * ld;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
     const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
@@ -1976,7 +1980,7 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int k = kb + k0 + 4 * q, kc = min(k, n - 1);
-            ra[q] = (kc == cm) ? 0.f : H[size_t(kc) * ld + cm];
+            ra[q] = (!GRAM && kc == cm) ? 0.f : H[size_t(kc) * ld + cm];
             rb[q] = (k < n) ? V[size_t(kc) * ld + cn] : 0.f;
         }
     };
@@ -2007,47 +2011,56 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[k + h][wm + l32], Bs[k + h][wn + l32], acc, 0, 0, 0);
     }
     const int k = n0 + wn + l32;
-    const double lam = wall[size_t(b) * n + min(k, n - 1)];
+    const double lam = GRAM ? 0.0 : wall[size_t(b) * n + min(k, n - 1)];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int i = m0 + wm + 8 * (q >> 2) + 4 * h + (q & 3);
-        if (i < n && k < n) {
+        if (i >= n || k >= n) continue;
+        if constexpr (GRAM) {
+            C[size_t(i) * ld + k] = 0.5f * ((i == k ? 1.f : 0.f) - (sum[q] + acc[q]));
+        } else {
             const double v = double(V[size_t(i) * ld + k]);
             C[size_t(i) * ld + k] = float(double(sum[q] + acc[q]) + (double(H[size_t(i) * ld + i]) - lam) * v);
         }
     }
 }
 
-// D -> E in place, the diagonal of D into dl.  E takes the symmetric part of
-// D: its antisymmetric part is V's own loss of orthogonality and the product's
-// rounding, which divided by small gaps would make it worse.  Pairs whose gap
-// is not large against D_ij are left as they are: a rotation by E_ij taken to
-// first order lengthens its vectors by E_ij^2, which the bound keeps below
-// FP32's rounding, and what a pair's mixing does to the results is D_ij against
-// the frequencies that they resolve, whatever the gap.  One workgroup per tile
-// on or above the diagonal and its mirror image.
+// D -> E in place, the diagonal of D into dl; Q = (I - V^T V) / 2 (its upper
+// triangle).  E_ij = Dsym_ij / (lambda_j - lambda_i) + Q_ij with the symmetric
+// part of D, which is D_ij / (lambda_j - lambda_i) in exact arithmetic: D's
+// antisymmetric part is V's own loss of orthogonality and the product's
+// rounding, which divided by small gaps would make it worse, so Q takes its
+// place.  Pairs whose gap is not large against D_ij are not rotated, only made
+// orthogonal: a rotation by E_ij taken to first order lengthens its vectors by
+// E_ij^2, which the bound keeps below FP32's rounding, and what a pair's mixing
+// does to the results is D_ij against the frequencies that they resolve,
+// whatever the gap.  (E's diagonal is left to the scaling of the columns.)  One
+// workgroup per tile on or above the diagonal and its mirror image.
 constexpr double kRotationGap = 2048.0;
 constexpr int kRotT = 32;
 __global__ void __launch_bounds__(256)
-rotation_kernel(int n, int ld, const double* __restrict__ wall, float* __restrict__ Dall, float* __restrict__ dlall) {
+rotation_kernel(int n, int ld, const double* __restrict__ wall, const float* __restrict__ Qall, float* __restrict__ Dall,
+                float* __restrict__ dlall) {
     __shared__ float lo[kRotT][kRotT + 1];  // the mirror tile, then its new values
     const int I = blockIdx.y * kRotT, J = blockIdx.x * kRotT, b = blockIdx.z;
     if (I > J) return;
     const double* w = wall + size_t(b) * n;
+    const float* Q = Qall + size_t(b) * n * ld;
     float* D = Dall + size_t(b) * n * ld;
     const int c = threadIdx.x % kRotT, r0 = threadIdx.x / kRotT;
     for (int r = r0; r < kRotT; r += 256 / kRotT)
         if (J + r < n && I + c < n) lo[r][c] = D[size_t(J + r) * ld + I + c];
     __syncthreads();
-    float up[kRotT * kRotT / 256];
+    float up[kRotT * kRotT / 256], qs[kRotT * kRotT / 256];
 #pragma unroll
     for (int q = 0; q < kRotT * kRotT / 256; ++q) {
         const int r = r0 + q * (256 / kRotT), i = I + r, j = J + c;
-        up[q] = 0.f;
+        up[q] = qs[q] = 0.f;
         if (i < n && j < n) {
             const double d = 0.5 * (double(D[size_t(i) * ld + j]) + double(lo[c][r]));
             const double gap = w[j] - w[i];
             if (i == j) dlall[size_t(b) * n + j] = float(d);
+            if (i != j) qs[q] = Q[size_t(min(i, j)) * ld + max(i, j)];
             if (i != j && fabs(gap) > kRotationGap * fabs(d)) up[q] = float(d / gap);
         }
     }
@@ -2055,8 +2068,8 @@ rotation_kernel(int n, int ld, const double* __restrict__ wall, float* __restric
 #pragma unroll
     for (int q = 0; q < kRotT * kRotT / 256; ++q) {
         const int r = r0 + q * (256 / kRotT), i = I + r, j = J + c;
-        if (i < n && j < n) D[size_t(i) * ld + j] = up[q];
-        lo[c][r] = -up[q];
+        if (i < n && j < n) D[size_t(i) * ld + j] = qs[q] + up[q];
+        lo[c][r] = qs[q] - up[q];
     }
     __syncthreads();
     if (I != J)
@@ -2373,7 +2386,10 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
             const int64_t mat = int64_t(n) * ld;
             const unsigned nt = unsigned(ceil_div(n, kRqT)), nc = unsigned(ceil_div(n, 256)),
                            nr = unsigned(ceil_div(n, kRotT));
-            hipLaunchKernelGGL(residual_kernel, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, H, V, w, C);
+            hipLaunchKernelGGL(residual_kernel<false>, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, H, V, w, C);
+            CIR_CHECK_LAUNCH();
+            // (the reflectors in A have been applied)
+            hipLaunchKernelGGL(residual_kernel<true>, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, V, V, w, A);
             CIR_CHECK_LAUNCH();
             auto product = [&](const float* a, int64_t a_m, int64_t a_k, const float* bb, float* c) {
                 GemmArgs g;
@@ -2392,7 +2408,7 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
                 return gemm(CIR_PREC_BF16X3, g, s);
             };
             CIR_TRY(product(V, 1, ld, C, H));
-            hipLaunchKernelGGL(rotation_kernel, dim3(nr, nr, unsigned(batch)), dim3(256), 0, s, n, ld, w, H, dl);
+            hipLaunchKernelGGL(rotation_kernel, dim3(nr, nr, unsigned(batch)), dim3(256), 0, s, n, ld, w, A, H, dl);
             CIR_CHECK_LAUNCH();
             CIR_TRY(product(V, ld, 1, H, C));
             hipLaunchKernelGGL(correct_w_kernel, dim3(unsigned(batch)), dim3(1024), 2 * size_t(n) * sizeof(double), s, n, dl,
