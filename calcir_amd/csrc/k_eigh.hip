@@ -39,7 +39,7 @@
 //      T12 = -T1 (Y1^T Y2) T2, so Z is read and written once per 256
 //      reflectors.
 //   5. FP32, where use_refine() says so: one first-order correction of the
-//      eigenpairs from a copy of H.
+//      eigenpairs from a copy of H, and of the eigenvectors' orthogonality.
 
 #include <cfloat>
 #include <cstdlib>
@@ -1936,18 +1936,22 @@ inline bool use_whole_gpu(int batch, int n) {
 // against 1.3e-7 by panels).  Where the reduction is
 // bound by its chains rather than by its arithmetic (small matrices, small
 // batches) three N^3 products cost little, and the eigenpairs get one step of
-// first-order correction from a copy of H: with the residuals C = H V - V L
-// and D = V^T C, lambda_j += D_jj and V += V E, E_ij = D_ij / (lambda_j -
-// lambda_i).  E is antisymmetric, so V stays orthogonal to second order.
-// Only C needs FP32's full accuracy (H's diagonal, its largest entries, is
-// taken out of the product and applied in FP64 with the eigenvalue; the rest
+// first-order correction from a copy of H: with the residuals C = H V - V L, D =
+// V^T C and Q = (I - V^T V) / 2, lambda_j += D_jj and V += V E, E_ij = Dsym_ij /
+// (lambda_j - lambda_i) + Q_ij (rotation_kernel).  Without Q, the loss of
+// orthogonality of a split-BF16 back-transform stays (V V^T off by 3e-5 at N =
+// 256 and 5e-5 at N = 766; 1e-7 with it), which a run applies at every step:
+// 150 points of N = 256 were up to 1.6e-5 off in VV and VH, and are 2e-6 .. 6e-6.
+// C and Q need FP32's full accuracy (H's diagonal, its largest entries, is
+// taken out of C's product and applied in FP64 with the eigenvalue; the rest
 // is summed in runs, an FP32 MFMA chain over all rows biases the eigenvalues by
-// 4e-6); D and E are corrections, formed in split-BF16x3.  The vectors are then
-// scaled to length one (first-order rotations lengthen them by E_ij^2, 2e-7 on
-// average).  After it: eigenvalues 2e-8, the density 5e-8 .. 2e-7 (one stage:
-// 2e-7 .. 3e-7 and 1e-7 .. 4e-7).  One matrix of n = 2048: 0.9 of 42 ms; 48 of
-// n = 766: 1.7 of 13; 24 of n = 3072: 30 of 168.  Above kRefineAboveN, where
-// only the one-stage form used to run, it is always made.
+// 4e-6); D and E are corrections, formed in split-BF16x3 in either precision
+// (their products' error, 1e-5 of a correction, is below FP32's rounding of V).
+// The vectors are then scaled to length one.  After it: eigenvalues 2e-8, the
+// density 5e-8 .. 2e-7 (one stage: 2e-7 .. 3e-7 and 1e-7 .. 4e-7).  One matrix of
+// n = 2048: 1.1 of 33 ms; 48 of n = 766: 2.1 of 11.8; 24 of n = 3072: 49 of 164
+// (Q's part of these 0.23, 0.43, 12).  Above kRefineAboveN, where only the
+// one-stage form used to run, it is always made.
 constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16, kRefineAboveN = 2080;
 inline bool use_refine(size_t esz, bool two, int batch, int n) {
     if (esz != sizeof(float) || !(two || n <= kSmallN)) return false;

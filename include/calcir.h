@@ -358,12 +358,16 @@ int cir_hamiltonian(int prec, int nframes, int n, int ld, int nchrom_mol, int is
                     float avef, const float* box_d, const void* sites_d, void* H_d, void* stream);
 /* Batched symmetric eigensolver replacing magma_ssyevd_gpu (calcIR.cu:443):
  * A_d holds batch matrices (n x n, leading dimension ld, batch stride n*ld,
- * symmetric, both triangles) and is destroyed (it receives the Householder
- * reflectors); V_d receives the eigenvectors row-major, V[b][i*ld + k] =
+ * symmetric, both triangles) and is destroyed (it holds the Householder
+ * reflectors, then intermediate products); V_d receives the eigenvectors row-major, V[b][i*ld + k] =
  * component i of eigenvector k, and w_d (batch*n doubles) the eigenvalues in
  * ascending order.  Real arrays are float unless prec == CIR_PREC_FP64;
  * CIR_PREC_BF16X3 keeps float arrays and forms the back-transform products
  * with split-BF16x3 MFMA (eigenvector error ~1e-5 instead of ~1e-6).
+ * Float eigenpairs of n < 1024, of 2080 < n <= 3104 and of batches of at most
+ * 16 in between are corrected once from a copy of A, the residuals in FP32 and
+ * the products that apply them in split-BF16x3 in both precisions: the
+ * eigenvectors come out orthogonal to FP32's rounding.
  * ld must be a multiple of 4 and A_d 16-byte aligned (rows are streamed as
  * 16-byte vectors).  work_d must hold cir_eigh_workspace() bytes. */
 size_t cir_eigh_workspace(int prec, int batch, int n, int ld);
