@@ -1942,16 +1942,17 @@ inline bool use_whole_gpu(int batch, int n) {
 // orthogonality of a split-BF16 back-transform stays (V V^T off by 3e-5 at N =
 // 256 and 5e-5 at N = 766; 1e-7 with it), which a run applies at every step:
 // 150 points of N = 256 were up to 1.6e-5 off in VV and VH, and are 2e-6 .. 6e-6.
-// C and Q need FP32's full accuracy (H's diagonal, its largest entries, is
-// taken out of C's product and applied in FP64 with the eigenvalue; the rest
-// is summed in runs, an FP32 MFMA chain over all rows biases the eigenvalues by
-// 4e-6); D and E are corrections, formed in split-BF16x3 in either precision
-// (their products' error, 1e-5 of a correction, is below FP32's rounding of V).
-// The vectors are then scaled to length one.  After it: eigenvalues 2e-8, the
-// density 5e-8 .. 2e-7 (one stage: 2e-7 .. 3e-7 and 1e-7 .. 4e-7).  One matrix of
-// n = 2048: 1.1 of 33 ms; 48 of n = 766: 2.1 of 11.8; 24 of n = 3072: 49 of 164
-// (Q's part of these 0.23, 0.43, 12).  Above kRefineAboveN, where only the
-// one-stage form used to run, it is always made.
+// C is formed in FP64: its sum cancels to the rounding of one element, and where
+// two molecules nearly overlap that is H's largest (max|H| = 1e5: eigenvalues
+// 3.5e-2 off with C from FP32 MFMA, 3e-4 here; in ordinary frames 2e-6 and 1e-9).
+// Q needs FP32's full accuracy; D and E are corrections, formed in split-BF16x3
+// in either precision (their products' error, 1e-5 of a correction, is below
+// FP32's rounding of V).  The vectors are then scaled to length one.  After it:
+// eigenvalues 2e-8, the density 5e-8 .. 2e-7 (one stage: 2e-7 .. 3e-7 and 1e-7 ..
+// 4e-7).  One matrix of n = 2048: 1.2 of 33 ms; 48 of n = 766: 2.4 of 12; 24 of n =
+// 3072: 58 of 173 (Q's part of these 0.23, 0.43, 12; C's FP64 costs 0.13, 0.26 and
+// 9 more than FP32).  Above kRefineAboveN, where only the one-stage form used to
+// run, it is always made.
 constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16, kRefineAboveN = 2080;
 inline bool use_refine(size_t esz, bool two, int batch, int n) {
     if (esz != sizeof(float) || !(two || n <= kSmallN)) return false;
@@ -1960,39 +1961,21 @@ inline bool use_refine(size_t esz, bool two, int batch, int n) {
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
 constexpr int kRqRun = 128;          // rows summed in one MFMA chain
-// C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major;
-// GRAM: C = (I - V^T V) / 2 on the tiles on and above the diagonal (Hall and
-// wall are not read).  64 x 64 tiles, four waves of one 32x32 fragment on the
-// FP32 MFMA.
-template <bool GRAM>
-__global__ void __launch_bounds__(256)
-residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __restrict__ Vall,
-                const double* __restrict__ wall, float* __restrict__ Call) {
-    __shared__ float As[kRqK][kRqT + 4], Bs[kRqK][kRqT + 4];
-    const int b = blockIdx.z, m0 = blockIdx.y * kRqT, n0 = blockIdx.x * kRqT;
-    if (GRAM && m0 > n0) return;
-    const float* V = Vall + size_t(b) * n * ld;
-    const float* H = GRAM ? V : Hall + size_t(b) * n * ld;
-    float* C = Call + size_t(b) * n * ld;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
-    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-    // each thread stages 4 values of either operand, 64 consecutive ones per wave
-    const int c = tid & 63, k0 = tid >> 6;
-    const int cm = min(m0 + c, n - 1), cn = min(n0 + c, n - 1);
+// The tiles of an n x n product A^T B (row-major operands, pitch ld): 64 x 64 per
+// workgroup, K steps of kRqK staged in LDS, each thread 4 values of either
+// operand, 64 consecutive ones per wave.  STEP(As, Bs, kb) uses a staged step.
+template <typename LA, typename LB, typename STEP>
+__device__ __forceinline__ void rq_tiles(int n, float (&As)[kRqK][kRqT + 4], float (&Bs)[kRqK][kRqT + 4], LA&& la, LB&& lb,
+                                         STEP&& step) {
+    const int c = threadIdx.x & 63, k0 = threadIdx.x >> 6;
     float ra[4], rb[4];
     auto load = [&](int kb) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int k = kb + k0 + 4 * q, kc = min(k, n - 1);
-            ra[q] = (!GRAM && kc == cm) ? 0.f : H[size_t(kc) * ld + cm];
-            rb[q] = (k < n) ? V[size_t(kc) * ld + cn] : 0.f;
+            ra[q] = la(kb + k0 + 4 * q);
+            rb[q] = lb(kb + k0 + 4 * q);
         }
     };
-    // summed in runs of kRqRun rows: each run's sum is small beside the whole,
-    // so is its rounding
-    floatx16 acc, sum;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = sum[q] = 0.f;
     load(0);
     for (int kb = 0; kb < n; kb += kRqK) {
         __syncthreads();
@@ -2003,29 +1986,97 @@ residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __re
         }
         __syncthreads();
         load(kb + kRqK);
-        if (kb % kRqRun == 0) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                sum[q] += acc[q];
-                acc[q] = 0.f;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < kRqK; k += 2)
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[k + h][wm + l32], Bs[k + h][wn + l32], acc, 0, 0, 0);
+        step(kb);
     }
+}
+
+// C = H V - V diag(w), all n x n with pitch ld, H symmetric, V and C row-major,
+// in FP64: four waves of 2 x 2 fragments on the 16x16x4 MFMA.
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(256)
+residual_kernel(int n, int ld, const float* __restrict__ Hall, const float* __restrict__ Vall,
+                const double* __restrict__ wall, float* __restrict__ Call) {
+    __shared__ float As[kRqK][kRqT + 4], Bs[kRqK][kRqT + 4];
+    const int b = blockIdx.z, m0 = blockIdx.y * kRqT, n0 = blockIdx.x * kRqT;
+    const float* H = Hall + size_t(b) * n * ld;
+    const float* V = Vall + size_t(b) * n * ld;
+    float* C = Call + size_t(b) * n * ld;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
+    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    const int cm = min(m0 + (tid & 63), n - 1), cn = min(n0 + (tid & 63), n - 1);
+    doublex4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
+    rq_tiles(
+        n, As, Bs, [&](int k) { return H[size_t(min(k, n - 1)) * ld + cm]; },
+        [&](int k) { return k < n ? V[size_t(k) * ld + cn] : 0.f; },
+        [&](int) {
+#pragma unroll
+            for (int k = 0; k < kRqK; k += 4) {
+                double a[2], bb[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[i] = double(As[k + kq][wm + 16 * i + l16]);
+                    bb[i] = double(Bs[k + kq][wn + 16 * i + l16]);
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bb[j], acc[i][j], 0, 0, 0);
+            }
+        });
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int k = n0 + wn + 16 * j + l16;
+        const double lam = wall[size_t(b) * n + min(k, n - 1)];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = m0 + wm + 16 * i + kq + 4 * r;
+                if (m < n && k < n) C[size_t(m) * ld + k] = float(acc[i][j][r] - lam * double(V[size_t(m) * ld + k]));
+            }
+    }
+}
+
+// Q = (I - V^T V) / 2 on the tiles on and above the diagonal, in FP32: four waves
+// of one 32x32 fragment, summed in runs of kRqRun rows (each run's sum is small
+// beside the whole, so is its rounding).
+__global__ void __launch_bounds__(256)
+gram_kernel(int n, int ld, const float* __restrict__ Vall, float* __restrict__ Qall) {
+    __shared__ float As[kRqK][kRqT + 4], Bs[kRqK][kRqT + 4];
+    const int b = blockIdx.z, m0 = blockIdx.y * kRqT, n0 = blockIdx.x * kRqT;
+    if (m0 > n0) return;
+    const float* V = Vall + size_t(b) * n * ld;
+    float* Q = Qall + size_t(b) * n * ld;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
+    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    const int cm = min(m0 + (tid & 63), n - 1), cn = min(n0 + (tid & 63), n - 1);
+    floatx16 acc, sum;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[q] = sum[q] = 0.f;
+    rq_tiles(
+        n, As, Bs, [&](int k) { return V[size_t(min(k, n - 1)) * ld + cm]; },
+        [&](int k) { return k < n ? V[size_t(k) * ld + cn] : 0.f; },
+        [&](int kb) {
+            if (kb % kRqRun == 0) {
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    sum[q] += acc[q];
+                    acc[q] = 0.f;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kRqK; k += 2)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[k + h][wm + l32], Bs[k + h][wn + l32], acc, 0, 0, 0);
+        });
     const int k = n0 + wn + l32;
-    const double lam = GRAM ? 0.0 : wall[size_t(b) * n + min(k, n - 1)];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int i = m0 + wm + 8 * (q >> 2) + 4 * h + (q & 3);
-        if (i >= n || k >= n) continue;
-        if constexpr (GRAM) {
-            C[size_t(i) * ld + k] = 0.5f * ((i == k ? 1.f : 0.f) - (sum[q] + acc[q]));
-        } else {
-            const double v = double(V[size_t(i) * ld + k]);
-            C[size_t(i) * ld + k] = float(double(sum[q] + acc[q]) + (double(H[size_t(i) * ld + i]) - lam) * v);
-        }
+        if (i < n && k < n) Q[size_t(i) * ld + k] = 0.5f * ((i == k ? 1.f : 0.f) - (sum[q] + acc[q]));
     }
 }
 
@@ -2390,10 +2441,10 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
             const int64_t mat = int64_t(n) * ld;
             const unsigned nt = unsigned(ceil_div(n, kRqT)), nc = unsigned(ceil_div(n, 256)),
                            nr = unsigned(ceil_div(n, kRotT));
-            hipLaunchKernelGGL(residual_kernel<false>, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, H, V, w, C);
+            hipLaunchKernelGGL(residual_kernel, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, H, V, w, C);
             CIR_CHECK_LAUNCH();
             // (the reflectors in A have been applied)
-            hipLaunchKernelGGL(residual_kernel<true>, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, V, V, w, A);
+            hipLaunchKernelGGL(gram_kernel, dim3(nt, nt, unsigned(batch)), dim3(256), 0, s, n, ld, V, A);
             CIR_CHECK_LAUNCH();
             auto product = [&](const float* a, int64_t a_m, int64_t a_k, const float* bb, float* c) {
                 GemmArgs g;
