@@ -1958,6 +1958,13 @@ inline bool use_refine(size_t esz, bool two, int batch, int n) {
     if (esz != sizeof(float) || !(two || n <= kSmallN)) return false;
     return n < kRefineMaxN || batch <= kRefineMaxBatch || n > kRefineAboveN;
 }
+// Matrices whose copies and residuals the work space holds: never fewer in a
+// larger batch than in a smaller one, since callers allocate for their largest
+// batch and run shorter ones in the same space.
+inline int refine_space(size_t esz, bool two, int batch, int n) {
+    if (use_refine(esz, two, batch, n)) return batch;
+    return use_refine(esz, two, kRefineMaxBatch, n) ? std::min(batch, kRefineMaxBatch) : 0;
+}
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
 constexpr int kRqRun = 128;          // rows summed in one MFMA chain
@@ -2212,6 +2219,7 @@ struct EighWork {
     int sub;  // matrices per inverse-iteration pass
 };
 
+// (every part, so the total too, never shrinks as the batch grows)
 inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
     EighWork L{};
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
@@ -2228,12 +2236,11 @@ inline EighWork eigh_layout(size_t esz, int batch, int n, int ld) {
         o = al(o + esz * batch * size_t(q2_blocks(n)) * kQ2BlockFloats);
     }
     L.refine = use_refine(esz, L.two, batch, n);
-    if (L.refine) {
-        L.off_h = o;
-        o = al(o + esz * batch * size_t(n) * ld);
-        L.off_r = o;
-        o = al(o + esz * batch * size_t(n) * ld);
-    }
+    const size_t nref = size_t(refine_space(esz, L.two, batch, n));
+    L.off_h = o;
+    o = al(o + esz * nref * size_t(n) * ld);
+    L.off_r = o;
+    o = al(o + esz * nref * size_t(n) * ld);
     L.off_d = o;
     o = al(o + esz * batch * n);
     L.off_e = o;

@@ -369,7 +369,9 @@ int cir_hamiltonian(int prec, int nframes, int n, int ld, int nchrom_mol, int is
  * the products that apply them in split-BF16x3 in both precisions: the
  * eigenvectors come out orthogonal to FP32's rounding.
  * ld must be a multiple of 4 and A_d 16-byte aligned (rows are streamed as
- * 16-byte vectors).  work_d must hold cir_eigh_workspace() bytes. */
+ * 16-byte vectors).  work_d must hold cir_eigh_workspace() bytes, which never
+ * decrease as the batch grows: a work space for the largest batch serves every
+ * smaller one of the same prec, n and ld. */
 size_t cir_eigh_workspace(int prec, int batch, int n, int ld);
 int cir_eigh_batched(int prec, int batch, int n, int ld, void* A_d, void* V_d, double* w_d, void* work_d,
                      void* stream);
