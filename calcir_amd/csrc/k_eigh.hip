@@ -1952,18 +1952,20 @@ inline bool use_whole_gpu(int batch, int n) {
 // 4e-7).  One matrix of n = 2048: 1.2 of 33 ms; 48 of n = 766: 2.4 of 12; 24 of n =
 // 3072: 58 of 173 (Q's part of these 0.23, 0.43, 12; C's FP64 costs 0.13, 0.26 and
 // 9 more than FP32).  Above kRefineAboveN, where only the one-stage form used to
-// run, it is always made.
+// run, it is always made; in deterministic mode by n alone, since a run's chunks
+// follow the free memory.
 constexpr int kRefineMaxN = 1024, kRefineMaxBatch = 16, kRefineAboveN = 2080;
 inline bool use_refine(size_t esz, bool two, int batch, int n) {
     if (esz != sizeof(float) || !(two || n <= kSmallN)) return false;
-    return n < kRefineMaxN || batch <= kRefineMaxBatch || n > kRefineAboveN;
+    if (n < kRefineMaxN || n > kRefineAboveN) return true;
+    return batch <= kRefineMaxBatch && !deterministic_mode();
 }
 // Matrices whose copies and residuals the work space holds: never fewer in a
 // larger batch than in a smaller one, since callers allocate for their largest
 // batch and run shorter ones in the same space.
 inline int refine_space(size_t esz, bool two, int batch, int n) {
-    if (use_refine(esz, two, batch, n)) return batch;
-    return use_refine(esz, two, kRefineMaxBatch, n) ? std::min(batch, kRefineMaxBatch) : 0;
+    if (esz != sizeof(float) || !(two || n <= kSmallN)) return 0;
+    return (n < kRefineMaxN || n > kRefineAboveN) ? batch : std::min(batch, kRefineMaxBatch);
 }
 
 constexpr int kRqT = 64, kRqK = 16;  // tile of the residual product, K step
