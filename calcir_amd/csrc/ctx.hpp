@@ -65,9 +65,16 @@ struct DevBuf {
         release();
         if (n == 0) n = 256;
         const PoolStream* ps = tl_pool;
-        const hipError_t e = ps ? hipMallocFromPoolAsync(&p, n, ps->pool, ps->stream)
-                             : tl_keep ? hipError_t(dev_cache_alloc(&p, n, &cap, &dev))
-                                       : hipMalloc(&p, n);
+        auto take = [&]() {
+            return ps ? hipMallocFromPoolAsync(&p, n, ps->pool, ps->stream)
+                      : tl_keep ? hipError_t(dev_cache_alloc(&p, n, &cap, &dev)) : hipMalloc(&p, n);
+        };
+        hipError_t e = take();
+        if (e == hipErrorOutOfMemory && dev_cache_bytes() > 0) {
+            (void)hipGetLastError();
+            dev_cache_release();
+            e = take();
+        }
         if (e != hipSuccess) {
             p = nullptr;
             return hip_fail(e, ps ? "hipMallocFromPoolAsync" : "hipMalloc", __FILE__, __LINE__);

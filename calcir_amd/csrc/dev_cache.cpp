@@ -150,11 +150,6 @@ int dev_cache_alloc(void** p, size_t n, size_t* cap, int* dev) {
     if (n >= kMinBlock && cache().take(n, *dev, p, cap)) return int(hipSuccess);
     *cap = n;
     e = hipMalloc(p, n);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        dev_cache_release();
-        e = hipMalloc(p, n);
-    }
     if (e != hipSuccess) *p = nullptr;
     return int(e);
 }

@@ -8,8 +8,9 @@
 //   - at most an eighth of the device's memory, the oldest block freed first,
 //     and only while a quarter of it is free for others;
 //   - for at most kCacheIdleSeconds without use, after which a thread frees
-//     them; all at once when an allocation does not fit, and at the end of
-//     cir_run_many, which leaves the device's memory as free as it can;
+//     them; all at once when an allocation of a context does not fit, whichever
+//     way it is made (DevBuf), and at both ends of cir_run_many, whose jobs take
+//     pooled memory instead;
 //   - a block is given back only after the stream that used it is through, so
 //     any thread and stream may take it.
 #pragma once

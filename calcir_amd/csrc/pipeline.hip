@@ -268,7 +268,9 @@ int auto_chunk(const cir_ctx* c, int nuniq) {
     auto need = [&](int B) { return double(B) * hv + double(eigh_workspace(c->real_prec, B, c->N, c->ld)); };
     size_t fr = 0, tot = 0;
     double budget = 24.0 * (1 << 30);
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess) budget = std::max(budget, 0.5 * double(fr + dev_cache_bytes()));
+    // (kept blocks are free memory to a thread that takes its buffers from them)
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess)
+        budget = std::max(budget, 0.5 * double(fr + (tl_pool ? 0 : dev_cache_bytes())));
     budget /= std::max(1, c->mem_share);
     int B = std::max(1, std::min(512, nuniq));
     while (B > 1 && need(B) > budget) B = std::max(1, std::min(B - 1, int(double(B) * budget / need(B))));
@@ -1176,6 +1178,7 @@ extern "C" int cir_run_many(int njob, cir_ctx* const* ctxs, const int* nframes, 
     std::vector<std::string> detail(njob);
     std::atomic<int> next{0};
     hipMemPool_t pool = job_pool();
+    dev_cache_release();  // kept blocks are no use to the jobs
     auto worker = [&]() {
         for (int q = next++; q < njob; q = next++) {
             const int j = order[q];
