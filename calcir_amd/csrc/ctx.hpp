@@ -23,9 +23,11 @@ struct PoolStream {
 inline thread_local const PoolStream* tl_pool = nullptr;
 
 // While a thread is in a KeepScope, the buffers that it takes (outside a
-// PoolStream) come from the memory kept between runs (dev_cache.hpp) and go
-// back to it once the work queued on the scope's stream, the only one that
-// uses them, is done.
+// PoolStream) come from the memory kept between runs (dev_cache.hpp); the ones
+// that it gives back go there once the work queued on the scope's stream, the
+// only one that uses them, is done.  A buffer given back outside a scope of its
+// stream (a context's own buffers, when it is destroyed) is freed: the stream
+// may be gone by then and its handle is not used.
 inline thread_local const hipStream_t* tl_keep = nullptr;
 struct KeepScope {
     const hipStream_t s;
@@ -51,7 +53,7 @@ struct DevBuf {
         if (p) {
             if (pooled)
                 (void)hipFreeAsync(p, fs);
-            else if (kept && hipStreamSynchronize(fs) == hipSuccess)
+            else if (kept && tl_keep && *tl_keep == fs && hipStreamSynchronize(fs) == hipSuccess)
                 dev_cache_free(p, cap, dev);
             else
                 (void)hipFree(p);

@@ -16,7 +16,8 @@
  *     null stream).  Per-stage calls enqueue work and return without
  *     synchronising.
  *   - A cir_ctx owns its device buffers, is bound to one stream and is not
- *     thread-safe; separate contexts may run concurrently.
+ *     thread-safe; separate contexts may run concurrently.  The stream must
+ *     live until the last call on the context other than cir_destroy() returns.
  *   - Real arrays of the per-stage calls hold "real_t" = float for
  *     CIR_PREC_FP32/CIR_PREC_BF16X3 and double for CIR_PREC_FP64.
  *

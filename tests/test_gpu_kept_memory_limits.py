@@ -1,11 +1,14 @@
-"""Device memory kept between runs: no growth over rounds, and no obstacle to jobs
-that need it."""
+"""Device memory kept between runs: no growth over rounds, no obstacle to jobs that
+need it, and no use of a stream that is gone."""
+
+import ctypes
 
 import numpy as np
 import pytest
 import torch
 
 import calcir_amd as C
+from calcir_amd.adjoint import LineshapeSession
 from conftest import announce
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +63,22 @@ def test_jobs_get_what_is_kept():
     for k in KEYS:
         for r in (got, alone):
             assert np.abs(np.asarray(r[k]) - np.asarray(ref[k])).max() <= 2e-5 * np.abs(np.asarray(ref[k])).max(), k
+
+
+def test_context_outlives_its_stream():
+    announce("kept memory limits: stream destroyed before the context")
+    L = C.lib()
+    L.hipStreamCreate.argtypes, L.hipStreamDestroy.argtypes = [ctypes.c_void_p], [ctypes.c_void_p]
+    xyz, box, times = C.synth_trajectory(100, 12, 9)
+    p = _params(10)
+    stream, ctx = ctypes.c_void_p(), ctypes.c_void_p()
+    assert L.hipStreamCreate(ctypes.byref(stream)) == 0
+    C.check(L.cir_create(ctypes.byref(p), xyz.shape[1], stream, ctypes.byref(ctx)))
+    f = np.zeros(p.ntcfpoints + p.nzeros)
+    C.check(L.cir_forward_ls(ctx, xyz.shape[0], xyz.ctypes.data, box.ctypes.data, times.ctypes.data, f.ctypes.data))
+    torch.cuda.synchronize()
+    assert L.hipStreamDestroy(stream) == 0
+    L.cir_destroy(ctx)  # its kept buffers are freed without the stream
+    s = LineshapeSession(p, xyz, box, times)
+    g = np.asarray(s.forward())
+    assert np.abs(f - g).max() <= 2e-5 * np.abs(g).max()
