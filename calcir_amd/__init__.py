@@ -18,7 +18,7 @@ import numpy as np
 
 __all__ = [
     "CalcirError", "Params", "Results", "lib", "default_params", "read_params", "write_outputs",
-    "synth_box_nm", "synth_trajectory", "run", "run_device", "nomega", "resolve_model", "resolve_species",
+    "synth_box_nm", "synth_trajectory", "run", "run_device", "release_memory", "nomega", "resolve_model", "resolve_species",
     "frame_index", "PREC_FP32", "PREC_FP64", "PREC_BF16X3", "MODE_PLAIN", "MODE_BATCHED", "NSITE",
     "SITE_E", "SITE_W", "SITE_X", "SITE_P", "SITE_MUP", "SITE_U", "SITE_R", "SITE_MU", "SITE_A",
 ]
@@ -130,6 +130,7 @@ SIGNATURES = {
     "cir_phase_times": (_i, [_vp, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_ll), _i]),
     "cir_tuning_report": (_i, [ctypes.c_char_p, _i]),
     "cir_destroy": (None, [_vp]),
+    "cir_release_memory": (_i, []),
     "cir_map_coefs": (_i, [_i, _i, _vp]),
     "cir_get_coefs": (_i, [_vp, _vp]),
     "cir_set_coefs": (_i, [_vp, _vp]),
@@ -497,6 +498,12 @@ def tuning_report():
         choice, _, times = rest.partition(" (")
         out[(fam,) + tuple(int(x) for x in shape)] = (int(choice), [float(x) for x in times.rstrip(" ms)").split()])
     return out
+
+
+def release_memory():
+    """Frees the device memory that runs keep for the next run (on the current
+    device), for torch's allocator or another process (cir_release_memory)."""
+    check(lib().cir_release_memory())
 
 
 def run_many(jobs, nthreads=8):

@@ -9,8 +9,8 @@
 //     and only while a quarter of it is free for others;
 //   - for at most kCacheIdleSeconds without use, after which a thread frees
 //     them; all at once when an allocation of a context does not fit, whichever
-//     way it is made (DevBuf), and at both ends of cir_run_many, whose jobs take
-//     pooled memory instead;
+//     way it is made (DevBuf), at both ends of cir_run_many, whose jobs take
+//     pooled memory instead, and by cir_release_memory();
 //   - a block is given back only after the stream that used it is through, so
 //     any thread and stream may take it.
 #pragma once

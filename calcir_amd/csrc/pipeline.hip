@@ -1242,6 +1242,13 @@ extern "C" int cir_get_results(cir_ctx* c, cir_results* r) try {
 
 extern "C" void cir_destroy(cir_ctx* c) { delete c; }
 
+extern "C" int cir_release_memory(void) try {
+    dev_cache_release();
+    return CIR_OK;
+} catch (...) {
+    return cir::host_exception("cir_release_memory");
+}
+
 // Per-stage C entry points over the kernels above -----------------------------
 
 extern "C" int cir_eigh_batched(int prec, int batch, int n, int ld, void* A_d, void* V_d, double* w_d, void* work_d,

@@ -15,9 +15,14 @@
  *     HIP device); "stream" is a hipStream_t passed as void* (NULL = the
  *     null stream).  Per-stage calls enqueue work and return without
  *     synchronising.
- *   - A cir_ctx owns its device buffers, is bound to one stream and is not
- *     thread-safe; separate contexts may run concurrently.  The stream must
- *     live until the last call on the context other than cir_destroy() returns.
+ *   - A cir_ctx is bound to one stream and is not thread-safe; separate
+ *     contexts may run concurrently.  The stream must live until the last
+ *     call on the context other than cir_destroy() returns.  Device memory that
+ *     a run no longer uses is kept for the next run of any context of the
+ *     process, instead of being freed and cleared again: at most an eighth of
+ *     the device's, only while a quarter of it is free, and for at most 30
+ *     seconds, after which a thread of the library frees it.
+ *     cir_release_memory() frees it at once; cir_run_many() leaves none.
  *   - Real arrays of the per-stage calls hold "real_t" = float for
  *     CIR_PREC_FP32/CIR_PREC_BF16X3 and double for CIR_PREC_FP64.
  *
@@ -318,6 +323,9 @@ int   cir_phase_times(cir_ctx* ctx, double* seconds, long long* groups, int npha
  * whole report.  CIR_NO_TUNE=1 in the environment turns the timing off. */
 int   cir_tuning_report(char* buf, int buflen);
 void  cir_destroy(cir_ctx* ctx);
+/* Frees the device memory kept between runs on the current device, for other
+ * users of it in the process or beside it. */
+int cir_release_memory(void);
 
 /* --- map coefficients and the lineshape adjoint ---------------------------- */
 /* The 13 map coefficients of a (map, species) row of calcIR.cu:1203-1242, in

@@ -1,5 +1,6 @@
-"""Device memory kept between runs: no growth over rounds, no obstacle to jobs that
-need it, and no use of a stream that is gone."""
+"""Device memory kept between runs: no growth over rounds, given back on request
+and by run_many, no obstacle to jobs that need it, and no use of a stream that
+is gone."""
 
 import ctypes
 
@@ -44,6 +45,22 @@ def test_no_growth_over_rounds():
         for j in jobs:
             C.run_device(*j)
     assert free0 - _free() < 256 * MB
+
+
+def test_given_back_on_request_and_by_run_many():
+    announce("kept memory limits: given back")
+    job = _device_job(384, 40, 77)
+    C.run_device(*job)
+    C.release_memory()
+    free0 = _free()
+    C.run_device(*job)
+    assert free0 - _free() > 256 * MB  # kept (over 20 MB a frame)
+    C.release_memory()
+    assert free0 - _free() < 64 * MB
+    C.run_device(*job)
+    xyz, box, times = C.synth_trajectory(64, 12, 5)
+    C.run_many([(_params(10), xyz, box, times)])
+    assert free0 - _free() < 64 * MB
 
 
 def test_jobs_get_what_is_kept():
