@@ -60,7 +60,7 @@ constexpr double kClusterRel = 1e-7;
 constexpr int kMaxCluster = 128;
 constexpr int kSingleMinN = 512;     // matrices at least this large may run the whole-GPU tridiagonalisation
 constexpr int kSingleMaxBatch = 16;  //   in batches of at most this many
-constexpr int kSinglePer = 512;      //   and at most n / kSinglePer (use_whole_gpu)
+                                     //   and of at most n / 320 (FP64) or n / 448 (use_whole_gpu)
 
 // Eigenvalue k joins the cluster of k-1 (ascending w).
 __device__ __forceinline__ bool joins_cluster(const double* w, int k) {
@@ -1909,9 +1909,11 @@ inline size_t larft_smem_bytes(size_t esz) { return size_t(kBtNB) * kLtP * esz; 
 // = 640 8.9 / 16.5, 32 of n = 2100 84 / 277, 24 of n = 3072 168 / 741; against
 // the whole-GPU form, one matrix of n = 512 8.8 / 13.8, n = 1024 22.6 / 30.7, n
 // = 2048 41 / 73.5, 8 of n = 512 8.9 / 104.  The whole-GPU form takes a time
-// that grows with the batch (n = 1024 in FP64: 27 per matrix), the batched form
-// one that does not up to a matrix per CU (76), and the ratio of the two grows
-// with n: the whole-GPU form runs batches of up to n / kSinglePer matrices.
+// that grows with the batch, the batched form one that does not up to a matrix
+// per CU: FP64 27 per matrix against 79 at n = 1024, 67 / 485 at 2048, 142 / 1560
+// at 3072, 266 / 3420 at 4096; FP32 140 / 984 at 3400, 180 / 1620 at 4096, 257 /
+// 2870 at 5000.  So the lines lie at 3, 7, 11, 13 matrices and at 7, 9, 11: about
+// n / 320 and n / 448.
 // CIR_EIGH_STAGES=1 or 2 in the environment forces one or two stages where
 // both apply (tests compare them).
 inline bool use_two_stage(size_t esz, int n, int ld) {
@@ -1924,8 +1926,9 @@ inline bool use_two_stage(size_t esz, int n, int ld) {
     if (forced == 2) return true;
     return n > kSmallN;
 }
-inline bool use_whole_gpu(int batch, int n) {
-    return n >= kSingleMinN && batch <= kSingleMaxBatch && int64_t(batch) * kSinglePer <= n;
+inline bool use_whole_gpu(size_t esz, int batch, int n) {
+    const int per = esz == 8 ? 320 : 448;
+    return n >= kSingleMinN && batch <= kSingleMaxBatch && int64_t(batch) * per <= n;
 }
 
 // The two-stage form's T carries the rounding of N bulge-chasing sweeps over
@@ -2311,7 +2314,7 @@ int eigh_impl(int gemm_prec, int batch, int n, int ld, T* A, T* V, double* w, un
         }
     }
     if (L.two) {
-    } else if (use_whole_gpu(batch, n)) {
+    } else if (use_whole_gpu(sizeof(T), batch, n)) {
         ProfScope ps(prof, CIR_PH_TRIDIAG, s);
         T* s1 = reinterpret_cast<T*>(work + L.off_s1);
         for (int b = 0; b < batch; ++b)

@@ -1,0 +1,55 @@
+"""FP64 batches on either side of the line between the whole-GPU form, one matrix
+at a time, and one workgroup per matrix: right on both, and a batch costs no
+more than its parts."""
+
+import time
+
+import numpy as np
+import pytest
+import torch
+
+from calcir_amd import stages as S
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _matrices(n, batch, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    H = torch.zeros((batch, n, (n + 3) // 4 * 4), dtype=torch.float64, device=DEV)
+    for b in range(batch):
+        a = torch.randn(n, n, generator=g, dtype=torch.float64, device=DEV) * 3.0
+        H[b, :, :n] = (a + a.T) / 2
+        H[b, :, :n].diagonal().add_(torch.rand(n, generator=g, dtype=torch.float64, device=DEV) * 700.0 - 400.0)
+    return H
+
+
+@pytest.mark.parametrize("n,batch", [(639, 2), (640, 2), (959, 3), (960, 3)])
+def test_fp64_on_both_sides(n, batch):
+    announce("whole-GPU line n=%d batch=%d" % (n, batch))
+    H = _matrices(n, batch, n)
+    ref = [H[b, :, :n].cpu().numpy() for b in range(batch)]
+    w, V = S.eigh(H, n)
+    eps = 2.2e-16
+    for b in range(batch):
+        v, k = V[b, :, :n].cpu().numpy(), w[b].cpu().numpy()
+        scale = np.abs(k).max()
+        assert np.abs(k - np.linalg.eigvalsh(ref[b])).max() <= 50 * eps * scale * np.sqrt(n)
+        assert np.abs(ref[b] @ v - v * k).max() / scale < 50 * eps * np.sqrt(n)
+
+
+def test_a_batch_costs_no_more_than_its_parts():
+    announce("whole-GPU line time")
+
+    def seconds(batch):
+        H = _matrices(2048, batch, batch)
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        S.eigh(H, 2048)
+        torch.cuda.synchronize()
+        return time.perf_counter() - t
+
+    seconds(1)
+    parts = seconds(4) + seconds(1)
+    assert seconds(5) <= 1.15 * parts  # runs of one side differ by less than a percent
