@@ -1348,15 +1348,12 @@ int tridiag_single(int n, int ld, T* A, T* d, T* e, T* tau, T* P, T* buf, hipStr
     return CIR_OK;
 }
 
-// 1/q from the hardware reciprocal (about 24 bits) refined by Newton-Raphson
-// steps r <- r + r (1 - q r): one step gives about 48 bits (measured max
-// relative error 2.2e-15), two give full double precision.
-template <bool FULL>
+// 1/q from the hardware reciprocal (about 24 bits) refined by one
+// Newton-Raphson step r <- r + r (1 - q r): about 48 bits (measured max
+// relative error 2.2e-15).
 __device__ __forceinline__ double nr_rcp(double q) {
-    double r = __builtin_amdgcn_rcp(q);
-    r = fma(r, fma(-q, r, 1.0), r);
-    if constexpr (FULL) r = fma(r, fma(-q, r, 1.0), r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(q);
+    return fma(fma(-q, r, 1.0), r, r);
 }
 
 // Number of eigenvalues of T below x: the sign changes of the leading
@@ -1531,12 +1528,12 @@ __device__ __forceinline__ LuRow invit_lu_row(double sub, double dn, double en, 
         o.r = 1.0 / den;
         o.l = num / den;
     } else {
-        o.r = nr_rcp<false>(den);
+        o.r = nr_rcp(den);
         o.l = num * o.r;
     }
     if (fabs(den) < pivmin) {
         const double u0 = (den < 0.0) ? -pivmin : pivmin;
-        o.r = (sizeof(T) == 8) ? 1.0 / u0 : nr_rcp<false>(u0);
+        o.r = (sizeof(T) == 8) ? 1.0 / u0 : nr_rcp(u0);
     }
     o.u1 = o.piv ? dn : bs;
     o.u2 = o.piv ? en : 0.0;

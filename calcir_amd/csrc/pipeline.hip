@@ -275,8 +275,9 @@ int auto_chunk(const cir_ctx* c, int nuniq) {
     int B = std::max(1, std::min(512, nuniq));
     while (B > 1 && need(B) > budget) B = std::max(1, std::min(B - 1, int(double(B) * budget / need(B))));
     // chunks of nearly equal size: a short last chunk would leave most CUs
-    // idle in the one-workgroup-per-matrix kernels (and at 16 or fewer large
-    // matrices take the one-matrix-at-a-time path)
+    // idle in the one-workgroup-per-matrix kernels (few FP64 matrices, and
+    // few of N > 3104, run one at a time on the whole GPU instead, and at most
+    // 16 FP32 ones of 1024 <= N <= 2080 have their eigenpairs corrected)
     const int nchunk = (nuniq + B - 1) / B;
     return (nuniq + nchunk - 1) / nchunk;
 }
