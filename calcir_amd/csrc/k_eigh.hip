@@ -2142,23 +2142,34 @@ rotation_kernel(int n, int ld, const double* __restrict__ wall, const float* __r
 }
 
 // w_k += dl_k, then kept ascending (a running maximum: neighbours closer than
-// the corrections' own error may come out exchanged).  One workgroup per matrix.
+// the corrections' own error may come out exchanged).  Left as bisection gave it
+// where a correction is far past the reductions' backward error (1e-6 of the
+// spectrum): the vectors are then no eigenvectors (a matrix of zeros, or one so
+// small that the whole spectrum lies within inverse iteration's cluster gap).
+// One workgroup per matrix.
+constexpr double kCorrectMax = 1e-4;
 __global__ void __launch_bounds__(1024)
 correct_w_kernel(int n, const float* __restrict__ dlall, double* __restrict__ wall) {
     extern __shared__ __align__(16) double sw_[];  // 2 n
     const int b = blockIdx.x;
     double* w = wall + size_t(b) * n;
-    for (int k = threadIdx.x; k < n; k += 1024) sw_[k] = w[k] + double(dlall[size_t(b) * n + k]);
+    const double most = kCorrectMax * fmax(fabs(w[0]), fabs(w[n - 1]));
+    bool far = false;
+    for (int k = threadIdx.x; k < n; k += 1024) {
+        const double d = double(dlall[size_t(b) * n + k]);
+        far |= !(fabs(d) <= most);
+        sw_[k] = w[k] + d;
+    }
+    if (__syncthreads_or(far)) return;
     double* a = sw_;
     double* c = sw_ + n;
     for (int off = 1; off < n; off <<= 1) {
-        __syncthreads();
         for (int k = threadIdx.x; k < n; k += 1024) c[k] = (k >= off) ? fmax(a[k], a[k - off]) : a[k];
         double* t = a;
         a = c;
         c = t;
+        __syncthreads();
     }
-    __syncthreads();
     for (int k = threadIdx.x; k < n; k += 1024) w[k] = a[k];
 }
 
