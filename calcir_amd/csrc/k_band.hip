@@ -92,15 +92,22 @@ __device__ __forceinline__ void wave_colsums32(const float (&x)[32], int lane, f
 // Newton step each way (the residual of |x|^2, of tau beta and of scale
 // (alpha - beta), each by one FMA, so each result is within an ulp); the IEEE
 // root and quotients are three chains of a dozen dependent instructions on a
-// task's critical path.  Squares too small for the hardware root take those.
-__device__ __forceinline__ void sb_householder(float alpha, float sigma, float& beta, float& tau, float& scale) {
+// task's critical path.  Squares too large for the hardware root take those.
+// False, and nothing done, for squares below kSbTiny: nearly equal columns leave
+// vectors whose length falls by FP32's rounding from column to column, and below
+// that the squares are lost to underflow, and with them the reflector its
+// orthogonality (eigenvalues off by 1e-4 of the spectrum).  The caller then sums
+// the squares of kSbUp x (sb_householder_up).
+constexpr float kSbTiny = 1e-30f, kSbUp = 0x1p60f;
+__device__ __forceinline__ bool sb_householder(float alpha, float sigma, float& beta, float& tau, float& scale) {
     const float a2 = alpha * alpha + sigma;
-    if (!(a2 >= 1e-30f && a2 <= 1e30f)) {
+    if (!(a2 >= kSbTiny && a2 <= 1e30f)) {
+        if (a2 < kSbTiny) return false;
         const float nrm = sqrtf(a2);
         beta = alpha >= 0.f ? -nrm : nrm;
         tau = (beta - alpha) / beta;
         scale = 1.f / (alpha - beta);
-        return;
+        return true;
     }
     const float y = __builtin_amdgcn_rsqf(a2);
     float nrm = a2 * y;
@@ -112,6 +119,14 @@ __device__ __forceinline__ void sb_householder(float alpha, float sigma, float& 
     tau = fmaf(fmaf(-tau, beta, -den), yb, tau);
     const float r = __builtin_amdgcn_rcpf(den);
     scale = fmaf(fmaf(-den, r, 1.f), r, r);
+    return true;
+}
+// The scalars from alpha and the square sum of kSbUp x.  What is still too short
+// (1e-33) is taken as zero.
+__device__ __forceinline__ void sb_householder_up(float alpha, float sigma, float& beta, float& tau, float& scale) {
+    if (!(sigma > 0.f) || !sb_householder(alpha * kSbUp, sigma, beta, tau, scale)) return;
+    beta *= 1.f / kSbUp;
+    scale *= kSbUp;
 }
 
 // Householder QR of one panel below the band and everything the trailing
@@ -139,7 +154,7 @@ __global__ void __launch_bounds__(kPanNT) sb_panel_kernel(int n, int ld, int j0,
                                                           float* __restrict__ Pall, float* __restrict__ Yhall) {
     constexpr int NB = kBandNB, CB = 8;
     static_assert(NB == 32, "the column sums and the rotation are written for 32 columns");
-    __shared__ float redC[2][kPanNW][NB], taus[NB];
+    __shared__ float redC[2][kPanNW][NB], redS[kPanNW], taus[NB];
     __shared__ __align__(16) float rowc[2][NB], gram[NB][NB + 4], Tc[NB][NB + 4];
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -192,7 +207,22 @@ __global__ void __launch_bounds__(kPanNT) sb_panel_kernel(int n, int ld, int j0,
             const float sigma = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tot), cc));
             const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pcq), cc));
             float tau = 0.f, beta = alpha, scale = 0.f;
-            if (sigma > 0.f) sb_householder(alpha, sigma, beta, tau, scale);
+            if (sigma > 0.f && !sb_householder(alpha, sigma, beta, tau, scale)) {
+                // (alpha and sigma are the same in every thread)
+                float x2 = 0.f;
+#pragma unroll
+                for (int i = 0; i < RPT; ++i) {
+                    const float x = (tid + kPanNT * i > c) ? p[i][cc] * kSbUp : 0.f;
+                    x2 += x * x;
+                }
+                x2 = bwave_sum(x2);
+                if (lane == 0) redS[wave] = x2;
+                __syncthreads();
+                x2 = 0.f;
+#pragma unroll
+                for (int w = 0; w < kPanNW; ++w) x2 += redS[w];
+                sb_householder_up(alpha, x2, beta, tau, scale);
+            }
             tot = scale * tot + pcq;  // v^T P(:, column of register q)
             if (wave == 0) {
                 const int qc = (q + CB * blk) & (NB - 1);
@@ -840,7 +870,11 @@ __device__ __forceinline__ void sb_task(int n, int s, int k, int off, float* w, 
     const float sigma = half_sum((i >= 1 && rowok) ? x * x : 0.f);
     const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 0));
     float tau = 0.f, beta = alpha, scale = 0.f;
-    if (__builtin_amdgcn_readfirstlane(__float_as_int(sigma)) != 0) sb_householder(alpha, sigma, beta, tau, scale);
+    if (__builtin_amdgcn_readfirstlane(__float_as_int(sigma)) != 0 &&
+        !sb_householder(alpha, sigma, beta, tau, scale)) {
+        const float xu = x * kSbUp;
+        sb_householder_up(alpha, half_sum((i >= 1 && rowok) ? xu * xu : 0.f), beta, tau, scale);
+    }
     const float vi = (i == 0) ? 1.f : (rowok ? x * scale : 0.f);
     if (h == 0) vs[i] = vi;
     wave_lds_sync();
