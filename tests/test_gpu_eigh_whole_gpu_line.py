@@ -43,13 +43,15 @@ def test_a_batch_costs_no_more_than_its_parts():
     announce("whole-GPU line time")
 
     def seconds(batch):
-        H = _matrices(2048, batch, batch)
-        torch.cuda.synchronize()
-        t = time.perf_counter()
-        S.eigh(H, 2048)
-        torch.cuda.synchronize()
-        return time.perf_counter() - t
+        best = np.inf  # (the first pass takes new memory)
+        for _ in range(3):
+            H = _matrices(2048, batch, batch)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            S.eigh(H, 2048)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best
 
-    seconds(1)
     parts = seconds(4) + seconds(1)
     assert seconds(5) <= 1.15 * parts  # runs of one side differ by less than a percent
